@@ -166,6 +166,10 @@ struct sl_ctx {
     uint32_t* d_geno2 = nullptr;
     double* d_lfreq = nullptr;     // [M][2] ln(1 - minor), ln(minor): the founder-allele terms
     double* d_lsum = nullptr;      // [M][kLsumK] a free component's term by allele-count difference
+    uint8_t* d_mcls = nullptr;     // [2(N-F)][M] classes of a meiosis's flip by locus
+    int32_t* d_joblist = nullptr;  // [2(N-F)][M] the loci whose flipped likelihood is computed
+    int32_t* d_jobcnt = nullptr;   // [2(N-F)]
+    int max_jobs = 0;              // the largest of d_jobcnt
     int32_t* d_meioses = nullptr;
     int32_t* d_order = nullptr;
     size_t order_cap = 0;
@@ -175,6 +179,7 @@ struct sl_ctx {
     double* d_lflip = nullptr;
     double* d_fbuf = nullptr;
     uint8_t* d_maps = nullptr;
+    double* d_mu = nullptr;        // [2][chains][M] uniforms of an M-step
     uint32_t* d_near = nullptr;
     uint32_t* d_near_loci = nullptr;  // [chains][ceil(M/32)] loci of L-sampler near-edge draws
     // CODA trace: a likelihood per chain at every scored sweep of sl_mcmc_run
@@ -391,8 +396,9 @@ int release_all(sl_ctx* c) {
                     c->d_ssched_ops_w, c->d_rlevel_off,
                     c->d_rlevel_ops, c->d_mother, c->d_father, c->d_legal_t, c->d_gprob_d, c->d_gprob_f,
                     c->d_theta, c->d_chains, c->d_status,
-                    c->d_gen_off, c->d_ptab, c->d_geno2, c->d_lfreq, c->d_lsum, c->d_meioses, c->d_order,
-                    c->d_fixed_order, c->d_lcur, c->d_lflip, c->d_fbuf, c->d_maps, c->d_near, c->d_near_loci,
+                    c->d_gen_off, c->d_ptab, c->d_geno2, c->d_lfreq, c->d_lsum, c->d_meioses, c->d_mcls,
+                    c->d_joblist, c->d_jobcnt, c->d_order,
+                    c->d_fixed_order, c->d_lcur, c->d_lflip, c->d_fbuf, c->d_maps, c->d_mu, c->d_near, c->d_near_loci,
                     c->d_ops, c->d_prevs, c->d_children, c->d_tasks, c->d_tinfo, c->d_idx, c->d_level_base,
                     c->d_sched_off,
                     c->d_sched_ops, c->d_trait_d,
@@ -513,7 +519,29 @@ int setup_msampler(sl_ctx* c, const sl_pedigree_desc* ped) {
         (rc = upload(c, &c->d_lsum, lsum.data(), lsum.size())) ||
         (rc = upload(c, &c->d_meioses, c->meioses_h.data(), c->meioses_h.size())))
         return rc;
-    SL_HIP(c, hipStreamSynchronize(c->stream));  // the host tables above go out of scope
+    // what each meiosis's flip does at each locus, and the loci left to compute
+    const size_t nb = 2 * (size_t)(N - F);
+    uint8_t* masks = nullptr;
+    if ((rc = upload<uint8_t>(c, &c->d_mcls, nullptr, nb * M)) ||
+        (rc = upload<int32_t>(c, &c->d_joblist, nullptr, nb * M)) ||
+        (rc = upload<int32_t>(c, &c->d_jobcnt, nullptr, nb)) ||
+        (rc = upload<uint8_t>(c, &masks, nullptr, (size_t)N * M)))
+        return rc;
+    sl::MsampArgs K{};
+    K.N = N;
+    K.F = F;
+    K.M = M;
+    K.ptab = c->d_ptab;
+    K.geno2 = c->d_geno2;
+    K.GW = GW;
+    std::vector<int32_t> cnt(nb);
+    hipError_t e = sl::launch_mclass(K, masks, c->d_mcls, c->d_joblist, c->d_jobcnt, c->stream);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(cnt.data(), c->d_jobcnt, nb * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);  // and the host tables above go out of scope
+    (void)hipFree(masks);
+    SL_HIP(c, e);
+    c->max_jobs = *std::max_element(cnt.begin(), cnt.end());
     c->m_ready = true;
     return SL_OK;
 }
@@ -1000,7 +1028,7 @@ static int alloc_chains(sl_ctx* c, int n_chains) {
     const size_t cm = (size_t)n_chains * c->M;
     if (n_chains != c->n_chains) {
         void** bufs[] = {(void**)&c->d_chains, (void**)&c->d_status, (void**)&c->d_lcur, (void**)&c->d_lflip,
-                         (void**)&c->d_fbuf, (void**)&c->d_maps, (void**)&c->d_near, (void**)&c->d_near_loci};
+                         (void**)&c->d_fbuf, (void**)&c->d_maps, (void**)&c->d_mu, (void**)&c->d_near, (void**)&c->d_near_loci};
         for (void** b : bufs) {
             if (*b) SL_HIP(c, hipFree(*b));
             *b = nullptr;
@@ -1012,6 +1040,7 @@ static int alloc_chains(sl_ctx* c, int n_chains) {
         SL_HIP(c, hipMalloc((void**)&c->d_lflip, 4 * cm * sizeof(double)));
         SL_HIP(c, hipMalloc((void**)&c->d_fbuf, 2 * cm * sizeof(double)));
         SL_HIP(c, hipMalloc((void**)&c->d_maps, cm));
+        SL_HIP(c, hipMalloc((void**)&c->d_mu, (c->m_ubuf ? 2 * cm : 1) * sizeof(double)));
         SL_HIP(c, hipMalloc((void**)&c->d_near, (size_t)n_chains * sizeof(uint32_t)));
         SL_HIP(c, hipMalloc((void**)&c->d_near_loci, (size_t)n_chains * near_words(c) * sizeof(uint32_t)));
         c->n_chains = n_chains;
@@ -1364,6 +1393,9 @@ static sl::MsampArgs msamp_args(sl_ctx* c) {
     A.lsum = c->d_lsum;
     A.theta = c->d_theta;
     A.meioses = c->d_meioses;
+    A.cls = c->d_mcls;
+    A.joblist = c->d_joblist;
+    A.jobcnt = c->d_jobcnt;
     A.n_meioses = (int)c->meioses_h.size();
     A.order = c->d_order;
     A.graphs = c->d_chains;
@@ -1380,6 +1412,7 @@ static sl::MsampArgs msamp_args(sl_ctx* c) {
     A.n_chains = c->n_chains;
     A.fp32 = c->precision == SL_FP32_RESCALED ? 1 : 0;
     A.fb_ubuf = c->m_ubuf ? 1 : 0;
+    A.udev = c->d_mu;
     return A;
 }
 
@@ -1433,10 +1466,15 @@ static int run_msweep(sl_ctx* c, uint64_t seed, uint32_t sweep, const int32_t* d
                       (launch_mode == SL_MSAMPLER_SPECULATIVE ||
                        (launch_mode == SL_MSAMPLER_AUTO && (int64_t)c->n_chains * c->M * 2 <= kSpecWaves));
     A.spec = spec ? 1 : 0;
+    // job slots of a step: a list's worth, or with few speculative chains one
+    // slot per locus (the job then knows its locus without the list's loads)
+    A.compact = spec && (int64_t)c->n_chains * c->M * 2 <= kSpecWaves ? 0 : 1;
+    const int jobs = A.compact ? c->max_jobs : c->M;
     // start of the sweep: the current columns and step 0's flipped columns
     A.with_lcur = 1;
     A.step = 0;
-    A.n_jobs = 2 * c->M;
+    A.n_jobs = c->M + jobs;
+    A.draw_uniforms = 1;
     SL_HIP(c, sl::launch_mstep(A, c->m_lds, c->stream));
     A.with_lcur = 0;
     if (spec)
@@ -1444,7 +1482,8 @@ static int run_msweep(sl_ctx* c, uint64_t seed, uint32_t sweep, const int32_t* d
             for (int k = 0; k < nm; ++k) {
                 A.fb_step = k;
                 A.step = k + 1;
-                A.n_jobs = k + 1 < nm ? 2 * c->M : 0;
+                A.n_jobs = k + 1 < nm ? 2 * jobs : 0;
+                A.draw_uniforms = k + 1 < nm ? 1 : 0;
                 SL_HIP(c, sl::launch_mspec(A, c->m_spec_lds, c->stream));
             }
             return SL_OK;
@@ -1453,8 +1492,8 @@ static int run_msweep(sl_ctx* c, uint64_t seed, uint32_t sweep, const int32_t* d
         A.fb_step = k;
         A.step = k + 1;
         rc = timed_launch(c, SL_KERNEL_MSAMPLER_FB, [&] { return sl::launch_mfb(A, c->stream); });
-        A.n_jobs = k + 1 < nm ? c->M : 0;
-        if (!rc && A.n_jobs)
+        A.n_jobs = k + 1 < nm ? jobs : 0;
+        if (!rc && k + 1 < nm)
             rc = timed_launch(c, SL_KERNEL_MSAMPLER, [&] { return sl::launch_mstep(A, c->m_lds, c->stream); });
         if (rc) return rc;
     }

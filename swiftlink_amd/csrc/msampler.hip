@@ -11,18 +11,25 @@
 //    complementary allele assignments; its result is the sum, over the allele
 //    assignments of the founder alleles that satisfy every genotype, of the
 //    product of allele frequencies, or 0 when none does.  Here the wave's
-//    lanes build the same components in parallel: founder-allele labels are
-//    propagated generation by generation, every typed person becomes an edge
-//    between its two founder alleles (heterozygous: the alleles differ,
-//    homozygous: both equal the genotype's allele), and a union-find with a
-//    parity bit per node (is the node's allele the opposite of its
-//    parent's?) is built by rounds of hooking roots onto smaller roots and
-//    path compression until no edge joins two components.  Then every edge is
-//    checked against the parities, homozygous edges fix their root's allele,
-//    and with n0/n1 the numbers of a root's nodes of parity 0/1 its component
-//    contributes maj^n0 min^n1 (root allele A), maj^n1 min^n0 (root allele B)
-//    or their sum, taken in log space.  Legality is exactly the reference's;
-//    the likelihood agrees with its products to rounding.
+//    lanes work on all persons at once: founder-allele labels are propagated
+//    generation by generation; every homozygous person fixes its two founder
+//    alleles, every heterozygous one is an edge between two alleles that
+//    differ; fixed alleles pass along the edges until nothing changes (two or
+//    three rounds).  The fixed nodes are counted by ballot: their share of the
+//    likelihood is maj^nA min^nB.  Components that no homozygous person reaches
+//    (a locus in twenty at ped150) get a union-find with a parity bit per node,
+//    built by rounds of hooking roots onto smaller roots and path compression;
+//    with n0/n1 the numbers of a root's nodes of parity 0/1 such a component
+//    contributes maj^n0 min^n1 + maj^n1 min^n0, taken in log space.  Legality is
+//    exactly the reference's; the likelihood agrees with its products to
+//    rounding.  With a union-find over every edge of every locus a launch for
+//    64 chains at ped150 (half of them on an M-sweep) took 41 us and one for 32
+//    at 600 people and 2000 loci 169 us; now 19 us and 67 us, a third of the
+//    loci being evaluated (next point).
+//  * Of the flips of a step only those whose outcome depends on the descent
+//    graph are evaluated: where the meiosis's parent cannot be heterozygous the
+//    flip changes nothing, and where its phase and the transmitted allele are
+//    known the flip is illegal (mclass_kernel, once per context).
 //  * Forward-backward (forward_backward): one workgroup per chain; a block
 //    scan of the 2x2 matrices T(theta_{l-1}) diag(e_l) gives the forward
 //    probabilities; a locus draws a uniform only when both its states are
@@ -97,22 +104,23 @@ __device__ __forceinline__ double wave_sum(double x) {
     return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
-// A wave's LDS: the locus's free-component terms, column words, union-find
-// words, per-node accumulators, edges and founder-allele labels.
+// A wave's LDS: column words, union-find words, per-node words, edges and
+// founder-allele labels.
 struct WaveArea {
-    double* lsum;     // [kLsumK] the locus's row of MsampArgs::lsum
     uint32_t* colw;   // [W]
     uint32_t* uf;     // [2F] parent (bits 0-15) | parity to parent (bit 16)
-    uint32_t* acc;    // [2F] root allele A needed (bit 0), B needed (bit 1), touched (bit 2),
-                      //      n0 (bits 3-13), n1 (bits 14-24)
-    uint32_t* edges;  // [N] x (bits 0-9) | y (bits 10-19) | heterozygous (bit 20) | allele B (bit 21)
+    uint32_t* acc;    // [2F] fixed to allele A (bit 0), to B (bit 1), touched (bit 2);
+                      //      a free component's root: n0 (bits 3-13), n1 (bits 14-24)
+    uint32_t* edges;  // [N] x (bits 0-9) | y (bits 10-19) | kEdge, 0 once settled
     uint16_t* lab;    // [2(N-F)] founder allele of (person, parent)
 };
 
+// an edge word in use (its nodes may both be node 0 only when it is illegal)
+constexpr uint32_t kEdge = 1u << 20;
+
 __device__ __forceinline__ WaveArea wave_area(const MsampArgs& A, unsigned char* base) {
     WaveArea w;
-    w.lsum = reinterpret_cast<double*>(base);
-    w.colw = reinterpret_cast<uint32_t*>(base + sizeof(double) * kLsumK);
+    w.colw = reinterpret_cast<uint32_t*>(base);
     w.uf = w.colw + A.W;
     w.acc = w.uf + 2 * A.F;
     w.edges = w.acc + 2 * A.F;
@@ -136,6 +144,40 @@ __device__ __forceinline__ uint32_t uf_find(const uint32_t* uf, uint32_t x, uint
 // genotype of person i at locus l from the 2-bit packed table (0: untyped)
 __device__ __forceinline__ int genotype_at(const MsampArgs& A, int l, int i) {
     return (int)((A.geno2[(size_t)l * A.GW + (i >> 4)] >> (2 * (i & 15))) & 3u);
+}
+
+// One typed person with genotype g and founder alleles x, y: both are touched,
+// and a homozygous person fixes them to its genotype's allele
+__device__ __forceinline__ void mark_person(const WaveArea& w, int g, uint32_t x, uint32_t y) {
+    const uint32_t mark = g == G_HETERO ? 4u : g == G_HOMOZ_B ? 6u : 5u;
+    atomicOr(&w.acc[x], mark);
+    atomicOr(&w.acc[y], mark);
+}
+
+// An edge whose nodes hold fixed alleles a, b (bits 0-1 of their words, 0:
+// none): passes the opposite allele on where one side is fixed.  Returns
+// whether the edge is settled (one side fixed), setting *conflict when both
+// sides hold the same allele.
+__device__ __forceinline__ bool pass_fixed(const WaveArea& w, uint32_t e, uint32_t a, uint32_t b, bool* changed,
+                                           bool* conflict) {
+    if ((a | b) == 0u) return false;
+    if (a == 0u || b == 0u) {
+        atomicOr(&w.acc[(a ? e >> 10 : e) & 0x3FFu], (a | b) ^ 3u);
+        *changed = true;
+    } else {
+        *conflict |= (a & b) != 0u;
+    }
+    return true;
+}
+
+// ln(e^l0 + e^l1) of a component free to take either assignment, from its
+// root's counts
+__device__ __forceinline__ double free_term(const MsampArgs& A, int l, uint32_t a, double lmaj, double lmin) {
+    const uint32_t c0 = (a >> 3) & 0x7FFu, c1 = (a >> 14) & 0x7FFu, kd = c0 > c1 ? c0 - c1 : c1 - c0;
+    const double n0 = (double)c0, n1 = (double)c1;
+    const double l0 = n0 * lmaj + n1 * lmin;  // root allele A
+    const double l1 = n1 * lmaj + n0 * lmin;  // root allele B
+    return fmax(l0, l1) + (kd < (uint32_t)kLsumK ? A.lsum[(size_t)l * kLsumK + kd] : log1p(exp(-fabs(l0 - l1))));
 }
 
 // log of the founder-allele-graph likelihood of the column in w.colw at locus
@@ -165,13 +207,10 @@ __device__ double fag_log_likelihood(const MsampArgs& A, const uint2* ptab, cons
         }
         wave_sync();
     }
-    for (int x = lane; x < nodes; x += 64) {
-        w.uf[x] = (uint32_t)x;
-        w.acc[x] = 0u;
-    }
+    for (int x = lane; x < nodes; x += 64) w.acc[x] = 0u;
     wave_sync();
-    // edges: the typed persons with a genotype at this locus; the founder
-    // alleles they touch are marked
+    // the typed persons with a genotype: a homozygous one fixes both its
+    // founder alleles, a heterozygous one is an edge between them
     const uint64_t below = (1ull << lane) - 1ull;
     int E = 0;
     bool bad = false;
@@ -182,36 +221,64 @@ __device__ double fag_log_likelihood(const MsampArgs& A, const uint2* ptab, cons
         for (int k = 0; k < kGenoPrefetch; ++k)
             if (c == k) g = gpre[k];
         if (c >= kGenoPrefetch) g = i < A.N ? genotype_at(A, l, i) : 0;
-        uint32_t e = 0;
+        uint32_t x = 0, y = 0;
         if (g) {
-            const uint32_t x = i < F ? (uint32_t)(2 * i) : w.lab[2 * (i - F)];
-            const uint32_t y = i < F ? (uint32_t)(2 * i + 1) : w.lab[2 * (i - F) + 1];
+            x = i < F ? (uint32_t)(2 * i) : w.lab[2 * (i - F)];
+            y = i < F ? (uint32_t)(2 * i + 1) : w.lab[2 * (i - F) + 1];
             bad |= g == G_HETERO && x == y;  // an autozygous heterozygote (:77-81)
-            e = x | (y << 10) | ((g == G_HETERO ? 1u : 0u) << 20) | ((g == G_HOMOZ_B ? 1u : 0u) << 21);
-            atomicOr(&w.acc[x], 4u);
-            atomicOr(&w.acc[y], 4u);
+            mark_person(w, g, x, y);
         }
-        const uint64_t mask = __ballot(g != 0);
-        if (g) w.edges[E + __popcll(mask & below)] = e;
+        const uint64_t mask = __ballot(g == G_HETERO);
+        if (g == G_HETERO) w.edges[E + __popcll(mask & below)] = x | (y << 10) | kEdge;
         E += __popcll(mask);
     }
     if (__ballot(bad)) return -INFINITY;
+    // fixed alleles pass along the edges until nothing changes
+    bool conflict = false, pending = false;
+    for (;;) {
+        wave_sync();
+        bool changed = false;
+        pending = false;
+        for (int e0 = 0; e0 < E; e0 += 64) {
+            const int e = e0 + lane;
+            uint32_t ed = e < E ? w.edges[e] : 0u;
+            if (ed) {
+                const uint32_t a = w.acc[ed & 0x3FFu] & 3u, b = w.acc[(ed >> 10) & 0x3FFu] & 3u;
+                if (pass_fixed(w, ed, a, b, &changed, &conflict)) w.edges[e] = 0u;
+                else pending = true;
+            }
+        }
+        if (!__ballot(changed)) break;
+    }
+    int nA = 0, nB = 0;
+    for (int x0 = 0; x0 < nodes; x0 += 64) {
+        const uint32_t a = x0 + lane < nodes ? w.acc[x0 + lane] & 3u : 0u;
+        conflict |= a == 3u;
+        nA += __popcll(__ballot(a == 1u));
+        nB += __popcll(__ballot(a == 2u));
+    }
+    if (__ballot(conflict)) return -INFINITY;
+    const double lmaj = A.lfreq[2 * (size_t)l], lmin = A.lfreq[2 * (size_t)l + 1];
+    const double ll = (double)nA * lmaj + (double)nB * lmin;
+    if (!__ballot(pending)) return ll;
+    // components no homozygous person reaches: hook the larger root under the
+    // smaller one with the parity the edge implies (the alleles of an edge
+    // differ), compress paths, until no edge joins two components (every
+    // productive round removes a component, so at most 2F rounds)
+    for (int x = lane; x < nodes; x += 64) w.uf[x] = (uint32_t)x;
     wave_sync();
-    // components: hook the larger root under the smaller one with the parity
-    // the edge implies, compress paths, until no edge joins two components
-    // (every productive round removes a component, so at most 2F rounds)
     bool converged = false;
     for (int round = 0; round <= nodes && !converged; ++round) {
         bool changed = false;
         for (int e0 = 0; e0 < E; e0 += 64) {
             const int e = e0 + lane;
-            if (e < E) {
+            if (e < E && w.edges[e]) {
                 const uint32_t ed = w.edges[e];
                 uint32_t px, py;
                 const uint32_t rx = uf_find(w.uf, ed & 0x3FFu, &px);
                 const uint32_t ry = uf_find(w.uf, (ed >> 10) & 0x3FFu, &py);
                 if (rx != ry) {
-                    w.uf[rx > ry ? rx : ry] = (rx < ry ? rx : ry) | ((px ^ py ^ ((ed >> 20) & 1u)) << 16);
+                    w.uf[rx > ry ? rx : ry] = (rx < ry ? rx : ry) | ((px ^ py ^ 1u) << 16);
                     changed = true;
                 }
             }
@@ -228,47 +295,29 @@ __device__ double fag_log_likelihood(const MsampArgs& A, const uint2* ptab, cons
         converged = !__ballot(changed);
     }
     // converged and compressed: every node's word holds its root and parity
-    // consistency: every edge's parity; homozygous edges fix their root's allele
     bool illegal = !converged;
     for (int e0 = 0; e0 < E; e0 += 64) {
         const int e = e0 + lane;
-        if (e < E) {
+        if (e < E && w.edges[e]) {
             const uint32_t ed = w.edges[e];
             const uint32_t ux = w.uf[ed & 0x3FFu], uy = w.uf[(ed >> 10) & 0x3FFu];
-            const uint32_t rx = ux & 0xFFFFu, px = (ux >> 16) & 1u;
-            const uint32_t het = (ed >> 20) & 1u, allele = (ed >> 21) & 1u;
-            illegal |= rx != (uy & 0xFFFFu) || (px ^ ((uy >> 16) & 1u)) != het;
-            if (!het) atomicOr(&w.acc[rx], 1u << (allele ^ px));
+            illegal |= (ux & 0xFFFFu) != (uy & 0xFFFFu) || (((ux ^ uy) >> 16) & 1u) != 1u;
         }
     }
-    wave_sync();
     if (__ballot(illegal)) return -INFINITY;
-    for (int x = lane; x < nodes; x += 64) {
-        if (w.acc[x] & 4u) {
+    // touched nodes without a fixed allele, counted at their root by parity
+    for (int x = lane; x < nodes; x += 64)
+        if ((w.acc[x] & 7u) == 4u) {
             const uint32_t u = w.uf[x];
             atomicAdd(&w.acc[u & 0xFFFFu], ((u >> 16) & 1u) ? (1u << 14) : (1u << 3));
         }
-    }
     wave_sync();
-    const double lmaj = A.lfreq[2 * (size_t)l], lmin = A.lfreq[2 * (size_t)l + 1];
-    double ll = 0.0;
-    bool conflict = false;
+    double free_ll = 0.0;
     for (int x = lane; x < nodes; x += 64) {
         const uint32_t a = w.acc[x];
-        if (!(a & 4u) || (w.uf[x] & 0xFFFFu) != (uint32_t)x) continue;  // untouched, or not a root
-        const uint32_t c0 = (a >> 3) & 0x7FFu, c1 = (a >> 14) & 0x7FFu, kd = c0 > c1 ? c0 - c1 : c1 - c0;
-        const double n0 = (double)c0, n1 = (double)c1;
-        const double l0 = n0 * lmaj + n1 * lmin;  // root allele A
-        const double l1 = n1 * lmaj + n0 * lmin;  // root allele B
-        const uint32_t need = a & 3u;
-        if (need == 3u) conflict = true;
-        else if (need == 1u) ll += l0;
-        else if (need == 2u) ll += l1;
-        else ll += fmax(l0, l1) + (kd < (uint32_t)kLsumK ? w.lsum[kd] : log1p(exp(-fabs(l0 - l1))));
+        if ((a & 7u) == 4u && (w.uf[x] & 0xFFFFu) == (uint32_t)x) free_ll += free_term(A, l, a, lmaj, lmin);
     }
-    if (__ballot(conflict)) return -INFINITY;
-    ll = wave_sum(ll);
-    return ll;
+    return ll + wave_sum(free_ll);
 }
 
 // The same likelihood for pedigrees of at most 64*KC people and 32*KC
@@ -302,7 +351,7 @@ struct JobInputs {
 };
 
 template <int KC>
-__device__ double fag_log_likelihood_r(const MsampArgs& A, const JobInputs<KC>& in, const WaveArea& w) {
+__device__ double fag_log_likelihood_r(const MsampArgs& A, const JobInputs<KC>& in, const WaveArea& w, int l) {
     constexpr int KN = KC;  // node chunks: the chunk class covers 2F too
     const int lane = lane_id();
     const int F = A.F, NF = A.N - A.F, nodes = 2 * A.F;
@@ -310,8 +359,8 @@ __device__ double fag_log_likelihood_r(const MsampArgs& A, const JobInputs<KC>& 
 #pragma unroll
     for (int c = 0; c < KC; ++c) g[c] = in.g[c];
     const double lmaj = in.lmaj, lmin = in.lmin;
-    // (the union-find words and accumulators were reset by fag_job while
-    // the job's loads were in flight)
+    // (the nodes' words were reset by fag_job while the job's loads were in
+    // flight)
     // label slots (reset, founder_allele_graph4.cc:543-569): the source of
     // each of a slot's two labels, a founder allele (bit 31 set) or the label
     // slot of the parent it came from
@@ -354,7 +403,8 @@ __device__ double fag_log_likelihood_r(const MsampArgs& A, const JobInputs<KC>& 
             }
         }
     }
-    // edges of the typed people; the founder alleles they touch are marked
+    // the typed people: homozygous ones fix both their founder alleles,
+    // heterozygous ones are edges between them
     uint32_t e[KC];
     bool bad = false;
 #pragma unroll
@@ -368,21 +418,66 @@ __device__ double fag_log_likelihood_r(const MsampArgs& A, const JobInputs<KC>& 
                 x = xy & 0xFFFFu;
                 y = xy >> 16;
             }
-            const uint32_t het = g[c] == G_HETERO ? 1u : 0u;
-            bad |= het && x == y;  // an autozygous heterozygote (:77-81)
-            e[c] = x | (y << 10) | (het << 20) | ((g[c] == G_HOMOZ_B ? 1u : 0u) << 21) | (1u << 22);
-            atomicOr(&w.acc[x], 4u);
-            atomicOr(&w.acc[y], 4u);
+            if (g[c] == G_HETERO) {
+                bad |= x == y;  // an autozygous heterozygote (:77-81)
+                e[c] = x | (y << 10) | kEdge;
+            }
+            mark_person(w, g[c], x, y);
         }
     }
     if (__ballot(bad)) return -INFINITY;
-    // rounds of hooking and compression until a round hooks nothing (each
-    // hooking round removes a component, so at most 2F rounds hook)
+    // fixed alleles pass along the edges until nothing changes
+    bool conflict = false, pending;
+    for (;;) {
+        wave_sync();
+        uint32_t fa[KC], fb[KC];
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+            fa[c] = fb[c] = 0u;
+            if (e[c]) {
+                fa[c] = w.acc[e[c] & 0x3FFu] & 3u;
+                fb[c] = w.acc[(e[c] >> 10) & 0x3FFu] & 3u;
+            }
+        }
+        bool changed = false;
+        pending = false;
+#pragma unroll
+        for (int c = 0; c < KC; ++c)
+            if (e[c]) {
+                if (pass_fixed(w, e[c], fa[c], fb[c], &changed, &conflict)) e[c] = 0u;
+                else pending = true;
+            }
+        if (!__ballot(changed)) break;
+    }
+    uint32_t t[KN];
+#pragma unroll
+    for (int n = 0; n < KN; ++n) {
+        const int x = 64 * n + lane;
+        t[n] = 0u;
+        if (x < nodes) t[n] = w.acc[x];
+    }
+    int nA = 0, nB = 0;
+#pragma unroll
+    for (int n = 0; n < KN; ++n) {
+        conflict |= (t[n] & 3u) == 3u;
+        nA += __popcll(__ballot((t[n] & 3u) == 1u));
+        nB += __popcll(__ballot((t[n] & 3u) == 2u));
+    }
+    if (__ballot(conflict)) return -INFINITY;
+    const double ll = (double)nA * lmaj + (double)nB * lmin;
+    if (!__ballot(pending)) return ll;
+    // components no homozygous person reaches: rounds of hooking and
+    // compression until a round hooks nothing (each hooking round removes a
+    // component, so at most 2F rounds hook); the alleles of an edge differ
     uint32_t ux[KC], uy[KC];
     // every node's compressed word (root | parity << 16), as the LDS holds it
     uint32_t r[KN];
 #pragma unroll
-    for (int n = 0; n < KN; ++n) r[n] = (uint32_t)(64 * n + lane);
+    for (int n = 0; n < KN; ++n) {
+        const int x = 64 * n + lane;
+        r[n] = (uint32_t)x;
+        if (x < nodes) w.uf[x] = (uint32_t)x;
+    }
     bool converged = false;
     for (int round = 0; round <= nodes; ++round) {
         wave_sync();
@@ -400,7 +495,7 @@ __device__ double fag_log_likelihood_r(const MsampArgs& A, const JobInputs<KC>& 
         for (int c = 0; c < KC; ++c) {
             const uint32_t rx = ux[c] & 0xFFFFu, ry = uy[c] & 0xFFFFu;
             if (e[c] && rx != ry) {
-                const uint32_t par = (((ux[c] ^ uy[c]) >> 16) ^ (e[c] >> 20)) & 1u;
+                const uint32_t par = (((ux[c] ^ uy[c]) >> 16) ^ 1u) & 1u;
                 w.uf[rx > ry ? rx : ry] = (rx < ry ? rx : ry) | (par << 16);
                 hooked = true;
             }
@@ -425,57 +520,24 @@ __device__ double fag_log_likelihood_r(const MsampArgs& A, const JobInputs<KC>& 
             if (x < nodes) w.uf[x] = r[n];
         }
     }
-    // the last round's words are compressed: check every edge's parity;
-    // homozygous edges fix their root's allele
+    // the last round's words are compressed: check every edge's parity
     bool illegal = !converged;
 #pragma unroll
-    for (int c = 0; c < KC; ++c) {
-        if (e[c]) {
-            const uint32_t het = (e[c] >> 20) & 1u, allele = (e[c] >> 21) & 1u, px = (ux[c] >> 16) & 1u;
-            illegal |= (((ux[c] ^ uy[c]) >> 16) & 1u) != het;
-            if (!het) atomicOr(&w.acc[ux[c] & 0xFFFFu], 1u << (allele ^ px));
-        }
-    }
+    for (int c = 0; c < KC; ++c)
+        if (e[c]) illegal |= (((ux[c] ^ uy[c]) >> 16) & 1u) != 1u;
     if (__ballot(illegal)) return -INFINITY;
-    // touched marks of every chunk read at once, then each touched node
-    // counted at its root by parity
-    uint32_t t[KN];
-#pragma unroll
-    for (int n = 0; n < KN; ++n) {
-        const int x = 64 * n + lane;
-        t[n] = 0u;
-        if (x < nodes) t[n] = w.acc[x];
-    }
+    // touched nodes without a fixed allele, counted at their root by parity
 #pragma unroll
     for (int n = 0; n < KN; ++n)
-        if (t[n] & 4u) atomicAdd(&w.acc[r[n] & 0xFFFFu], ((r[n] >> 16) & 1u) ? (1u << 14) : (1u << 3));
+        if ((t[n] & 7u) == 4u) atomicAdd(&w.acc[r[n] & 0xFFFFu], ((r[n] >> 16) & 1u) ? (1u << 14) : (1u << 3));
     wave_sync();
-    uint32_t ar[KN];
+    double free_ll = 0.0;
 #pragma unroll
     for (int n = 0; n < KN; ++n) {
         const int x = 64 * n + lane;
-        ar[n] = 0u;
-        if (x < nodes && r[n] == (uint32_t)x) ar[n] = w.acc[x];  // roots only
+        if ((t[n] & 7u) == 4u && r[n] == (uint32_t)x) free_ll += free_term(A, l, w.acc[x], lmaj, lmin);
     }
-    double ll = 0.0;
-    bool conflict = false;
-#pragma unroll
-    for (int n = 0; n < KN; ++n) {
-        const uint32_t a = ar[n];
-        if (!(a & 4u)) continue;  // not a root, or untouched
-        const uint32_t c0 = (a >> 3) & 0x7FFu, c1 = (a >> 14) & 0x7FFu, kd = c0 > c1 ? c0 - c1 : c1 - c0;
-        const double n0 = (double)c0, n1 = (double)c1;
-        const double l0 = n0 * lmaj + n1 * lmin;
-        const double l1 = n1 * lmaj + n0 * lmin;
-        const uint32_t need = a & 3u;
-        if (need == 3u) conflict = true;
-        else if (need == 1u) ll += l0;
-        else if (need == 2u) ll += l1;
-        else ll += fmax(l0, l1) + (kd < (uint32_t)kLsumK ? w.lsum[kd] : log1p(exp(-fabs(l0 - l1))));
-    }
-    if (__ballot(conflict)) return -INFINITY;
-    ll = wave_sum(ll);
-    return ll;
+    return ll + wave_sum(free_ll);
 }
 
 // The forward-backward pass runs in FP64 (SL_FP64 contexts: the reference's
@@ -492,24 +554,28 @@ using Mat = MatT<double>;
 // product with an exact power-of-two rescale keeping the largest entry in
 // [0.5, 1): for a normal largest entry m with biased exponent E the factor is
 // 2^(1022-E) (FP64) or 2^(126-E) (FP32), built from its bits; a subnormal m
-// takes frexp/ldexp
+// takes frexp/ldexp, behind a wavefront-wide test that is seldom taken, so
+// that the usual product has no divergent branch (a pass is one wavefront's
+// instruction chain: with a branch per product it was a third longer)
 __device__ __forceinline__ Mat mmul(const Mat& x, const Mat& y) {
     Mat r{x.a * y.a + x.b * y.c, x.a * y.b + x.b * y.d, x.c * y.a + x.d * y.c, x.c * y.b + x.d * y.d};
     const double m = fmax(fmax(r.a, r.b), fmax(r.c, r.d));
     const uint32_t E = (uint32_t)(__builtin_bit_cast(uint64_t, m) >> 52) & 0x7FFu;
-    if (E != 0u && E < 2045u) {
-        const double f = __builtin_bit_cast(double, (uint64_t)(2045u - E) << 52);
-        r.a *= f;
-        r.b *= f;
-        r.c *= f;
-        r.d *= f;
-    } else if (m > 0.0 && E == 0u) {
-        int e;
-        (void)frexp(m, &e);
-        r.a = ldexp(r.a, -e);
-        r.b = ldexp(r.b, -e);
-        r.c = ldexp(r.c, -e);
-        r.d = ldexp(r.d, -e);
+    const double f = __builtin_bit_cast(double, (uint64_t)(E - 1u < 2044u ? 2045u - E : 1023u) << 52);
+    r.a *= f;
+    r.b *= f;
+    r.c *= f;
+    r.d *= f;
+    const bool sub = m > 0.0 && E == 0u;
+    if (__builtin_expect(__ballot(sub) != 0ull, 0)) {
+        if (sub) {
+            int e;
+            (void)frexp(m, &e);
+            r.a = ldexp(r.a, -e);
+            r.b = ldexp(r.b, -e);
+            r.c = ldexp(r.c, -e);
+            r.d = ldexp(r.d, -e);
+        }
     }
     return r;
 }
@@ -519,18 +585,20 @@ __device__ __forceinline__ MatT<float> mmul(const MatT<float>& x, const MatT<flo
     MatT<float> r{x.a * y.a + x.b * y.c, x.a * y.b + x.b * y.d, x.c * y.a + x.d * y.c, x.c * y.b + x.d * y.d};
     const float m = fmaxf(fmaxf(r.a, r.b), fmaxf(r.c, r.d));
     const uint32_t E = (__float_as_uint(m) >> 23) & 0xFFu;
-    if (E != 0u && E < 253u) {
-        const float f = __uint_as_float((253u - E) << 23);
-        r.a *= f;
-        r.b *= f;
-        r.c *= f;
-        r.d *= f;
-    } else if (m > 0.0f && E == 0u) {
-        const int e = __builtin_amdgcn_frexp_expf(m);
-        r.a = __builtin_amdgcn_ldexpf(r.a, -e);
-        r.b = __builtin_amdgcn_ldexpf(r.b, -e);
-        r.c = __builtin_amdgcn_ldexpf(r.c, -e);
-        r.d = __builtin_amdgcn_ldexpf(r.d, -e);
+    const float f = __uint_as_float((E - 1u < 252u ? 253u - E : 127u) << 23);
+    r.a *= f;
+    r.b *= f;
+    r.c *= f;
+    r.d *= f;
+    const bool sub = m > 0.0f && E == 0u;
+    if (__builtin_expect(__ballot(sub) != 0ull, 0)) {
+        if (sub) {
+            const int e = __builtin_amdgcn_frexp_expf(m);
+            r.a = __builtin_amdgcn_ldexpf(r.a, -e);
+            r.b = __builtin_amdgcn_ldexpf(r.b, -e);
+            r.c = __builtin_amdgcn_ldexpf(r.c, -e);
+            r.d = __builtin_amdgcn_ldexpf(r.d, -e);
+        }
     }
     return r;
 }
@@ -544,7 +612,7 @@ __device__ __forceinline__ uint32_t compose(uint32_t f, uint32_t h) {
 // wave_shr:1 / wave_shl:1 across the wavefront, row_bcast:15 / row_bcast:31
 // from the last lane of a row to the rows above it.  Lanes without a source,
 // and rows outside the row mask, keep `old`.
-constexpr int kDppWaveShl1 = 0x130, kDppWaveShr1 = 0x138, kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143;
+constexpr int kDppWaveShr1 = 0x138, kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143;
 constexpr int dpp_row_shl(int n) { return 0x100 + n; }
 constexpr int dpp_row_shr(int n) { return 0x110 + n; }
 
@@ -606,6 +674,11 @@ __device__ __forceinline__ size_t lflip_index(const MsampArgs& A, int k, int v, 
     return (((size_t)(k & 1) * 2 + (size_t)v) * (size_t)A.n_chains + (size_t)chain) * (size_t)A.M + (size_t)l;
 }
 
+// the uniforms of step k: [step parity][chain][draw index]
+__device__ __forceinline__ size_t udev_index(const MsampArgs& A, int k, int chain) {
+    return ((size_t)(k & 1) * (size_t)A.n_chains + (size_t)chain) * (size_t)A.M;
+}
+
 __device__ __forceinline__ int order_at(const MsampArgs& A, int chain, int k) {
     return A.order[(size_t)chain * A.n_meioses + k];
 }
@@ -614,10 +687,13 @@ __device__ __forceinline__ int order_at(const MsampArgs& A, int chain, int k) {
 //  * with A.with_lcur, jobs [0, M) are the current columns (into lcur; a zero
 //    marks the chain's graph illegal, meiosis_sampler.cc:33-36);
 //  * the other jobs are step A.step's columns with meiosis m_k flipped (into
-//    lflip, MeiosisSampler::step, :116-134).  With A.spec and k > 0, variant
-//    v first forces meiosis m_{k-1}'s bit to v: the forward-backward pass of
-//    step k-1 may be deciding that bit in the same launch, and it is the only
-//    bit it changes.
+//    lflip, MeiosisSampler::step, :116-134), at the loci where that has to be
+//    computed (class kFlipCompute).  With A.spec and k > 0, variant v first
+//    forces meiosis m_{k-1}'s bit to v: the forward-backward pass of step k-1
+//    may be deciding that bit in the same launch, and it is the only bit it
+//    changes.  Where m_{k-1}'s own flip changes nothing or is illegal one job
+//    serves both variants: the bit's value does not matter (it is taken as 0),
+//    or it cannot change.
 template <int KC>
 __device__ void fag_job(const MsampArgs& A, int chain, int q, const uint2* ptab, unsigned char* wbase) {
     const int lane = lane_id(), M = A.M;
@@ -625,57 +701,66 @@ __device__ void fag_job(const MsampArgs& A, int chain, int q, const uint2* ptab,
     // graph is illegal keeps its buffers as they are
     const int status = A.status[chain];
     int l, v = 0, flip = -1, force = -1;
-    bool current = false;
+    int fc = kFlipCompute, pc = kFlipCompute;
+    bool current = false, two = false;
     if (A.with_lcur && q < M) {
         l = q;
         current = true;
     } else {
-        // with two variants (A.spec, k > 0), jobs 2l and 2l+1 share a
-        // workgroup, and so an XCD's L2, for locus l's column
+        // with two variants (A.spec, k > 0), jobs 2e and 2e+1 share a
+        // workgroup, and so an XCD's L2, for their locus's column
         const int r = A.with_lcur ? q - M : q;
-        const bool two = A.spec && A.step > 0;
+        two = A.spec && A.step > 0;
         v = two ? (r & 1) : 0;
-        l = two ? (r >> 1) : r;
+        const int e = two ? (r >> 1) : r;
         flip = order_at(A, chain, A.step);
         if (two) force = order_at(A, chain, A.step - 1);
+        if (A.compact) {
+            // an illegal chain's order may be stale
+            if (status != 0 || e >= A.jobcnt[flip]) return;
+            l = A.joblist[(size_t)flip * M + e];
+        } else {
+            // the class is read beside the job's data, whatever the status;
+            // a stale order may hold anything
+            l = e;
+            const int top = 2 * (A.N - A.F) - 1;
+            fc = A.cls[(size_t)min((uint32_t)flip, (uint32_t)top) * M + l];
+            if (two) force = (int)min((uint32_t)force, (uint32_t)top);
+        }
+        if (two) pc = A.cls[(size_t)force * M + l];
     }
     WaveArea w = wave_area(A, wbase);
     const uint32_t* src = A.graphs + ((size_t)chain * M + l) * A.W;
     // where the likelihood goes, formed before the work that produces it
     double* const dst = current ? A.lcur + (size_t)chain * M + l : A.lflip + lflip_index(A, A.step, v, chain, l);
+    if (pc == kFlipIllegal) force = -1;
+    const bool serves_both = two && pc != kFlipCompute;
+    double* const dst1 = serves_both ? A.lflip + lflip_index(A, A.step, 1, chain, l) : nullptr;
     JobInputs<KC> in;
     if constexpr (KC > 0) {
         in.load(A, l);
-        // every node its own root with nothing counted, written while the
-        // loads above are in flight
+        // no node fixed or touched, written while the loads above are in flight
 #pragma unroll
         for (int n = 0; n < KC; ++n) {
             const int x = 64 * n + lane;
-            if (x < 2 * A.F) {
-                w.uf[x] = (uint32_t)x;
-                w.acc[x] = 0u;
-            }
+            if (x < 2 * A.F) w.acc[x] = 0u;
         }
     }
-    static_assert(kLsumK % 64 == 0, "the term row is copied 64 entries at a time");
-    double ls[kLsumK / 64];
-#pragma unroll
-    for (int j = 0; j < kLsumK / 64; ++j) ls[j] = A.lsum[(size_t)l * kLsumK + 64 * j + lane];
     for (int k = lane; k < A.W; k += 64) {
         uint32_t x = src[k];
         if (force >= 0 && (force >> 5) == k) x = (x & ~(1u << (force & 31))) | ((uint32_t)v << (force & 31));
         if (flip >= 0 && (flip >> 5) == k) x ^= 1u << (flip & 31);
         w.colw[k] = x;
     }
-#pragma unroll
-    for (int j = 0; j < kLsumK / 64; ++j) w.lsum[64 * j + lane] = ls[j];
+    if (fc != kFlipCompute || (serves_both && v)) return;
     wave_sync();
     double L;
-    if constexpr (KC > 0) L = fag_log_likelihood_r<KC>(A, in, w);
+    if constexpr (KC > 0) L = fag_log_likelihood_r<KC>(A, in, w, l);
     else L = fag_log_likelihood(A, ptab, w, l);
     if (status != 0) return;
     if (lane == 0) {
         *dst = L;
+        if (serves_both) *dst1 = L;
         if (current && L == -INFINITY) A.status[chain] = kIllegalGraph;
     }
 }
@@ -687,7 +772,10 @@ struct StepView {
     int chain, k, word, pword;
     uint32_t bm, pbm;
     bool spec;
-    __device__ __forceinline__ double lf(const uint32_t* g, int l) const {
+    const uint8_t* cls;  // the classes of m_k's flip by locus
+    __device__ __forceinline__ double lf(const uint32_t* g, int l, double lcur) const {
+        const int c = cls[l];
+        if (c != kFlipCompute) return c == kFlipSame ? lcur : -INFINITY;
         const int v = spec ? ((g[(size_t)l * A->W + pword] & pbm) ? 1 : 0) : 0;
         return A->lflip[lflip_index(*A, k, v, chain, l)];
     }
@@ -775,19 +863,14 @@ __device__ __forceinline__ uint32_t locus_map_u(bool last, double theta, T f0, T
         // an FP32 underflow of a state the FP64 pass keeps is counted
         if (draws && !(w0[0] != 0.0f && w1[0] != 0.0f && w0[1] != 0.0f && w1[1] != 0.0f)) ++*near;
     }
+    // w0 = 0 gives a threshold of 0 (0/0: NaN) and so bit 1, w1 = 0 one of 1 and
+    // so bit 0, for any u in [0, 1)
     uint32_t map = 0;
 #pragma unroll
     for (int bn = 0; bn < 2; ++bn) {
-        uint32_t b, edge = 0;
-        if (w0[bn] == (T)0) {
-            b = 1u;
-        } else if (w1[bn] == (T)0) {
-            b = 0u;
-        } else {
-            const double thr = (double)(w0[bn] / (w0[bn] + w1[bn]));
-            b = u < thr ? 0u : 1u;
-            edge = fabs(u - thr) < edge_tol<T>() ? 1u : 0u;
-        }
+        const double thr = (double)(w0[bn] / (w0[bn] + w1[bn]));
+        const uint32_t b = u < thr ? 0u : 1u;
+        const uint32_t edge = w0[bn] != (T)0 && w1[bn] != (T)0 && fabs(u - thr) < edge_tol<T>() ? 1u : 0u;
         map |= (b << bn) | (edge << (2 + bn));
     }
     return map;
@@ -802,10 +885,12 @@ __device__ __forceinline__ uint32_t locus_map(const MsampArgs& A, int chain, int
 
 // exclusive left-to-right product of the threads' segment products: within
 // wavefronts by DPP, across them through LDS (by one row of lanes when there
-// are more than four)
+// are more than four).  The one barrier also publishes what the caller wrote
+// to LDS before.
 template <typename T>
 __device__ __forceinline__ MatT<T> scan_products(MatT<T> P, MatT<T>* wtot) {
-    const int lane = lane_id(), wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int lane = lane_id(), nw = blockDim.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     P = wave_products(P);
     if (lane == 63) wtot[wave] = P;
     __syncthreads();
@@ -817,13 +902,50 @@ __device__ __forceinline__ MatT<T> scan_products(MatT<T> P, MatT<T>* wtot) {
         Q = mmul(mat_dpp<dpp_row_shr(1)>(Q), Q);
         Q = mmul(mat_dpp<dpp_row_shr(2)>(Q), Q);
         Q = mmul(mat_dpp<dpp_row_shr(4)>(Q), Q);
-        Q = mmul(mat_dpp<dpp_row_shr(8)>(Q), Q);
-        const int wu = __builtin_amdgcn_readfirstlane(wave);
-        if (wu > 0)
-            R = MatT<T>{readlane_t(Q.a, wu - 1), readlane_t(Q.b, wu - 1), readlane_t(Q.c, wu - 1),
-                        readlane_t(Q.d, wu - 1)};
+        if (nw > 8) Q = mmul(mat_dpp<dpp_row_shr(8)>(Q), Q);  // lanes below 8 have no source
+        if (wave > 0)
+            R = MatT<T>{readlane_t(Q.a, wave - 1), readlane_t(Q.b, wave - 1), readlane_t(Q.c, wave - 1),
+                        readlane_t(Q.d, wave - 1)};
     }
     return mmul(R, mat_dpp<kDppWaveShr1>(P));
+}
+
+// Draws and decision maps are single bits per (thread, locus of its segment),
+// so their scans across a wavefront are ballots: a suffix count is the number
+// of set bits above the lane, and a composition of 2-bit maps is the nearest
+// constant map above, inverted by each inverting map on the way.
+
+// bits of m above this lane
+__device__ __forceinline__ uint32_t count_above(uint64_t m) {
+    const uint32_t upto = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+    return (uint32_t)__popcll(m) - upto - (uint32_t)((m >> lane_id()) & 1ull);
+}
+
+// the total over the wavefronts after this one of per-wavefront counts
+__device__ __forceinline__ uint32_t counts_after(const uint32_t* wcnt) {
+    const int lane = lane_id(), wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    uint32_t v = lane < nw && lane > wave ? wcnt[lane] : 0u;
+    v += u32_dpp<dpp_row_shr(1)>(0u, v);
+    v += u32_dpp<dpp_row_shr(2)>(0u, v);
+    v += u32_dpp<dpp_row_shr(4)>(0u, v);
+    v += u32_dpp<dpp_row_shr(8)>(0u, v);
+    return readlane_u32(v, 15);  // at most 16 wavefronts
+}
+
+// per-thread bit counts v (a ballot per locus of the segments, formed by the
+// caller's masks): the sum over the threads after this one; wave_total is the
+// wavefront's sum
+template <int SM>
+__device__ __forceinline__ uint32_t sum_above_bits(uint32_t bits, uint32_t* wave_total) {
+    uint32_t r = 0, tot = 0;
+#pragma unroll
+    for (int s = 0; s < SM; ++s) {
+        const uint64_t m = __ballot((bits >> s) & 1u);
+        r += count_above(m);
+        tot += (uint32_t)__popcll(m);
+    }
+    *wave_total = tot;
+    return r;
 }
 
 // within a wavefront: inclusive suffix sums of v (this lane and the lanes
@@ -840,69 +962,38 @@ __device__ __forceinline__ uint32_t wave_suffix_sums(uint32_t v) {
     return sc + (row < 1 ? t1 : 0u) + (row < 2 ? t2 : 0u) + (row < 3 ? t3 : 0u);
 }
 
-// scan_products and sum_above in one exchange between wavefronts: the
-// exclusive product before this thread's segment, and in *above the sum of v
-// over the threads after this one
-template <typename T>
-__device__ __forceinline__ MatT<T> scan_products_counts(MatT<T> P, uint32_t v, MatT<T>* wtot, uint32_t* wcnt,
-                                                        uint32_t* above) {
-    const int lane = lane_id(), wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    P = wave_products(P);
-    const uint32_t sc = wave_suffix_sums(v);
-    if (lane == 63) wtot[wave] = P;
-    if (lane == 0) wcnt[wave] = sc;
-    __syncthreads();
-    uint32_t r = sc - v;
-    for (int q = wave + 1; q < nw; ++q) r += wcnt[q];
-    *above = r;
-    MatT<T> R{(T)1, (T)0, (T)0, (T)1};
-    if (nw <= 4) {
-        for (int q = 0; q < wave; ++q) R = mmul(R, wtot[q]);
-    } else {
-        MatT<T> Q = lane < nw ? wtot[lane] : MatT<T>{(T)1, (T)0, (T)0, (T)1};
-        Q = mmul(mat_dpp<dpp_row_shr(1)>(Q), Q);
-        Q = mmul(mat_dpp<dpp_row_shr(2)>(Q), Q);
-        Q = mmul(mat_dpp<dpp_row_shr(4)>(Q), Q);
-        Q = mmul(mat_dpp<dpp_row_shr(8)>(Q), Q);
-        const int wu = __builtin_amdgcn_readfirstlane(wave);
-        if (wu > 0)
-            R = MatT<T>{readlane_t(Q.a, wu - 1), readlane_t(Q.b, wu - 1), readlane_t(Q.c, wu - 1),
-                        readlane_t(Q.d, wu - 1)};
-    }
-    return mmul(R, mat_dpp<kDppWaveShr1>(P));
-}
-
 // sum of v over the threads after this one
 __device__ __forceinline__ uint32_t sum_above(uint32_t v, uint32_t* wcnt) {
-    const int lane = lane_id(), wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int lane = lane_id(), wave = threadIdx.x >> 6;
     const uint32_t sc = wave_suffix_sums(v);
     if (lane == 0) wcnt[wave] = sc;
     __syncthreads();
-    uint32_t r = sc - v;
-    for (int q = wave + 1; q < nw; ++q) r += wcnt[q];
-    return r;
+    return sc - v + counts_after(wcnt);
+}
+
+// image of anything under the composition of the maps of the lanes in `sel`
+// (lowest applied last): cst: constant maps, one: those giving 1, neg:
+// inverting maps; `in` enters above the topmost lane
+__device__ __forceinline__ uint32_t through_maps(uint64_t cst, uint64_t one, uint64_t neg, uint32_t in) {
+    const int j = cst ? __ffsll((unsigned long long)cst) - 1 : 64;
+    const uint64_t below = j < 64 ? (1ull << j) - 1ull : ~0ull;
+    const uint32_t v = cst ? (uint32_t)((one >> j) & 1ull) : in;
+    return v ^ ((uint32_t)__popcll(neg & below) & 1u);
 }
 
 // indicator entering this thread's segment from above: the composition of the
 // segment maps of every later thread applied to anything (the map of locus M-1
 // is constant, so the composite is too)
 __device__ __forceinline__ uint32_t bit_from_above(uint32_t comp, uint32_t* wmap) {
-    const int lane = lane_id(), wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    uint32_t sc = comp;  // this map composed with every later one, within rows, then across them
-    sc = compose(sc, u32_dpp<dpp_row_shl(1)>(2u, sc));
-    sc = compose(sc, u32_dpp<dpp_row_shl(2)>(2u, sc));
-    sc = compose(sc, u32_dpp<dpp_row_shl(4)>(2u, sc));
-    sc = compose(sc, u32_dpp<dpp_row_shl(8)>(2u, sc));
-    const uint32_t t3 = readlane_u32(sc, 48);
-    const uint32_t t2 = compose(readlane_u32(sc, 32), t3);
-    const uint32_t t1 = compose(readlane_u32(sc, 16), t2);
-    const int row = lane >> 4;
-    sc = compose(sc, row == 0 ? t1 : row == 1 ? t2 : row == 2 ? t3 : 2u);
-    if (lane == 0) wmap[wave] = sc;
+    const int lane = lane_id(), nw = blockDim.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint64_t cst = __ballot(comp == 0u || comp == 3u), one = __ballot(comp == 3u), neg = __ballot(comp == 1u);
+    if (lane == 0) wmap[wave] = through_maps(cst, one, neg, 0u) | (through_maps(cst, one, neg, 1u) << 1);
     __syncthreads();
-    uint32_t up = 2u;
-    for (int q = nw - 1; q > wave; --q) up = compose(wmap[q], up);
-    return compose(u32_dpp<kDppWaveShl1>(2u, sc), up) & 1u;
+    const uint32_t wm = lane < nw && lane > wave ? wmap[lane] : 2u;
+    const uint32_t up = through_maps(__ballot(wm == 0u || wm == 3u), __ballot(wm == 3u), __ballot(wm == 1u), 0u);
+    const uint64_t above = lane < 63 ? ~0ull << (lane + 1) : 0ull;
+    return through_maps(cst & above, one, neg & above, up);
 }
 
 // Forward-backward pass of step k on one chain by the whole workgroup; thread
@@ -911,9 +1002,8 @@ __device__ __forceinline__ uint32_t bit_from_above(uint32_t comp, uint32_t* wmap
 // whose likelihoods, forward probabilities and maps stay in registers; SM = 0:
 // any length, through the chain's global scratch.  T: the arithmetic of the
 // forward values and thresholds.  A chain whose status is set or whose sweep
-// is an L-sweep is left as it is.  ubuf (SM > 0, may be null): LDS for M
-// uniforms, filled with draw indices 0..M-1 of the step while the loads are
-// in flight.
+// is an L-sweep is left as it is.  ubuf (SM > 0, may be null): LDS for the M
+// uniforms that draw indices 0..M-1 of the step take.
 template <int SM, typename T>
 __device__ void forward_backward(const MsampArgs& A, int chain, int k, MatT<T>* wtot, uint32_t* wcnt,
                                  uint32_t* wmap, double* ubuf) {
@@ -930,6 +1020,7 @@ __device__ void forward_backward(const MsampArgs& A, int chain, int k, MatT<T>* 
     sv.word = m >> 5;
     sv.bm = 1u << (m & 31);
     sv.spec = A.spec && k > 0;
+    sv.cls = A.cls + (size_t)m * M;
     const int pm = sv.spec ? order_at(A, chain, k - 1) : 0;
     if (status != 0) return;
     sv.pword = pm >> 5;
@@ -946,6 +1037,7 @@ __device__ void forward_backward(const MsampArgs& A, int chain, int k, MatT<T>* 
         // m_{k-1}, the current column's likelihood, both flipped variants and
         // the thetas of the segment's intervals
         uint32_t gw[SM], pw[SM];
+        int cl[SM];
         double lcv[SM], lf0[SM], lf1[SM], thv[SM + 1];
 #pragma unroll
         for (int s = 0; s <= SM; ++s) {
@@ -957,7 +1049,9 @@ __device__ void forward_backward(const MsampArgs& A, int chain, int k, MatT<T>* 
             const int l = a0 + s;
             gw[s] = pw[s] = 0u;
             lcv[s] = lf0[s] = lf1[s] = 0.0;
+            cl[s] = kFlipCompute;
             if (l < a1) {
+                cl[s] = sv.cls[l];
                 gw[s] = g[(size_t)l * A.W + word];
                 lcv[s] = lc[l];
                 lf0[s] = A.lflip[lflip_index(A, k, 0, chain, l)];
@@ -967,11 +1061,17 @@ __device__ void forward_backward(const MsampArgs& A, int chain, int k, MatT<T>* 
                 }
             }
         }
-        // the step's uniforms by draw index, while the loads are in flight
-        // (the first barrier of the scans below publishes them)
-        if (ubuf)
-            for (int i = tid; i < M; i += B)
-                ubuf[i] = philox_uniform(A.seed, (uint32_t)chain, sweep_of(A), (uint32_t)k, (uint32_t)i);
+        // the step's uniforms by draw index, drawn beside the step's
+        // likelihoods (the first barrier of the scans below publishes them)
+        if (ubuf) {
+            const double* ud = A.udev + udev_index(A, k, chain);
+            double uv[SM];
+#pragma unroll
+            for (int s = 0; s < SM; ++s) uv[s] = tid + s * B < M ? ud[tid + s * B] : 0.0;
+#pragma unroll
+            for (int s = 0; s < SM; ++s)
+                if (tid + s * B < M) ubuf[tid + s * B] = uv[s];
+        }
         T e0[SM], e1[SM], f0[SM], f1[SM];
         double lfv[SM];
         uint32_t curm = 0, drm = 0, both = 0;
@@ -979,6 +1079,7 @@ __device__ void forward_backward(const MsampArgs& A, int chain, int k, MatT<T>* 
         for (int s = 0; s < SM; ++s) {
             const bool cur = (gw[s] & bm) != 0;
             lfv[s] = (pw[s] & sv.pbm) ? lf1[s] : lf0[s];
+            if (cl[s] != kFlipCompute) lfv[s] = cl[s] == kFlipSame ? lcv[s] : -INFINITY;
             e0[s] = e1[s] = (T)0;
             if (a0 + s < a1) both |= (emissions(cur, lcv[s], lfv[s], &e0[s], &e1[s]) ? 1u : 0u) << s;
             curm |= (cur ? 1u : 0u) << s;
@@ -990,16 +1091,15 @@ __device__ void forward_backward(const MsampArgs& A, int chain, int k, MatT<T>* 
         // the backward pass runs from the last locus down, so a drawing
         // locus's draw index counts the draws of later threads and of the
         // later loci of this segment.  FP32 draws where FP64 emissions allow
-        // both states, known before the forward pass: one exchange carries
-        // both scans
-        MatT<T> R;
-        uint32_t cnt;
+        // both states, known before the forward pass: the products' barrier
+        // then publishes the counts too
+        uint32_t cnt, wtotal;
         if constexpr (sizeof(T) == 4) {
             drm = both;
-            R = scan_products_counts(P, (uint32_t)__popc(drm), wtot, wcnt, &cnt);
-        } else {
-            R = scan_products(P, wtot);
+            cnt = sum_above_bits<SM>(drm, &wtotal);
+            if (lane_id() == 0) wcnt[tid >> 6] = wtotal;
         }
+        MatT<T> R = scan_products(P, wtot);
 #pragma unroll
         for (int s = 0; s < SM; ++s) {
             f0[s] = f1[s] = (T)0;
@@ -1014,7 +1114,12 @@ __device__ void forward_backward(const MsampArgs& A, int chain, int k, MatT<T>* 
                 }
             }
         }
-        if constexpr (sizeof(T) == 8) cnt = sum_above((uint32_t)__popc(drm), wcnt);
+        if constexpr (sizeof(T) == 8) {
+            cnt = sum_above_bits<SM>(drm, &wtotal);
+            if (lane_id() == 0) wcnt[tid >> 6] = wtotal;
+            __syncthreads();
+        }
+        cnt += counts_after(wcnt);
         uint32_t mp[SM];
 #pragma unroll
         for (int s = 0; s < SM; ++s) {
@@ -1051,7 +1156,7 @@ __device__ void forward_backward(const MsampArgs& A, int chain, int k, MatT<T>* 
         uint8_t* mp = A.maps + (size_t)chain * M;
         auto locus = [&](int l, bool* both) {
             T e0, e1;
-            const bool b = emissions((g[(size_t)l * A.W + word] & bm) != 0, lc[l], sv.lf(g, l), &e0, &e1);
+            const bool b = emissions((g[(size_t)l * A.W + word] & bm) != 0, lc[l], sv.lf(g, l, lc[l]), &e0, &e1);
             if (both) *both = b;
             return emission_matrix(A, e0, e1, l);
         };
@@ -1085,7 +1190,7 @@ __device__ void forward_backward(const MsampArgs& A, int chain, int k, MatT<T>* 
             near += (map >> (2 + next)) & 1u;
             uint32_t* wp = g + (size_t)l * A.W + word;
             if (nb != ((*wp & bm) ? 1u : 0u)) {
-                lc[l] = sv.lf(g, l);
+                lc[l] = sv.lf(g, l, lc[l]);
                 *wp ^= bm;
             }
             next = nb;
@@ -1101,6 +1206,17 @@ template <int KC>
 __device__ __forceinline__ void run_jobs(const MsampArgs& A, int chain, int block, unsigned char* smem) {
     if (!is_msweep(A, chain)) return;
     const int nw = blockDim.x >> 6, wave = threadIdx.x >> 6;
+    const int job_blocks = (A.n_jobs + nw - 1) / nw;
+    if (block >= job_blocks) {
+        // the workgroups past the jobs draw the step's uniforms: a Philox
+        // call is 20 quarter-rate multiplies, which the forward-backward
+        // pass's one workgroup would wait for
+        const int i = (block - job_blocks) * (int)blockDim.x + (int)threadIdx.x;
+        if (i < A.M)
+            A.udev[udev_index(A, A.step, chain) + i] =
+                philox_uniform(A.seed, (uint32_t)chain, sweep_of(A), (uint32_t)A.step, (uint32_t)i);
+        return;
+    }
     uint2* ptab = reinterpret_cast<uint2*>(smem);
     if constexpr (KC == 0) {
         for (int k = threadIdx.x; k < A.N - A.F; k += blockDim.x) ptab[k] = A.ptab[k];
@@ -1108,6 +1224,92 @@ __device__ __forceinline__ void run_jobs(const MsampArgs& A, int chain, int bloc
     }
     const int q = block * nw + wave;
     if (q < A.n_jobs) fag_job<KC>(A, chain, q, ptab, smem + A.ptab_bytes + (size_t)wave * A.wave_bytes);
+}
+
+// What flipping a meiosis does to a legal column, for every meiosis and locus,
+// by genotype elimination (a descent graph only adds constraints, so what no
+// assignment of phased genotypes to the family allows, no column allows).  A
+// thread per locus keeps each person's possible (maternal, paternal) alleles
+// as a 4-bit mask, bit 2 maternal + paternal, and narrows every trio down and
+// up the generations until nothing changes.  Any narrowing is sound, so the
+// rounds are bounded; two or three settle.  For a meiosis of person p from
+// parent q:
+//  * q cannot be heterozygous: in every assignment consistent with a column q's
+//    two founder alleles are equal, so exchanging them in the edges below p
+//    keeps every constraint: flipping the bit leaves the likelihood as it is;
+//  * q is heterozygous with known phase and the allele p took from q is known:
+//    the bit is fixed, and the flipped column has no consistent assignment.
+// At ped150 (10% missing) 55% of the (meiosis, locus) pairs are the first,
+// and together about two thirds need no founder-allele graph.
+constexpr int kClassBlock = 64;
+constexpr int kClassRounds = 8;
+
+__device__ __forceinline__ uint32_t transmits(uint32_t m) { return ((m & 0x7u) ? 1u : 0u) | ((m & 0xEu) ? 2u : 0u); }
+__device__ __forceinline__ uint32_t maternal_alleles(uint32_t m) {
+    return ((m & 0x3u) ? 1u : 0u) | ((m & 0xCu) ? 2u : 0u);
+}
+__device__ __forceinline__ uint32_t paternal_alleles(uint32_t m) {
+    return ((m & 0x5u) ? 1u : 0u) | ((m & 0xAu) ? 2u : 0u);
+}
+__device__ __forceinline__ uint32_t carries(uint32_t s) { return ((s & 1u) ? 0x7u : 0u) | ((s & 2u) ? 0xEu : 0u); }
+
+__global__ void __launch_bounds__(kClassBlock) mclass_kernel(MsampArgs A, uint8_t* masks, uint8_t* cls) {
+    const int l = blockIdx.x * kClassBlock + threadIdx.x;
+    if (l >= A.M) return;
+    const int M = A.M, F = A.F, NF = A.N - F;
+    uint8_t* mk = masks + l;
+    for (int i = 0; i < A.N; ++i) {
+        const int g = genotype_at(A, l, i);
+        mk[(size_t)i * M] = g == 0 ? 0xFu : g == G_HETERO ? 0x6u : g == G_HOMOZ_B ? 0x8u : 0x1u;
+    }
+    for (int round = 0; round < kClassRounds; ++round) {
+        bool changed = false;
+        for (int j = 0; j < 2 * NF; ++j) {
+            const uint2 e = A.ptab[j < NF ? j : 2 * NF - 1 - j];  // down the generations, then up
+            uint8_t* pc = mk + (size_t)(e.x & 0xFFFFu) * M;
+            uint8_t* pm = mk + (size_t)(e.y & 0xFFFFu) * M;
+            uint8_t* pf = mk + (size_t)(e.y >> 16) * M;
+            const uint32_t c = *pc, mo = *pm, fa = *pf;
+            const uint32_t tm = transmits(mo), tf = transmits(fa);
+            const uint32_t c2 = c & (((tm & 1u) ? 0x3u : 0u) | ((tm & 2u) ? 0xCu : 0u)) &
+                                (((tf & 1u) ? 0x5u : 0u) | ((tf & 2u) ? 0xAu : 0u));
+            const uint32_t m2 = mo & carries(maternal_alleles(c2)), f2 = fa & carries(paternal_alleles(c2));
+            if (c2 != c) *pc = (uint8_t)c2;
+            if (m2 != mo) *pm = (uint8_t)m2;
+            if (f2 != fa) *pf = (uint8_t)f2;
+            changed |= c2 != c || m2 != mo || f2 != fa;
+        }
+        if (!changed) break;
+    }
+    for (int j = 0; j < NF; ++j) {
+        const uint2 e = A.ptab[j];
+        const int p = (int)(e.x & 0xFFFFu);
+        const uint32_t c = mk[(size_t)p * M];
+#pragma unroll
+        for (int side = 0; side < 2; ++side) {
+            const uint32_t q = mk[(size_t)(side ? e.y >> 16 : e.y & 0xFFFFu) * M];
+            const uint32_t got = side ? paternal_alleles(c) : maternal_alleles(c);
+            int k = kFlipCompute;
+            if (q != 0u && (q & 0x6u) == 0u) k = kFlipSame;
+            else if ((q == 0x2u || q == 0x4u) && (got == 1u || got == 2u)) k = kFlipIllegal;
+            cls[(size_t)(2 * (p - F) + side) * M + l] = (uint8_t)k;
+        }
+    }
+}
+
+// the kFlipCompute loci of meiosis blockIdx.x, ascending; one wavefront
+__global__ void __launch_bounds__(64) mjobs_kernel(int M, const uint8_t* cls, int32_t* joblist, int32_t* jobcnt) {
+    const int b = blockIdx.x, lane = threadIdx.x;
+    const uint64_t below = (1ull << lane) - 1ull;
+    int n = 0;
+    for (int l0 = 0; l0 < M; l0 += 64) {
+        const int l = l0 + lane;
+        const bool take = l < M && cls[(size_t)b * M + l] == kFlipCompute;
+        const uint64_t mask = __ballot(take);
+        if (take) joblist[(size_t)b * M + n + __popcll(mask & below)] = l;
+        n += __popcll(mask);
+    }
+    if (lane == 0) jobcnt[b] = n;
 }
 
 // founder-allele likelihood jobs only; grid (jobs / waves, chains).  KC > 0:
@@ -1271,7 +1473,7 @@ int msampler_people_chunks(int N, int F) {
 }
 
 size_t msampler_wave_bytes(int N, int F, int W) {
-    const size_t b = sizeof(double) * kLsumK + 4 * (size_t)W + 2 * 4 * (size_t)(2 * F) + 4 * (size_t)N +
+    const size_t b = 4 * (size_t)W + 2 * 4 * (size_t)(2 * F) + 4 * (size_t)N +
                      2 * 2 * (size_t)(N - F);
     return (b + 15) / 16 * 16;
 }
@@ -1283,6 +1485,13 @@ size_t msampler_lds_bytes(const MsampArgs& A, int block) {
 }
 
 namespace {
+
+// workgroups of `block` threads for a launch's jobs and, where the passes read
+// them, its step's uniforms
+int job_blocks(const MsampArgs& A, int block) {
+    const int nw = block / 64;
+    return (A.n_jobs + nw - 1) / nw + (A.fb_ubuf && A.draw_uniforms ? (A.M + block - 1) / block : 0);
+}
 
 hipError_t set_lds(const void* kernel, size_t b) {
     if (b <= 64 * 1024) return hipSuccess;
@@ -1310,9 +1519,8 @@ hipError_t set_lds_kc(size_t job, size_t spec) {
 
 template <int KC, typename T>
 void launch_mspec_kc(const MsampArgs& A, size_t lds, hipStream_t s) {
-    const int nw = kSpecBlock / 64;
     const int seg = (A.M + kSpecBlock - 1) / kSpecBlock;
-    const dim3 grid(1 + (A.n_jobs + nw - 1) / nw, A.n_chains), block(kSpecBlock);
+    const dim3 grid(1 + job_blocks(A, kSpecBlock), A.n_chains), block(kSpecBlock);
     if (seg <= 1) hipLaunchKernelGGL((mspec_kernel<1, KC, T>), grid, block, lds, s, A);
     else if (seg <= 2) hipLaunchKernelGGL((mspec_kernel<2, KC, T>), grid, block, lds, s, A);
     else if (seg <= 4) hipLaunchKernelGGL((mspec_kernel<4, KC, T>), grid, block, lds, s, A);
@@ -1352,14 +1560,22 @@ hipError_t configure_msampler_lds(size_t job_lds, size_t spec_lds) {
     return e;
 }
 
+hipError_t launch_mclass(const MsampArgs& A, uint8_t* masks, uint8_t* cls, int32_t* joblist, int32_t* jobcnt,
+                         hipStream_t s) {
+    hipLaunchKernelGGL(mclass_kernel, dim3((A.M + kClassBlock - 1) / kClassBlock), dim3(kClassBlock), 0, s, A, masks,
+                       cls);
+    hipLaunchKernelGGL(mjobs_kernel, dim3(2 * (A.N - A.F)), dim3(64), 0, s, A.M, cls, joblist, jobcnt);
+    return hipGetLastError();
+}
+
 hipError_t launch_morder(const MsampArgs& A, const int32_t* fixed_order, hipStream_t s) {
     hipLaunchKernelGGL(morder_kernel, dim3(A.n_chains), dim3(kOrderBlock), 0, s, A, fixed_order);
     return hipGetLastError();
 }
 
 hipError_t launch_mstep(const MsampArgs& A, size_t lds, hipStream_t s) {
-    const int nw = kMsampBlock / 64;
-    const dim3 grid((A.n_jobs + nw - 1) / nw, A.n_chains);
+    const dim3 grid(job_blocks(A, kMsampBlock), A.n_chains);
+    if (grid.x == 0) return hipSuccess;  // no flip needs a graph
     switch (A.people_chunks) {
         case 2: hipLaunchKernelGGL(mstep_kernel<2>, grid, dim3(kMsampBlock), lds, s, A); break;
         case 3: hipLaunchKernelGGL(mstep_kernel<3>, grid, dim3(kMsampBlock), lds, s, A); break;

@@ -35,6 +35,11 @@ struct MsampArgs {
     const int32_t* meioses;       // [n_meioses] non-ignorable meioses (bit index 2(p-F)+parent)
     int n_meioses;                // meioses sampled by this sweep
     int32_t* order;               // [chains][n_meioses] this sweep's meiosis order
+    const uint8_t* cls;           // [2(N-F)][M] what flipping meiosis b at locus l does to a legal column
+                                  // (kFlipCompute, kFlipSame, kFlipIllegal)
+    const int32_t* joblist;       // [2(N-F)][M] the kFlipCompute loci of each meiosis, ascending
+    const int32_t* jobcnt;        // [2(N-F)] how many
+    int compact;                  // 1: a step's jobs are taken from joblist; 0: job index = locus
     uint32_t* graphs;             // [chains][M][W]
     double* lcur;                 // [chains][M] log-likelihood of the current column
     double* lflip;                // [2 step parities][2 variants][chains][M] flipped-column log-likelihoods
@@ -59,12 +64,23 @@ struct MsampArgs {
     int fp32;                     // 1: the forward-backward pass in FP32 (FP32-rescaled contexts)
     int fb_ubuf;                  // 1: forward-backward launches carry M doubles of dynamic LDS for the
                                   //    step's uniforms (mspec: within its dynamic LDS)
+    int draw_uniforms;            // 1: this job launch also draws step `step`'s uniforms into udev
+    double* udev;                 // [2 step parities][chains][M] uniforms of a step by draw index
 };
 
 // Loci up to which a forward-backward pass keeps the step's uniforms in LDS
 constexpr int kFbUbufLoci = 4096;
 // Entries per locus of MsampArgs::lsum (count differences past it are computed)
 constexpr int kLsumK = 64;
+
+// Classes of MsampArgs::cls, from genotype elimination alone (so of every chain)
+constexpr int kFlipCompute = 0;  // the flipped column's likelihood has to be computed
+constexpr int kFlipSame = 1;     // the parent is homozygous in every consistent assignment: same likelihood
+constexpr int kFlipIllegal = 2;  // the transmitted allele is known: the flipped column is illegal
+
+// Fills cls, joblist and jobcnt of A for its 2(N-F) meioses; masks: N x M bytes of scratch.
+hipError_t launch_mclass(const MsampArgs& A, uint8_t* masks, uint8_t* cls, int32_t* joblist, int32_t* jobcnt,
+                         hipStream_t s);
 
 bool msampler_supported(int N, int F);
 int msampler_people_chunks(int N, int F);  // register chunks for N people, F founders; 0 when too many

@@ -1,0 +1,62 @@
+"""M-sweeps over families and maps where the flip classes and the founder-allele
+components take every form: fully typed (most flips need no graph), sparsely
+typed (components no homozygous person reaches), map lengths around the 64 loci
+of a job list's chunk, one and several chains (job index = locus, and job
+lists)."""
+import numpy as np
+import pytest
+
+from oracle_lib import Oracle
+from swiftlink_amd import native, synth
+from test_gpu_msampler import shuffled_order
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", (native.SL_MSAMPLER_AUTO, native.SL_MSAMPLER_TWO_LAUNCH,
+                                  native.SL_MSAMPLER_TWO_LAUNCH | native.SL_MSAMPLER_LDS_GRAPHS))
+@pytest.mark.parametrize("markers,missing", ((63, 0.0), (64, 0.3), (65, 0.7), (130, 0.95)))
+def test_msweep_over_missing_genotypes(tmp_path, markers, missing, mode):
+    case, data = synth.make_case("ped30_snp100", str(tmp_path), n_markers=markers, missing=missing)
+    o = Oracle(case)
+    starts = np.repeat(synth.true_graph(data, case)[None], 3, axis=0)
+    with native.Context(case, native.SL_FP64, msampler_mode=mode) as ctx:
+        ctx.mcmc_init(starts)
+        ctx.msweep(99, 0)
+        ctx.msweep(99, 1)
+        out = ctx.mcmc_graphs()
+        assert np.all(ctx.mcmc_status() == 0)
+        assert np.all(ctx.mcmc_near_edge() == 0)
+        lik = ctx.mcmc_likelihood()
+    for c in range(3):
+        g = o.msweep(starts[c], shuffled_order(o, 99, c, 0), 99, c, 0)
+        g = o.msweep(g, shuffled_order(o, 99, c, 1), 99, c, 1)
+        assert np.array_equal(out[c], g), c
+        ref = np.array([o.fag(g, l) for l in range(case.M)])
+        assert np.all(ref > 0) and np.all(np.abs(lik[c] / ref - 1.0) <= 1e-12)
+
+
+def test_classes_hold_for_every_flip(tmp_path):
+    """The rule itself, on the CPU side: with the family's possible phased
+    genotypes, a parent that cannot be heterozygous makes a flip change
+    nothing, and a parent of known phase with a known transmitted allele makes
+    it illegal."""
+    case, data = synth.make_case("ped30_snp100", str(tmp_path), n_markers=20, missing=0.2)
+    o = Oracle(case)
+    g = synth.true_graph(data, case)
+    het = 0b1100  # AU, UA
+    seen = [0, 0]
+    for l in range(case.M):
+        cur = o.fag(g, l)
+        for p in range(case.F, case.N):
+            for side in range(2):
+                q = int((case.father if side else case.mother)[p])
+                mq, mp = int(case.legal[q, l]), int(case.legal[p, l])
+                got = {(0, 1, 0, 1)[t] if side else (0, 1, 1, 0)[t] for t in range(4) if mp >> t & 1}
+                f = g.copy()
+                f[l, 2 * p + side] ^= 1
+                if not mq & het:
+                    seen[0] += 1
+                    assert abs(o.fag(f, l) / cur - 1.0) < 1e-12
+                elif mq in (0b0100, 0b1000) and len(got) == 1:
+                    seen[1] += 1
+                    assert o.fag(f, l) == 0.0
+    assert min(seen) > 20
