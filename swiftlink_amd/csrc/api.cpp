@@ -12,6 +12,7 @@
 
 #include "../../include/swiftlink_amd.h"
 #include "kernels.h"
+#include "lane64.h"
 #include "msampler_kernels.h"
 #include "peelseq.h"
 #include "philox.h"
@@ -33,6 +34,11 @@ constexpr int64_t kSpecWaves = 8192;
 constexpr int kMaxGridZ = 65535;
 // graphs from which the lane kernel scores a launch by default (half its lanes busy)
 constexpr int kLaneMinGraphs = 32;
+// evaluations (graphs x intervals x positions) from which FP64 scoring and the
+// adjoint run one evaluation per lane (lane64.hip)
+constexpr int64_t kL64MinEvals = 16384;
+constexpr int64_t kL64MinGradEvals = 6144;
+constexpr int kL64LeastWaves = 256;
 }
 
 struct sl_ctx;
@@ -69,6 +75,14 @@ struct sl_ctx {
     double* d_scalar = nullptr;
     sl::SeqOp* d_seq = nullptr;  // the program's sequential form (lane kernel)
     uint32_t* d_lstream = nullptr;  // and its descriptor stream
+    uint32_t* d_l64_hdr = nullptr;   // the FP64 lane program
+    uint32_t* d_l64_fwd = nullptr;
+    uint32_t* g_l64_hdr = nullptr;   // and the adjoint's
+    uint32_t* g_l64_fwd = nullptr;
+    uint32_t* g_l64_rev = nullptr;
+    double* d_l64 = nullptr;         // its wavefronts' table slots
+    size_t l64_cap = 0;
+    size_t l64_limit = SIZE_MAX;     // bytes past which an allocation has failed
     bool lod_global = false;     // the workgroup kernel's arena in global-memory slots (too large for LDS)
     void* d_lgt = nullptr;       // kLodGlobalSlots slots of arena_bytes
     size_t lgt_cap = 0;
@@ -322,6 +336,61 @@ int lod_chunks(const sl_ctx* c, int G) {
     return (G + per - 1) / per;
 }
 
+// FP64 scoring with one evaluation per lane: its terms are the workgroup
+// kernel's bit for bit, each graph a chunk of its own, so it serves launches
+// of one graph per chunk when nothing else was asked for.  Few evaluations
+// leave most of the device idle for the length of one wavefront's peel: the two
+// kernels cross near 16 k evaluations at 30 to 400 people (us, workgroup
+// against lanes: 118/121 at 15840 and 30 people, 413/276 at 19980 and 150,
+// 1057/526 at 39980 and 200).
+bool lane64_mode(const sl_ctx* c, int G) {
+    return c->precision == SL_FP64 && c->lod_kernel == SL_LOD_AUTO && c->gpw == 1 && c->prog.l64_ok &&
+           sl::lane64_lds_bytes(c->W) <= 64 * 1024 && (int64_t)G * (c->M - 1) * c->npos >= kL64MinEvals;
+}
+
+// A lane program's table slots for a launch of E evaluations: the wavefronts
+// that have one, or 0 when the device has no memory for even a quarter of the
+// device's SIMDs (the workgroup kernel then serves the call).  A size that was
+// refused is not asked for again.
+int ensure_lane64(sl_ctx* c, const PeelProgram& P, int64_t E) {
+    const size_t slot = sl::lane64_slot_bytes(P.l64_arena, P.l64_adj);
+    const size_t want = (size_t)sl::lane64_waves(E, slot);
+    const size_t least = std::min(want, (size_t)kL64LeastWaves);
+    for (;;) {
+        const size_t waves = std::min(want, c->l64_limit / slot);
+        if (waves < least) return 0;
+        if (waves * slot <= c->l64_cap * sizeof(double)) return (int)waves;
+        if (c->d_l64) (void)hipFree(c->d_l64);
+        c->d_l64 = nullptr;
+        c->l64_cap = 0;
+        if (hipMalloc((void**)&c->d_l64, waves * slot) == hipSuccess) {
+            c->l64_cap = waves * slot / sizeof(double);
+            return (int)waves;
+        }
+        (void)hipGetLastError();
+        c->d_l64 = nullptr;
+        c->l64_limit = waves * slot / 2;
+    }
+}
+
+sl::Lane64Args lane64_args(const sl_ctx* c, const PeelProgram& P) {
+    sl::Lane64Args A{};
+    A.n_ops = P.n_ops;
+    A.arena_cells = P.l64_arena;
+    A.adj_cells = P.l64_adj;
+    A.N = c->N;
+    A.F = c->F;
+    A.M = c->M;
+    A.W = c->W;
+    A.npos = c->npos;
+    A.trans = std::log(0.5) * (2.0 * (c->N - c->F));
+    A.partial_theta = c->d_ptheta;
+    A.log_theta = c->d_logt;
+    A.log_anti = c->d_loga;
+    A.scratch = c->d_l64;
+    return A;
+}
+
 hipError_t launch_scoring(sl_ctx* c, sl::LodArgs A, int nchunks) {
     if (lane_mode(c, A.G)) return sl::launch_lane_lod(A, c->precision, c->lane_lds, nchunks, c->stream);
     const int nl = c->M - 1;
@@ -407,7 +476,8 @@ int release_all(sl_ctx* c) {
                     c->g_ops, c->g_prevs, c->g_children, c->g_tasks, c->g_tinfo, c->g_idx, c->g_level_base,
                     c->g_sched_off, c->g_sched_ops, c->d_gdp, c->d_jac, c->d_gterms, c->d_gstate, c->d_sweep,
                     c->d_imp_graphs, c->d_imp_draw, c->d_imp_weight, c->d_imp_status, c->d_elod_pairs,
-                    c->d_gtables, c->d_lgt, c->d_lstream, c->d_trace};
+                    c->d_gtables, c->d_lgt, c->d_lstream, c->d_trace,
+                    c->d_l64_hdr, c->d_l64_fwd, c->g_l64_hdr, c->g_l64_fwd, c->g_l64_rev, c->d_l64};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& e : c->ev_pool) (void)hipEventDestroy(e);
@@ -700,6 +770,8 @@ int sl_create(const sl_pedigree_desc* ped, const sl_map_desc* map, const sl_peel
         (rc = upload(c, &c->d_sched_ops, c->prog.sched_ops.data(), c->prog.sched_ops.size())) ||
         (rc = upload(c, &c->d_seq, c->prog.seq.data(), c->prog.seq.size())) ||
         (rc = upload(c, &c->d_lstream, c->prog.lstream.data(), c->prog.lstream.size())) ||
+        (rc = upload(c, &c->d_l64_hdr, c->prog.l64_hdr.data(), c->prog.l64_hdr.size())) ||
+        (rc = upload(c, &c->d_l64_fwd, c->prog.l64_fwd.data(), c->prog.l64_fwd.size())) ||
         (rc = upload(c, &c->d_trait_d, ped->disease_prob, 4 * (size_t)c->N)) ||
         (rc = upload(c, &c->d_trait_f, tf.data(), tf.size())) ||
         (rc = upload(c, &c->d_ptheta, c->ptheta.data(), c->ptheta.size())) ||
@@ -850,6 +922,7 @@ static int lod_run(sl_ctx* c, const uint32_t* dev_graphs, int G, double* terms_d
     const size_t nacc = (size_t)(c->M - 1) * c->npos;
     int rc = ensure(c, &c->d_partial, &c->partial_cap, nacc * nchunks);
     if (rc) return rc;
+    const int waves = lane64_mode(c, G) ? ensure_lane64(c, c->prog, (int64_t)nacc * G) : 0;
     sl::LodArgs A = lod_args(c);
     A.graphs = dev_graphs;
     A.G = G;
@@ -864,7 +937,21 @@ static int lod_run(sl_ctx* c, const uint32_t* dev_graphs, int G, double* terms_d
         e1 = take_event(c);
         if (e0 && e1) SL_HIP(c, hipEventRecord(e0, c->stream));
     }
-    SL_HIP(c, launch_scoring(c, A, nchunks));
+    if (waves) {
+        sl::Lane64Args B = lane64_args(c, c->prog);
+        B.hdr = c->d_l64_hdr;
+        B.fwd = c->d_l64_fwd;
+        B.graphs = dev_graphs;
+        B.G = G;
+        B.partial = c->d_partial;
+        B.terms = terms_dev;
+        B.gate_sweep = gate;
+        B.gate_burnin = gate_burnin;
+        B.gate_period = gate_period;
+        SL_HIP(c, sl::launch_lane64(B, false, waves, sl::lane64_lds_bytes(c->W), c->stream));
+    } else {
+        SL_HIP(c, launch_scoring(c, A, nchunks));
+    }
     if (c->prof && e0 && e1) {
         SL_HIP(c, hipEventRecord(e1, c->stream));
         c->ev_used.push_back({SL_KERNEL_LOD, e0, e1, 1});
@@ -1852,6 +1939,7 @@ int sl_batch_run(sl_batch* b, const sl_schedule* sch, sl_mcmc_stats* stats) {
         }
         const int nchunks = lod_chunks(c, C);
         int rc = ensure(c, &c->d_partial, &c->partial_cap, (size_t)(c->M - 1) * c->npos * nchunks);
+        if (!rc && lane64_mode(c, C)) (void)ensure_lane64(c, c->prog, (int64_t)(c->M - 1) * c->npos * C);
         if (!rc && c->m_ready) rc = ensure(c, &c->d_order, &c->order_cap, c->meioses_h.size() * (size_t)C);
         if (!rc && c->samp_ready) rc = ensure_gtables(c);
         if (rc) return rc;
@@ -1976,7 +2064,7 @@ int install_lod_program(sl_ctx* c) {
     void** bufs[] = {(void**)&c->d_ops, (void**)&c->d_prevs, (void**)&c->d_children, (void**)&c->d_tasks,
                      (void**)&c->d_tinfo, (void**)&c->d_idx, (void**)&c->d_level_base, (void**)&c->d_sched_off,
                      (void**)&c->d_sched_ops, (void**)&c->d_trait_d, (void**)&c->d_trait_f, (void**)&c->d_seq,
-                     (void**)&c->d_lstream};
+                     (void**)&c->d_lstream, (void**)&c->d_l64_hdr, (void**)&c->d_l64_fwd};
     for (void** b : bufs) {
         if (*b) SL_HIP(c, hipFree(*b));
         *b = nullptr;
@@ -2005,9 +2093,26 @@ int install_lod_program(sl_ctx* c) {
         (rc = upload(c, &c->d_sched_ops, c->prog.sched_ops.data(), c->prog.sched_ops.size())) ||
         (rc = upload(c, &c->d_seq, c->prog.seq.data(), c->prog.seq.size())) ||
         (rc = upload(c, &c->d_lstream, c->prog.lstream.data(), c->prog.lstream.size())) ||
+        (rc = upload(c, &c->d_l64_hdr, c->prog.l64_hdr.data(), c->prog.l64_hdr.size())) ||
+        (rc = upload(c, &c->d_l64_fwd, c->prog.l64_fwd.data(), c->prog.l64_fwd.size())) ||
         (rc = upload(c, &c->d_trait_d, c->dp_h.data(), c->dp_h.size())) ||
         (rc = upload(c, &c->d_trait_f, tf.data(), tf.size())))
         return rc;
+    SL_HIP(c, hipStreamSynchronize(c->stream));
+    return SL_OK;
+}
+
+// The adjoint's lane program with the current model's disease probabilities in
+// its headers (the program itself does not depend on them).
+int upload_grad_lanes(sl_ctx* c) {
+    PeelProgram& P = c->gprog;
+    if (!P.l64_ok) return SL_OK;
+    for (int i = 0; i < P.n_ops; ++i) {
+        uint32_t* h = P.l64_hdr.data() + (size_t)i * sl::kL64Header;
+        memcpy(h + sl::kHTrait, c->dp_h.data() + 4 * (size_t)h[sl::kHPerson], 4 * sizeof(double));
+    }
+    SL_HIP(c, hipMemcpyAsync(c->g_l64_hdr, P.l64_hdr.data(), P.l64_hdr.size() * sizeof(uint32_t),
+                             hipMemcpyHostToDevice, c->stream));
     SL_HIP(c, hipStreamSynchronize(c->stream));
     return SL_OK;
 }
@@ -2036,7 +2141,10 @@ int ensure_grad_program(sl_ctx* c) {
         (rc = upload(c, &c->g_idx, P.idx.data(), P.idx.size())) ||
         (rc = upload(c, &c->g_level_base, P.level_base.data(), P.level_base.size())) ||
         (rc = upload(c, &c->g_sched_off, P.sched_off.data(), P.sched_off.size())) ||
-        (rc = upload(c, &c->g_sched_ops, P.sched_ops.data(), P.sched_ops.size())))
+        (rc = upload(c, &c->g_sched_ops, P.sched_ops.data(), P.sched_ops.size())) ||
+        (rc = upload<uint32_t>(c, &c->g_l64_hdr, nullptr, P.l64_hdr.size())) ||
+        (rc = upload(c, &c->g_l64_fwd, P.l64_fwd.data(), P.l64_fwd.size())) ||
+        (rc = upload(c, &c->g_l64_rev, P.l64_rev.data(), P.l64_rev.size())) || (rc = upload_grad_lanes(c)))
         return rc;
     SL_HIP(c, hipStreamSynchronize(c->stream));
     c->g_ready = true;
@@ -2069,6 +2177,31 @@ sl::LodArgs grad_args(sl_ctx* c) {
     return A;
 }
 
+// One launch of the adjoint over A.graphs (A.G of them) into out: one
+// evaluation per lane from kL64MinGradEvals evaluations, else one workgroup
+// each (a lane's reverse pass takes milliseconds, however few there are: at 30,
+// 77 and 150 people the two cross at 6 to 7 k evaluations).
+int launch_adjoint(sl_ctx* c, const sl::LodArgs& A, double* out) {
+    const int64_t E = (int64_t)A.G * (c->M - 1) * c->npos;
+    const bool lanes = c->gprog.l64_ok && E >= kL64MinGradEvals && sl::lane64_lds_bytes(c->W) <= 64 * 1024;
+    const int waves = lanes ? ensure_lane64(c, c->gprog, E) : 0;
+    if (!waves) {
+        sl::GradArgs Gd{c->d_jac, out, c->npos};
+        SL_HIP(c, sl::launch_grad(A, Gd, 0, c->g_lds, c->stream));
+        return SL_OK;
+    }
+    sl::Lane64Args B = lane64_args(c, c->gprog);
+    B.hdr = c->g_l64_hdr;
+    B.fwd = c->g_l64_fwd;
+    B.rev = c->g_l64_rev;
+    B.graphs = A.graphs;
+    B.G = A.G;
+    B.jac = c->d_jac;
+    B.out = out;
+    SL_HIP(c, sl::launch_lane64(B, true, waves, sl::lane64_lds_bytes(c->W), c->stream));
+    return SL_OK;
+}
+
 }  // namespace
 
 int sl_trait_model_tables(const sl_trait_model* model, int32_t N, int32_t F, double* dp, double* jac) {
@@ -2094,6 +2227,7 @@ int sl_set_trait_model(sl_ctx* c, const sl_trait_model* model) {
     SL_HIP(c, hipStreamSynchronize(c->stream));
     c->has_model = true;
     c->trait_prob_valid = false;
+    if (c->g_ready) return upload_grad_lanes(c);
     return SL_OK;
 }
 
@@ -2111,8 +2245,7 @@ int sl_trait_grad(sl_ctx* c, const int32_t* graphs, int32_t G, double* out) {
     for (int g0 = 0; g0 < G; g0 += kMaxGridZ) {  // the grid's z extent is the graph
         A.graphs = c->d_packed + (size_t)g0 * c->M * c->W;
         A.G = std::min(kMaxGridZ, G - g0);
-        sl::GradArgs Gd{c->d_jac, c->d_gterms + (size_t)g0 * per_graph, c->npos};
-        SL_HIP(c, sl::launch_grad(A, Gd, 0, c->g_lds, c->stream));
+        if ((rc = launch_adjoint(c, A, c->d_gterms + (size_t)g0 * per_graph))) return rc;
     }
     SL_HIP(c, hipMemcpyAsync(out, c->d_gterms, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     SL_HIP(c, hipStreamSynchronize(c->stream));
@@ -2156,8 +2289,7 @@ int sl_lod_grad(sl_ctx* c, const uint32_t* dev_graphs, int32_t G, double* lod, d
         const int gc = std::min(chunk, G - g0);
         A.graphs = dev_graphs + (size_t)g0 * c->M * c->W;
         A.G = gc;
-        sl::GradArgs Gd{c->d_jac, c->d_gterms, c->npos};
-        SL_HIP(c, sl::launch_grad(A, Gd, 0, c->g_lds, c->stream));
+        if ((rc = launch_adjoint(c, A, c->d_gterms))) return rc;
         SL_HIP(c, sl::launch_grad_fold(c->d_gstate, c->d_gterms, gc, n, c->stream));
     }
     // P(T) and its derivatives after the state
