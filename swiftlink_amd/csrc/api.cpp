@@ -39,6 +39,8 @@ constexpr int kLaneMinGraphs = 32;
 constexpr int64_t kL64MinEvals = 16384;
 constexpr int64_t kL64MinGradEvals = 6144;
 constexpr int kL64LeastWaves = 256;
+// records of the flat L-sampler (32 bytes per cell and trait value) a context may hold
+constexpr size_t kFlatMaxBytes = (size_t)4 << 30;
 }
 
 struct sl_ctx;
@@ -162,6 +164,13 @@ struct sl_ctx {
     int32_t* d_status = nullptr;    // [chains]
     int n_chains = 0;
     bool samp_ready = false;
+    // the flat L-sampler's per-locus records (unset when the tables are outside what it takes)
+    bool flat_ok = false;
+    size_t flat_lds = 0;
+    uint32_t* d_task = nullptr;
+    uint32_t* d_task_base = nullptr;
+    uint32_t* d_level_task = nullptr;
+    uint32_t* d_rrec = nullptr;
     std::string samp_why;           // why the sampler program was rejected, if it was
     std::vector<int32_t> mother_h, father_h;
     // M-sampler
@@ -477,7 +486,7 @@ int release_all(sl_ctx* c) {
                     c->g_sched_off, c->g_sched_ops, c->d_gdp, c->d_jac, c->d_gterms, c->d_gstate, c->d_sweep,
                     c->d_imp_graphs, c->d_imp_draw, c->d_imp_weight, c->d_imp_status, c->d_elod_pairs,
                     c->d_gtables, c->d_lgt, c->d_lstream, c->d_trace,
-                    c->d_l64_hdr, c->d_l64_fwd, c->g_l64_hdr, c->g_l64_fwd, c->g_l64_rev, c->d_l64};
+                    c->d_task, c->d_task_base, c->d_level_task, c->d_rrec, c->d_l64_hdr, c->d_l64_fwd, c->g_l64_hdr, c->g_l64_fwd, c->g_l64_rev, c->d_l64};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& e : c->ev_pool) (void)hipEventDestroy(e);
@@ -653,6 +662,8 @@ int timed_span(sl_ctx* c, int kind, int launches, Fn body) {
 }
 
 }  // namespace
+
+static int setup_flat(sl_ctx* c);
 
 extern "C" {
 
@@ -865,6 +876,12 @@ int sl_create(const sl_pedigree_desc* ped, const sl_map_desc* map, const sl_peel
                 return fail(nullptr, SL_E_DEVICE, m);
             }
             c->samp_ready = true;
+            if ((rc = setup_flat(c))) {
+                std::string m = c->err;
+                release_all(c);
+                delete c;
+                return fail(nullptr, rc, m);
+            }
         }
     }
     e = sl::launch_fill(c->d_acc, -INFINITY, nacc, c->stream);
@@ -1102,6 +1119,45 @@ int sl_lod_kernel_for(sl_ctx* c, int32_t n_graphs, int32_t* kernel) {
     return SL_OK;
 }
 
+static sl::SampArgs samp_args(sl_ctx* c);
+
+// The flat L-sampler's records (lsampler.hip).  Leaves flat_ok false where it
+// does not apply: an op consumes more than three tables or has more than three
+// children, an index passes 16 bits, the workgroup does not fit LDS, or the
+// records pass kFlatMaxBytes or the memory there is (the loci's steps are then
+// decoded in the kernel).
+static int setup_flat(sl_ctx* c) {
+    const sl::SampProgram& P = c->sprog;
+    c->flat_lds = sl::lsampler_flat_lds_bytes(c->precision, c->cells_cap, P.n_ops, P.n_levels, c->N, c->F);
+    if (P.max_prev > sl::kFlatMaxPrev || P.max_child > sl::kFlatMaxKids || P.cell_base.empty() || c->N >= 8000 ||
+        c->flat_lds > 160 * 1024 || sl::lsampler_build_lds_bytes(P.n_ops, c->N) > 64 * 1024)
+        return SL_OK;
+    const size_t words = 4 * (size_t)P.cell_base[c->M] * sl::kTaskWords;
+    if (words * sizeof(uint32_t) > kFlatMaxBytes) return SL_OK;
+    uint32_t** bufs[] = {&c->d_task, &c->d_level_task, &c->d_rrec, &c->d_task_base};
+    const size_t sizes[] = {words, (size_t)c->M * (P.n_levels + 1), (size_t)c->M * P.n_ops * sl::kRevWords,
+                            (size_t)c->M + 1};
+    for (int i = 0; i < 4; ++i)
+        if (hipMalloc((void**)bufs[i], sizes[i] * sizeof(uint32_t)) != hipSuccess) {
+            (void)hipGetLastError();
+            *bufs[i] = nullptr;
+            for (int j = 0; j < i; ++j) {
+                (void)hipFree(*bufs[j]);
+                *bufs[j] = nullptr;
+            }
+            return SL_OK;
+        }
+    SL_HIP(c, hipMemcpyAsync(c->d_task_base, P.cell_base.data(), sizes[3] * sizeof(uint32_t), hipMemcpyHostToDevice,
+                             c->stream));
+    sl::SampArgs A = samp_args(c);
+    SL_HIP(c, sl::launch_lsampler_build(A, c->precision, c->d_task, c->d_level_task, c->d_rrec,
+                                        sl::lsampler_build_lds_bytes(P.n_ops, c->N), c->stream));
+    SL_HIP(c, sl::configure_lsampler_flat_lds(c->precision, c->flat_lds));
+    SL_HIP(c, hipStreamSynchronize(c->stream));
+    c->flat_ok = true;
+    return SL_OK;
+}
+
 static int need_sampler(sl_ctx* c) {
     if (!c->samp_ready) return fail(c, SL_E_UNSUPPORTED, "sampler unavailable: " + c->samp_why);
     return SL_OK;
@@ -1226,6 +1282,11 @@ static sl::SampArgs samp_args(sl_ctx* c) {
     A.near_edge = c->d_near;
     A.near_loci = c->d_near_loci;
     A.near_words = near_words(c);
+    A.task = c->d_task;
+    A.task_base = c->d_task_base;
+    A.level_task = c->d_level_task;
+    A.rrec = c->d_rrec;
+    A.max_rlevel_ops = c->sprog.max_ops_per_rlevel;
     return A;
 }
 
@@ -1265,6 +1326,10 @@ static int ensure_gtables(sl_ctx* c) {
 static int launch_samp(sl_ctx* c, sl::SampArgs A, int block, int gx, int gy) {
     A.block0 = A.chain0 = 0;
     A.gtables = nullptr;
+    if (c->flat_ok) {
+        SL_HIP(c, sl::launch_lsampler_flat(A, c->precision, c->flat_lds, gx, gy, c->stream));
+        return SL_OK;
+    }
     if (!c->samp_global) {
         SL_HIP(c, sl::launch_lsampler(A, c->precision, block, c->samp_lds, gx, gy, c->stream));
         return SL_OK;

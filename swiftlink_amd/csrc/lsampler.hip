@@ -23,7 +23,10 @@
 //     heterozygous parents fix the bit, homozygous parents draw in person
 //     order after the op draws; the whole column l is rewritten.
 //
-// The same kernel runs sequential imputation (SequentialImputation,
+// A locus step runs from per-locus task records where they apply (the flat form
+// below); the decoding kernel serves the rest.
+//
+// Both run sequential imputation (SequentialImputation,
 // sequential_imputation.cc:47-114): one workgroup per replicate, one launch
 // per step of the replicates' locus walks, the walked-from neighbour as the
 // only conditioning column, each replicate's uniforms taken in sequence from
@@ -714,6 +717,496 @@ __global__ void __launch_bounds__(kLsamplerBlockWide) lsampler_kernel(SampArgs A
     }
 }
 
+// ---- The flat form: per-locus task records ----
+//
+// Which products a locus's peel forms depends on its legal masks only, not on
+// the chain: the builder writes them down once per context, one record per
+// (cell, value of the peel node), and a locus step reads each level's records
+// with one coalesced load per lane, issued a level ahead.  A level is then one
+// pass over its records by the whole workgroup, whatever ops they belong to, a
+// product of a handful of LDS entries per lane.  The kernel above decodes every
+// cell of every op again for each chain, op after op within a wavefront: one
+// chain's parity launch at ped150 took 105 us of dependent instructions, now 36;
+// 64 chains' (half of them) 1907 us, now 345; 1000 imputation replicates 164 us a
+// step, now 41; 65535 ELOD replicates in FP64 16.4 ms a step, now 7.4 (its 2550
+// cells per locus leave one workgroup per CU).
+// Products, sums and scales are those of sampler_op, in its order, so tables,
+// draws and graphs are the same bit for bit.
+
+__device__ __forceinline__ uint32_t half_index(uint32_t bit, uint32_t t, uint32_t a, uint32_t one) {
+    // parent_factor as an index: constants for homozygous parents
+    if (t == PT_UU) return a ? one + 1u : one;
+    if (t == PT_AA) return a ? one : one + 1u;
+    return 4u * bit + (t == PT_AU ? 0u : 2u) + a;
+}
+
+// One workgroup per locus.
+__global__ void __launch_bounds__(kFlatBlock) lsampler_build_kernel(SampArgs A, int fp64, uint32_t* task,
+                                                                    uint32_t* level_task, uint32_t* rrec) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int N = A.N, F = A.F, n = A.n_ops, W = A.waves, locus = blockIdx.x, tid = threadIdx.x;
+    int* off = reinterpret_cast<int*>(smem);  // [n+1] first cell of the op at each position of the level order
+    int* pos = off + n + 1;                   // [n] position of each op
+    int* tmp = pos + n;                       // [1]
+    uint8_t* mask = reinterpret_cast<uint8_t*>(tmp + 1);  // [N]
+    for (int p = tid; p < N; p += blockDim.x) mask[p] = A.legal_t[(size_t)locus * N + p] & 15u;
+    __syncthreads();
+    for (int i = tid; i < n; i += blockDim.x) {
+        const SampOp* d = A.ops + A.sched_ops[i];
+        int s = 1;
+        for (int q = 0; q < d->k; ++q) s *= __popc(mask[d->cut[q]]);
+        off[i] = s;
+        pos[A.sched_ops[i]] = i;
+    }
+    __syncthreads();
+    const int cells = block_exclusive_scan(off, n, tmp);
+    if (tid == 0) off[n] = cells;
+    __syncthreads();
+    const uint32_t base = A.task_base[locus];
+    if ((uint32_t)cells != A.task_base[locus + 1] - base) return;  // cannot happen: the host counted the same masks
+    for (int L = tid; L <= A.n_levels; L += blockDim.x)
+        level_task[(size_t)locus * (A.n_levels + 1) + L] = 4u * (uint32_t)off[A.sched_off[L * W]];
+    for (int i = tid; i < n; i += blockDim.x) {
+        const int op = A.rlevel_ops[i];
+        const SampOp* d = A.ops + op;
+        uint32_t* r = rrec + ((size_t)locus * n + i) * kRevWords;
+        uint32_t m = 0, who[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        for (int q = 0; q < d->k; ++q) {
+            m |= (uint32_t)mask[d->cut[q]] << (4 * q);
+            who[q] = (uint32_t)d->cut[q];
+        }
+        who[7] = (uint32_t)d->peel;
+        r[0] = m;
+        r[1] = (uint32_t)off[pos[op]];
+        for (int w = 0; w < 4; ++w) r[2 + w] = who[2 * w] | (who[2 * w + 1] << 16);
+        r[6] = (uint32_t)d->k | ((uint32_t)op << 8);
+        r[7] = 0u;
+    }
+    const uint32_t one = 8u * (uint32_t)(N - F);
+    for (int t = tid; t < 4 * cells; t += blockDim.x) {
+        const int cell = t >> 2;
+        const uint32_t v = (uint32_t)t & 3u;
+        int lo = 0, hi = n;  // the op whose cells hold this one
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (off[mid] <= cell) lo = mid;
+            else hi = mid;
+        }
+        const int op = A.sched_ops[lo];
+        const SampOp* d = A.ops + op;
+        const int k = d->k, peel = d->peel;
+        uint32_t cmw = 0, val[kMaxCut + 1], rank[kMaxCut + 1];
+        int rem = cell - off[lo];
+        for (int q = 0; q < k; ++q) {
+            const uint32_t m = mask[d->cut[q]];
+            const int c = __popc(m);
+            cmw |= m << (4 * q);
+            rank[q] = (uint32_t)(rem % c);
+            val[q] = select_bit(m, rank[q]);
+            rem /= c;
+        }
+        const uint32_t pm = mask[peel];
+        cmw |= pm << (4 * k);
+        val[k] = v;
+        rank[k] = rank_in(pm, v);
+        uint32_t w[kTaskWords] = {0, 0, 0, 0, 0, 0, 0, 0};
+        const bool first = t == 4 * off[lo];
+        w[1] = ((uint32_t)op << 16) | (first ? 512u : 0u);
+        const size_t gi = ((size_t)locus * N + peel) * 4 + v;
+        const double tr = fp64 ? A.geno_prob_d[gi] : (double)A.geno_prob_f[gi];
+        if (((pm >> v) & 1u) != 0u && tr != 0.0) {
+            uint32_t fac[2 * kFlatMaxKids] = {0, 0, 0, 0, 0, 0}, nf = 0;
+            if (d->type == kChild) {
+                const uint32_t am = v == PT_AA || v == PT_AU ? 1u : 0u, ap = v == PT_AA || v == PT_UA ? 1u : 0u;
+                const uint32_t b = 2u * (uint32_t)(peel - F);
+                fac[0] = half_index(b, val[d->mat_digit], am, one);
+                fac[1] = half_index(b + 1u, val[d->pat_digit], ap, one);
+                nf = 2;
+            } else if (d->type == kParent) {
+                for (int ch = 0; ch < d->n_child; ++ch) {
+                    const uint32_t c = d->child[ch];
+                    const uint32_t b = (c & 0xFFFFu) >> 2, info = c >> 16;  // 8 (person - F) -> 2 (person - F)
+                    const uint32_t kid = val[info & 15u], other = val[(info >> 4) & 15u];
+                    const uint32_t am = kid == PT_AA || kid == PT_AU ? 1u : 0u, ap = kid == PT_AA || kid == PT_UA ? 1u : 0u;
+                    const bool pim = (info >> 8) != 0u;
+                    fac[2 * ch] = half_index(b, pim ? v : other, am, one);
+                    fac[2 * ch + 1] = half_index(b + 1u, pim ? other : v, ap, one);
+                }
+                nf = 2u * (uint32_t)d->n_child;
+                w[1] |= 256u;
+            }
+            uint32_t prev[kFlatMaxPrev] = {0, 0, 0}, pop[kFlatMaxPrev] = {0, 0, 0};
+            for (int q = 0; q < d->n_prev; ++q) {
+                const SampPrev* pd = A.prevs + d->prev_off + q;
+                uint32_t ix = 0, st = 1;
+                for (int j = 0; j < pd->nd; ++j) {
+                    const int src = pd->src[j];
+                    ix += rank[src] * st;
+                    st *= (uint32_t)__popc((cmw >> (4 * src)) & 15u);
+                }
+                pop[q] = (uint32_t)pd->op;
+                prev[q] = (uint32_t)off[pos[pd->op]] + ix;
+            }
+            if (fp64) {
+                const unsigned long long bits = (unsigned long long)__double_as_longlong(tr);
+                w[0] = (uint32_t)bits;
+                w[7] = (uint32_t)(bits >> 32);
+            } else {
+                w[0] = __float_as_uint((float)tr);
+                w[7] = pop[0] | (pop[1] << 16);
+            }
+            w[1] |= (uint32_t)d->n_prev | (nf << 4);
+            for (int j = 0; j < 3; ++j) w[2 + j] = fac[2 * j] | (fac[2 * j + 1] << 16);
+            w[5] = prev[0] | (prev[1] << 16);
+            w[6] = prev[2] | (pop[2] << 16);
+        } else if (first) {
+            // the op's consumed scales are counted at its first task, legal or not
+            w[1] |= (uint32_t)d->n_prev;
+            uint32_t pop[kFlatMaxPrev] = {0, 0, 0};
+            for (int q = 0; q < d->n_prev; ++q) pop[q] = (uint32_t)A.prevs[d->prev_off + q].op;
+            w[6] = pop[2] << 16;
+            w[7] = fp64 ? 0u : pop[0] | (pop[1] << 16);
+        }
+        uint4* out = reinterpret_cast<uint4*>(task + ((size_t)4 * base + t) * kTaskWords);
+        out[0] = make_uint4(w[0], w[1], w[2], w[3]);
+        out[1] = make_uint4(w[4], w[5], w[6], w[7]);
+    }
+}
+
+// LDS of a flat workgroup
+template <typename T>
+struct FlatArea {
+    double* uop;        // [n_ops] op draws
+    double* um;         // [2NF] meiosis draws by index
+    double* thr;        // [4] draw threshold of a homozygous parent's meiosis by neighbour bits
+    T* tab;             // [cells_cap]
+    T* pre;             // [4 cells_cap]
+    T* dist;            // [8NF+2] transmission entries, then 1 and 0
+    T* f4;              // [16] the entries by neighbour bits
+    uint32_t* maxbits;  // [n_ops]
+    uint32_t* lvl;      // [n_levels+1]
+    uint32_t* cnt;      // [kFlatBlock/64]
+    uint8_t* pmk;       // [N]
+    uint8_t* cmb;       // [2NF] neighbour bits: left | right << 1
+    __device__ FlatArea(unsigned char* p, const SampArgs& A) {
+        const int NF = A.N - A.F;
+        uop = reinterpret_cast<double*>(p);
+        um = uop + A.n_ops;
+        thr = um + 2 * NF;
+        tab = reinterpret_cast<T*>(thr + 4);
+        pre = tab + A.cells_cap;
+        dist = pre + 4 * (size_t)A.cells_cap;
+        f4 = dist + 8 * NF + 4;
+        maxbits = reinterpret_cast<uint32_t*>(f4 + 16);
+        lvl = maxbits + A.n_ops;
+        cnt = lvl + A.n_levels + 1;
+        pmk = reinterpret_cast<uint8_t*>(cnt + kFlatBlock / 64);
+        cmb = pmk + A.N;
+    }
+};
+
+// One record's product, the sum over its cell's quad, and their stores.
+template <typename T, bool RESCALE>
+__device__ __forceinline__ void flat_task(const SampArgs& A, const FlatArea<T>& S, int t, const uint4& lo,
+                                          const uint4& hi, int* scale_exp) {
+    const uint32_t np = lo.y & 15u, nf = (lo.y >> 4) & 15u;
+    T x;
+    if constexpr (sizeof(T) == 4) x = __uint_as_float(lo.x);
+    else x = __longlong_as_double((long long)(((unsigned long long)hi.w << 32) | lo.x));
+    // consumed cells and their scales, all read before the products
+    T pv[kFlatMaxPrev];
+    const uint32_t cell[3] = {hi.y & 0xFFFFu, hi.y >> 16, hi.z & 0xFFFFu};
+    const uint32_t pop[3] = {hi.w & 0xFFFFu, hi.w >> 16, hi.z >> 16};
+    int se = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < 3; ++q) {
+        pv[q] = (T)1;
+        if (q < np) {
+            pv[q] = S.tab[cell[q]];
+            if (RESCALE) {
+                const uint32_t mb = S.maxbits[pop[q]];
+                pv[q] *= (T)scale_from_bits(mb);
+                const int ef = (int)((mb >> 23) & 0xFFu);
+                se += ef ? 126 - ef : 0;
+            }
+        }
+    }
+    T fa[3];
+    const uint32_t fw[3] = {lo.z, lo.w, hi.x};
+#pragma unroll
+    for (uint32_t j = 0; j < 3; ++j) {
+        fa[j] = (T)1;
+        if (2 * j < nf) fa[j] = S.dist[fw[j] & 0xFFFFu] * S.dist[fw[j] >> 16];
+    }
+    if (RESCALE && A.impute && (lo.y & 512u) && se != 0) atomicAdd(scale_exp, se);
+    if (x != (T)0) {
+        const bool parent = (lo.y & 256u) != 0u;
+        if (!parent && nf) x *= fa[0];
+#pragma unroll
+        for (uint32_t q = 0; q < 3; ++q)
+            if (q < np) x *= pv[q];
+        if (parent) x *= (fa[0] * fa[1]) * fa[2];
+    }
+    S.pre[t] = x;
+    const T s0 = quad_lane<T, 0x00>(x), s1 = quad_lane<T, 0x55>(x), s2 = quad_lane<T, 0xAA>(x), s3 = quad_lane<T, 0xFF>(x);
+    const T total = ((s0 + s1) + s2) + s3;
+    if ((t & 3) == 0) {
+        S.tab[t >> 2] = total;
+        if (RESCALE) atomicMax(&S.maxbits[lo.y >> 16], __float_as_uint((float)total));
+    }
+}
+
+__device__ __forceinline__ void lds_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Reverse step of one op (SamplerRfunction::sample, sampler_rfunction.cc:159-188)
+template <typename T>
+__device__ __forceinline__ void flat_sample(const SampArgs& A, const FlatArea<T>& S, int chain, int locus, const uint4& lo,
+                                            const uint4& hi) {
+    const uint32_t k = hi.z & 255u, op = hi.z >> 8, m = lo.x;
+    const uint32_t who[7] = {lo.z & 0xFFFFu, lo.z >> 16, lo.w & 0xFFFFu, lo.w >> 16,
+                             hi.x & 0xFFFFu, hi.x >> 16, hi.y & 0xFFFFu};
+    uint32_t base = lo.y, st = 1;
+#pragma unroll
+    for (uint32_t q = 0; q < 7; ++q) {
+        if (q < k) {
+            const uint32_t mq = (m >> (4 * q)) & 15u;
+            base += rank_in(mq, S.pmk[who[q]]) * st;
+            st *= (uint32_t)__popc(mq);
+        }
+    }
+    const T* pc = S.pre + 4 * (size_t)base;
+    T pdv[4] = {pc[0], pc[1], pc[2], pc[3]};
+    const T tot = pdv[0] + pdv[1] + pdv[2] + pdv[3];
+    if (tot != (T)0)
+        for (int v = 0; v < 4; ++v) pdv[v] /= tot;
+    const double u = S.uop[op];
+    T run = (T)0;
+    int last = 0, chosen = -1;
+    bool edge = false;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        run += pdv[v];
+        if (chosen < 0 && u < (double)run) chosen = v;
+        if (pdv[v] != (T)0) last = v;
+        if (v < 3 && pdv[v] != (T)0 && fabs(u - (double)run) < kEdgeTol<T>) edge = true;
+    }
+    S.pmk[hi.y >> 16] = (uint8_t)(chosen >= 0 ? chosen : last);
+    if (A.near_edge && edge) {
+        atomicAdd(&A.near_edge[chain], 1u);
+        atomicOr(&A.near_loci[(size_t)chain * A.near_words + (locus >> 5)], 1u << (locus & 31));
+    }
+}
+
+template <typename T, bool RESCALE>
+__global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ int s_scale_exp;
+    const int N = A.N, F = A.F, M = A.M, n_ops = A.n_ops, NF = N - F, tid = threadIdx.x;
+    const FlatArea<T> S(smem, A);
+    const int chain = (int)blockIdx.y;
+    const uint32_t sweep = A.impute ? A.sweep : sweep_of(A);
+    int locus;
+    bool use_left = true, use_right = true;
+    uint32_t step_id, draw0 = 0;
+    const uint32_t rng_chain = (uint32_t)chain + (A.impute ? A.chain_base : 0u);
+    if (A.impute) {
+        if (A.status[chain] != 0) return;
+        locus = impute_locus(A.impute, A.impute_t, M, A.impute_start, A.seed, rng_chain, A.sweep, &use_left,
+                             &use_right);
+        step_id = kStepImpute;
+        draw0 = A.imp_draw[chain];
+    } else {
+        int parity = A.parity;
+        if (A.check_kind) {
+            if (!(philox_uniform(A.seed, (uint32_t)chain, sweep, kStepSched, 0) < A.lprob)) return;
+            const int p0 = philox_uniform(A.seed, (uint32_t)chain, sweep, kStepSched, 1) < 0.5 ? 0 : 1;
+            parity = A.pass == 0 ? p0 : 1 - p0;
+        }
+        locus = parity + 2 * (int)blockIdx.x;
+        if (locus >= M || A.status[chain] != 0) return;  // uniform over the workgroup
+        step_id = (uint32_t)locus;
+    }
+    const uint32_t base = A.task_base[locus];
+    const uint4* task = reinterpret_cast<const uint4*>(A.task + (size_t)4 * base * kTaskWords);
+    const uint32_t* lt = A.level_task + (size_t)locus * (A.n_levels + 1);
+    // the first level's records, in flight during the set-up
+    uint4 lo = make_uint4(0, 0, 0, 0), hi = lo;
+    if ((uint32_t)tid < lt[1]) {
+        lo = task[2 * tid];
+        hi = task[2 * tid + 1];
+    }
+    uint32_t* g = A.graphs + (size_t)chain * M * A.W;
+    const uint32_t* colL = locus > 0 && use_left ? g + (size_t)(locus - 1) * A.W : nullptr;
+    const uint32_t* colR = locus < M - 1 && use_right ? g + (size_t)(locus + 1) * A.W : nullptr;
+    // 1. what depends on the neighbours' bits of one meiosis: four cases
+    if (tid < 4) {
+        const double thL = locus > 0 ? A.theta[locus - 1] : 1.0, thR = locus < M - 1 ? A.theta[locus] : 1.0;
+        const bool bl = (tid & 1) != 0, br = (tid & 2) != 0;
+        double tmp0 = 0.5, tmp1 = 0.5, p0 = 1.0, p1 = 1.0;
+        if (colL) {
+            tmp0 *= bl ? thL : 1.0 - thL;
+            tmp1 *= bl ? 1.0 - thL : thL;
+            p0 *= bl ? thL : 1.0 - thL;
+            p1 *= bl ? 1.0 - thL : thL;
+        }
+        if (colR) {
+            tmp0 *= br ? thR : 1.0 - thR;
+            tmp1 *= br ? 1.0 - thR : thR;
+            p0 *= br ? thR : 1.0 - thR;
+            p1 *= br ? 1.0 - thR : thR;
+        }
+        const double total = tmp0 + tmp1;
+        const double uAU = tmp1 / total, uUA = tmp0 / total;
+        S.f4[4 * tid] = (T)uAU;
+        S.f4[4 * tid + 1] = (T)(1.0 - uAU);
+        S.f4[4 * tid + 2] = (T)uUA;
+        S.f4[4 * tid + 3] = (T)(1.0 - uUA);
+        S.thr[tid] = p0 / (p0 + p1);
+    }
+    if (tid == 4) {
+        s_scale_exp = 0;
+        S.dist[8 * NF] = (T)1;
+        S.dist[8 * NF + 1] = (T)0;
+    }
+    for (int L = tid; L <= A.n_levels; L += kFlatBlock) S.lvl[L] = lt[L];
+    for (int o = tid; o < n_ops; o += kFlatBlock) {
+        S.uop[o] = philox_uniform(A.seed, rng_chain, sweep, step_id, draw0 + (uint32_t)(n_ops - 1 - o));
+        S.maxbits[o] = 0u;
+    }
+    __syncthreads();
+    for (int b = tid; b < 2 * NF; b += kFlatBlock) {
+        uint32_t c = 0;
+        if (colL) c |= (colL[b >> 5] >> (b & 31)) & 1u;
+        if (colR) c |= ((colR[b >> 5] >> (b & 31)) & 1u) << 1;
+        S.cmb[b] = (uint8_t)c;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S.dist[4 * b + e] = S.f4[4 * c + e];
+    }
+    __syncthreads();
+    // 2. forward peel, a level per pass
+    for (int L = 0; L < A.n_levels; ++L) {
+        const int t0 = uni((int)S.lvl[L]), t1 = uni((int)S.lvl[L + 1]);
+        uint4 nlo = make_uint4(0, 0, 0, 0), nhi = nlo;
+        if (L + 1 < A.n_levels) {
+            const int tn = t1 + tid;
+            if (tn < uni((int)S.lvl[L + 2])) {
+                nlo = task[2 * tn];
+                nhi = task[2 * tn + 1];
+            }
+        }
+        for (int t = t0 + tid; t < t1; t += kFlatBlock) {
+            if (t != t0 + tid) {
+                lo = task[2 * t];
+                hi = task[2 * t + 1];
+            }
+            flat_task<T, RESCALE>(A, S, t, lo, hi, &s_scale_exp);
+        }
+        lo = nlo;
+        hi = nhi;
+        __syncthreads();
+    }
+    // likelihood of the locus (locus_sampler2.cc:137-142): the last cell
+    const T like = S.tab[S.lvl[A.n_levels] / 4 - 1];
+    if (!(like > (T)0)) {
+        if (tid == 0) A.status[chain] = -4;
+        return;
+    }
+    if (A.impute && tid == 0) {
+        // ln of the locus likelihood (locus_sampler2.cc:221, 228, 235): the
+        // rescaled last table divided by the scale factors it absorbed
+        double w = log((double)like);
+        if (RESCALE) w -= (double)s_scale_exp * 0.69314718055994530942;
+        A.imp_weight[chain] += w;
+    }
+    // 3. reverse sampling by reverse levels: the first wavefront while the
+    // others draw the meioses' uniforms (by draw index; not all are used), or
+    // the whole workgroup where levels are wide
+    const uint4* rrec = reinterpret_cast<const uint4*>(A.rrec + (size_t)locus * n_ops * kRevWords);
+    const bool narrow = A.max_rlevel_ops <= 64;
+    if (narrow && tid >= 64) {
+        for (int i = tid - 64; i < 2 * NF; i += kFlatBlock - 64)
+            S.um[i] = philox_uniform(A.seed, rng_chain, sweep, step_id, draw0 + (uint32_t)(n_ops + i));
+    } else {
+        if (!narrow)
+            for (int i = tid; i < 2 * NF; i += kFlatBlock)
+                S.um[i] = philox_uniform(A.seed, rng_chain, sweep, step_id, draw0 + (uint32_t)(n_ops + i));
+        const int stride = narrow ? 64 : kFlatBlock;
+        int r1 = ((cint_p)A.rlevel_off)[1];
+        uint4 rl = make_uint4(0, 0, 0, 0), rh = rl;
+        if (tid < r1) {
+            rl = rrec[2 * tid];
+            rh = rrec[2 * tid + 1];
+        }
+        int r0 = 0;
+        for (int R = 0; R < A.n_rlevels; ++R) {
+            const int r2 = R + 1 < A.n_rlevels ? ((cint_p)A.rlevel_off)[R + 2] : r1;
+            uint4 nl = make_uint4(0, 0, 0, 0), nh = nl;
+            if (r1 + tid < r2) {
+                nl = rrec[2 * (r1 + tid)];
+                nh = rrec[2 * (r1 + tid) + 1];
+            }
+            for (int i = r0 + tid; i < r1; i += stride) {
+                if (i != r0 + tid) {
+                    rl = rrec[2 * i];
+                    rh = rrec[2 * i + 1];
+                }
+                flat_sample<T>(A, S, chain, locus, rl, rh);
+            }
+            rl = nl;
+            rh = nh;
+            r0 = r1;
+            r1 = r2;
+            if (narrow) lds_wave_sync();
+            else __syncthreads();
+        }
+    }
+    __syncthreads();
+    // 4. meiosis indicators: a homozygous parent's draw index counts those before it
+    uint32_t* col = g + (size_t)locus * A.W;
+    const int lane = tid & 63, wave = tid >> 6;
+    uint32_t drawn = 0;
+    for (int b0 = 0; b0 < 2 * NF; b0 += kFlatBlock) {
+        const int b = b0 + tid;
+        const bool in = b < 2 * NF;
+        uint32_t pt = PT_AU, t = 0;
+        const int side = b & 1;
+        if (in) {
+            const int person = F + (b >> 1);
+            pt = S.pmk[side ? A.father[person] : A.mother[person]];
+            t = S.pmk[person];
+        }
+        const bool homo = in && (pt == PT_UU || pt == PT_AA);
+        const uint64_t hm = __ballot(homo);
+        if (lane == 0) S.cnt[wave] = (uint32_t)__popcll(hm);
+        __syncthreads();
+        uint32_t before = drawn + (uint32_t)__popcll(hm & ((1ull << lane) - 1ull));
+#pragma unroll
+        for (int w = 0; w < kFlatBlock / 64; ++w) {
+            const uint32_t c = S.cnt[w];
+            before += w < wave ? c : 0u;
+            drawn += c;
+        }
+        uint32_t bit = 0;
+        if (homo) {
+            bit = S.um[before] < S.thr[S.cmb[b]] ? 0u : 1u;
+        } else if (in) {
+            // allele the kid got from this parent; heterozygous parent fixes the indicator
+            const bool allele_u = side ? (t == PT_UU || t == PT_AU) : (t == PT_UU || t == PT_UA);
+            bit = allele_u ? (pt == PT_UA ? 0u : 1u) : (pt == PT_UA ? 1u : 0u);
+        }
+        const uint64_t bits = __ballot(bit != 0u);
+        const int w0 = (b0 + 64 * wave) >> 5;
+        if (lane == 0 && w0 < A.W) col[w0] = (uint32_t)bits;
+        if (lane == 32 && w0 + 1 < A.W) col[w0 + 1] = (uint32_t)(bits >> 32);
+        __syncthreads();
+    }
+    if (A.impute && tid == 0) A.imp_draw[chain] = draw0 + (uint32_t)n_ops + drawn;
+}
+
 }  // namespace
 
 size_t lsampler_lds_bytes(int precision, int cells_cap, int n_ops, int N, int F, int block, bool global_tables) {
@@ -754,6 +1247,39 @@ hipError_t launch_lsampler(const SampArgs& A, int precision, int block, size_t l
         if (gt) hipLaunchKernelGGL((lsampler_kernel<float, true, true>), grid, dim3(block), lds, s, A);
         else hipLaunchKernelGGL((lsampler_kernel<float, true, false>), grid, dim3(block), lds, s, A);
     }
+    return hipGetLastError();
+}
+
+size_t lsampler_build_lds_bytes(int n_ops, int N) { return 4 * (2 * (size_t)n_ops + 2) + (size_t)N; }
+
+size_t lsampler_flat_lds_bytes(int precision, int cells_cap, int n_ops, int n_levels, int N, int F) {
+    const size_t esz = precision == 0 ? 8 : 4;
+    const int NF = N - F;
+    size_t b = 8 * ((size_t)n_ops + 2 * NF + 4);                              // uop, um, thr
+    b += esz * (5 * (size_t)cells_cap + 8 * NF + 4 + 16);                     // tab, pre, dist, f4
+    b += 4 * ((size_t)n_ops + n_levels + 1 + kFlatBlock / 64) + N + 2 * NF;   // maxbits, lvl, cnt, pmk, cmb
+    return (b + 15) / 16 * 16;
+}
+
+hipError_t configure_lsampler_flat_lds(int precision, size_t lds) {
+    if (lds <= 64 * 1024) return hipSuccess;
+    const void* k = precision == 0 ? (const void*)lsampler_flat_kernel<double, false>
+                                   : (const void*)lsampler_flat_kernel<float, true>;
+    return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+}
+
+hipError_t launch_lsampler_build(const SampArgs& A, int precision, uint32_t* task, uint32_t* level_task, uint32_t* rrec,
+                                 size_t lds, hipStream_t s) {
+    hipLaunchKernelGGL(lsampler_build_kernel, dim3(A.M), dim3(kFlatBlock), lds, s, A, precision == 0 ? 1 : 0, task,
+                       level_task, rrec);
+    return hipGetLastError();
+}
+
+hipError_t launch_lsampler_flat(const SampArgs& A, int precision, size_t lds, int blocks_x, int blocks_y,
+                                hipStream_t s) {
+    const dim3 grid(blocks_x, blocks_y), block(kFlatBlock);
+    if (precision == 0) hipLaunchKernelGGL((lsampler_flat_kernel<double, false>), grid, block, lds, s, A);
+    else hipLaunchKernelGGL((lsampler_flat_kernel<float, true>), grid, block, lds, s, A);
     return hipGetLastError();
 }
 

@@ -55,7 +55,40 @@ struct SampArgs {
     // slot (blockIdx.x + gridDim.x blockIdx.y) of 5 cells_cap entries
     // (pedigrees whose tables exceed LDS at some locus)
     void* gtables;
+    // the flat kernel's per-locus tables (lsampler_build fills them): task
+    // records of kTaskWords words (4 per cell, cells in level order), the first
+    // task of each level, and the reverse records of kRevWords words in
+    // reverse-level order
+    const uint32_t* task;
+    const uint32_t* task_base;   // [M+1] first cell of each locus
+    const uint32_t* level_task;  // [M][n_levels+1]
+    const uint32_t* rrec;        // [M][n_ops]
+    int max_rlevel_ops;
 };
+
+// Words of a task record: the product one (cell, value of the peel node) needs.
+// Factor indices address the locus's transmission entries (4 per meiosis, then
+// the constants 1 and 0), table indices its cells.
+//   0     trait probability (FP32 bits; FP64: low word, word 7 the high one), 0 when illegal
+//   1     consumed tables (bits 0-3) | factors (4-7) | PARENT (8) | first task of its op (9) | op << 16
+//   2-4   factor indices, two per word: parents' pair (CHILD), a pair per child (PARENT)
+//   5     first two consumed cells; 6: the third | its op << 16; 7: the first two's ops (FP32)
+constexpr int kTaskWords = 8;
+constexpr int kFlatMaxPrev = 3, kFlatMaxKids = 3;
+// Words of a reverse record: 0 legal masks (4 bits per cutset digit) | 1 first
+// cell | 2-5 cutset persons and the peel node, 16 bits each (peel: high half of
+// word 5) | 6 cutset size | op << 8
+constexpr int kRevWords = 8;
+constexpr int kFlatBlock = 256;
+
+// Fills task, level_task and rrec of every locus.
+hipError_t launch_lsampler_build(const SampArgs& A, int precision, uint32_t* task, uint32_t* level_task, uint32_t* rrec,
+                                 size_t lds, hipStream_t s);
+size_t lsampler_build_lds_bytes(int n_ops, int N);
+size_t lsampler_flat_lds_bytes(int precision, int cells_cap, int n_ops, int n_levels, int N, int F);
+hipError_t configure_lsampler_flat_lds(int precision, size_t lds);
+hipError_t launch_lsampler_flat(const SampArgs& A, int precision, size_t lds, int blocks_x, int blocks_y,
+                                hipStream_t s);
 
 // L-sampler workgroup: four wavefronts share each peel level; launches of
 // at most kLsamplerWideGroups workgroups (too few to fill the device) use

@@ -163,7 +163,12 @@ std::string compile_sampler_program(const PedigreeView& ped, const PeelView& pv,
     P.rlevel_off[P.n_rlevels] = (int)P.rlevel_ops.size();
 
     // LDS bound: summed compact table sizes at the worst locus
-    int64_t worst = 0;
+    for (const SampOp& d : P.ops) {
+        P.max_prev = std::max(P.max_prev, d.n_prev);
+        P.max_child = std::max(P.max_child, d.n_child);
+    }
+    int64_t worst = 0, sum = 0;
+    P.cell_base.assign((size_t)M + 1, 0u);
     for (int l = 0; l < M; ++l) {
         int64_t tot = 0;
         for (int o = 0; o < n; ++o) {
@@ -172,7 +177,10 @@ std::string compile_sampler_program(const PedigreeView& ped, const PeelView& pv,
             tot += s;
         }
         worst = std::max(worst, tot);
+        sum += tot;
+        P.cell_base[(size_t)l + 1] = (uint32_t)sum;
     }
+    if (sum > (int64_t)UINT32_MAX / 4) P.cell_base.clear();
     *max_cells = worst;
     return "";
 }

@@ -66,6 +66,8 @@ struct SampProgram {
     std::vector<int32_t> rlevel_off;   // [n_rlevels+1] reverse-sampling levels
     std::vector<int32_t> rlevel_ops;
     int max_ops_per_rlevel = 0;
+    int max_prev = 0, max_child = 0;   // consumed tables and PARENT children of any op
+    std::vector<uint32_t> cell_base;   // [M+1] prefix sums of the loci's table cells; empty when they pass 32 bits
 };
 
 // Compiles the sampler program.  `legal` is [N][M] (bit t: trait t legal at
