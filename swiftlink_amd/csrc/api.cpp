@@ -12,7 +12,7 @@
 
 #include "../../include/swiftlink_amd.h"
 #include "kernels.h"
-#include "lane64.h"
+#include "lanepeel.h"
 #include "msampler_kernels.h"
 #include "peelseq.h"
 #include "philox.h"
@@ -35,10 +35,14 @@ constexpr int kMaxGridZ = 65535;
 // graphs from which the lane kernel scores a launch by default (half its lanes busy)
 constexpr int kLaneMinGraphs = 32;
 // evaluations (graphs x intervals x positions) from which FP64 scoring and the
-// adjoint run one evaluation per lane (lane64.hip)
-constexpr int64_t kL64MinEvals = 16384;
-constexpr int64_t kL64MinGradEvals = 6144;
-constexpr int kL64LeastWaves = 256;
+// adjoint run one evaluation per lane (lanepeel.hip)
+constexpr int64_t kLpMinEvals = 16384;
+constexpr int64_t kLpMinGradEvals = 6144;
+constexpr int64_t kCus = 256;
+constexpr size_t kLpLeastWaves = 256;
+// bytes of the lane peel's table slots: for scoring, and for the adjoint
+constexpr size_t kLpScoreBytes = (size_t)256 << 20;
+constexpr size_t kLpGradBytes = (size_t)4 << 30;
 // records of the flat L-sampler (32 bytes per cell and trait value) a context may hold
 constexpr size_t kFlatMaxBytes = (size_t)4 << 30;
 }
@@ -77,14 +81,14 @@ struct sl_ctx {
     double* d_scalar = nullptr;
     sl::SeqOp* d_seq = nullptr;  // the program's sequential form (lane kernel)
     uint32_t* d_lstream = nullptr;  // and its descriptor stream
-    uint32_t* d_l64_hdr = nullptr;   // the FP64 lane program
-    uint32_t* d_l64_fwd = nullptr;
-    uint32_t* g_l64_hdr = nullptr;   // and the adjoint's
-    uint32_t* g_l64_fwd = nullptr;
-    uint32_t* g_l64_rev = nullptr;
-    double* d_l64 = nullptr;         // its wavefronts' table slots
-    size_t l64_cap = 0;
-    size_t l64_limit = SIZE_MAX;     // bytes past which an allocation has failed
+    uint32_t* d_lp_hdr = nullptr;    // the lane peel's program
+    uint32_t* d_lp_fwd = nullptr;
+    uint32_t* g_lp_hdr = nullptr;   // and the adjoint's
+    uint32_t* g_lp_fwd = nullptr;
+    uint32_t* g_lp_rev = nullptr;
+    void* d_lp = nullptr;            // its wavefronts' table slots
+    size_t lp_bytes = 0;
+    size_t lp_limit = SIZE_MAX;      // bytes past which an allocation has failed
     bool lod_global = false;     // the workgroup kernel's arena in global-memory slots (too large for LDS)
     void* d_lgt = nullptr;       // kLodGlobalSlots slots of arena_bytes
     size_t lgt_cap = 0;
@@ -340,53 +344,87 @@ bool lane_mode(const sl_ctx* c, int G) {
     return c->lod_kernel == SL_LOD_LANES || G >= kLaneMinGraphs;
 }
 
+// Scoring with one evaluation per lane (lanepeel.hip): the form that serves a
+// launch of G graphs, or -1.  Each form gives the terms and chunks of the kernel
+// it stands in for, so it serves only what that kernel would by default: the
+// FP32 lane kernel's launches, and the workgroup kernel's of one graph per
+// chunk.  Few evaluations leave most of the device idle for the length of one
+// wavefront's peel; the kernels cross near 16 k evaluations at 30 to 400 people
+// (FP64, us, workgroup against lanes: 118/121 at 15840 and 30 people, 413/276 at
+// 19980 and 150, 1057/526 at 39980 and 200).
+int lanepeel_form(const sl_ctx* c, int G) {
+    if (!c->prog.lp_ok || c->lod_kernel != SL_LOD_AUTO || sl::lanepeel_lds_bytes(c->W) > 64 * 1024 ||
+        (int64_t)G * (c->M - 1) * c->npos < kLpMinEvals)
+        return -1;
+    const size_t slot = sl::lanepeel_slot_bytes(c->prog.lp_arena, 0, c->precision == SL_FP64);
+    if (c->lp_bytes < std::max(slot, std::min(kLpScoreBytes, kLpLeastWaves * slot))) return -1;  // no memory for them
+    if (lane_mode(c, G)) {
+        // the FP32 lane kernel's wavefronts hold their tables in LDS; while all
+        // of a launch's are on the device at once it is the faster (30 people,
+        // 64 graphs: 82 us against 97), past that the lane peel (150 people, 64
+        // graphs: 1328 us against 790; 77 people, 70 graphs: 318 against 227)
+        const int64_t waves = (int64_t)(c->M - 1) * c->npos * ((G + 63) / 64);
+        if (waves <= kCus * (int64_t)(160 * 1024 / c->lane_lds)) return -1;
+        // 64 graphs to a wavefront where that leaves few lanes empty
+        return (G + 63) / 64 * 64 > G + G / 16 ? sl::kLpFloatLanesFlat : sl::kLpFloatLanes;
+    }
+    if (c->gpw != 1) return -1;
+    return c->precision == SL_FP64 ? sl::kLpDouble : sl::kLpFloat;
+}
+
+// graphs whose log-sum is one partial of a launch of G graphs
+int graphs_per_chunk(const sl_ctx* c, int G) {
+    const int form = lanepeel_form(c, G);
+    if (form >= 0) return form == sl::kLpFloatLanes || form == sl::kLpFloatLanesFlat ? sl::kLaneGraphs : 1;
+    return lane_mode(c, G) ? sl::kLaneGraphs : c->gpw;
+}
+
 int lod_chunks(const sl_ctx* c, int G) {
-    const int per = lane_mode(c, G) ? sl::kLaneGraphs : c->gpw;
+    const int per = graphs_per_chunk(c, G);
     return (G + per - 1) / per;
 }
 
-// FP64 scoring with one evaluation per lane: its terms are the workgroup
-// kernel's bit for bit, each graph a chunk of its own, so it serves launches
-// of one graph per chunk when nothing else was asked for.  Few evaluations
-// leave most of the device idle for the length of one wavefront's peel: the two
-// kernels cross near 16 k evaluations at 30 to 400 people (us, workgroup
-// against lanes: 118/121 at 15840 and 30 people, 413/276 at 19980 and 150,
-// 1057/526 at 39980 and 200).
-bool lane64_mode(const sl_ctx* c, int G) {
-    return c->precision == SL_FP64 && c->lod_kernel == SL_LOD_AUTO && c->gpw == 1 && c->prog.l64_ok &&
-           sl::lane64_lds_bytes(c->W) <= 64 * 1024 && (int64_t)G * (c->M - 1) * c->npos >= kL64MinEvals;
+// partials a launch of G graphs writes, in units of (M-1) x npos: one per chunk,
+// and every graph's terms where the chunks are summed from them
+size_t partial_rows(const sl_ctx* c, int G) {
+    return (size_t)lod_chunks(c, G) + (lanepeel_form(c, G) == sl::kLpFloatLanesFlat ? (size_t)G : 0);
 }
 
-// A lane program's table slots for a launch of E evaluations: the wavefronts
-// that have one, or 0 when the device has no memory for even a quarter of the
-// device's SIMDs (the workgroup kernel then serves the call).  A size that was
-// refused is not asked for again.
-int ensure_lane64(sl_ctx* c, const PeelProgram& P, int64_t E) {
-    const size_t slot = sl::lane64_slot_bytes(P.l64_arena, P.l64_adj);
-    const size_t want = (size_t)sl::lane64_waves(E, slot);
-    const size_t least = std::min(want, (size_t)kL64LeastWaves);
+// The lane peel's table slots: at least `bytes`, or as much as the device gives
+// down to a quarter of its SIMDs' wavefronts of `slot` bytes each (none below
+// that: the other kernels then serve the calls).  A size that was refused is not
+// asked for again.
+void ensure_lanepeel(sl_ctx* c, size_t bytes, size_t slot) {
+    const size_t least = std::min(bytes, kLpLeastWaves * slot);
     for (;;) {
-        const size_t waves = std::min(want, c->l64_limit / slot);
-        if (waves < least) return 0;
-        if (waves * slot <= c->l64_cap * sizeof(double)) return (int)waves;
-        if (c->d_l64) (void)hipFree(c->d_l64);
-        c->d_l64 = nullptr;
-        c->l64_cap = 0;
-        if (hipMalloc((void**)&c->d_l64, waves * slot) == hipSuccess) {
-            c->l64_cap = waves * slot / sizeof(double);
-            return (int)waves;
+        const size_t want = std::min(bytes, c->lp_limit);
+        if (want <= c->lp_bytes || want < least) return;
+        if (c->d_lp) (void)hipFree(c->d_lp);
+        c->d_lp = nullptr;
+        c->lp_bytes = 0;
+        if (hipMalloc(&c->d_lp, want) == hipSuccess) {
+            c->lp_bytes = want;
+            return;
         }
         (void)hipGetLastError();
-        c->d_l64 = nullptr;
-        c->l64_limit = waves * slot / 2;
+        c->d_lp = nullptr;
+        c->lp_limit = want / 2;
     }
 }
 
-sl::Lane64Args lane64_args(const sl_ctx* c, const PeelProgram& P) {
-    sl::Lane64Args A{};
+// Scoring's slots are allocated with the program, so that scoring itself never
+// allocates (captured sweeps, the allocation-free entry point).
+void ensure_scoring_slots(sl_ctx* c) {
+    if (!c->prog.lp_ok || sl::lanepeel_lds_bytes(c->W) > 64 * 1024) return;
+    const size_t slot = sl::lanepeel_slot_bytes(c->prog.lp_arena, 0, c->precision == SL_FP64);
+    ensure_lanepeel(c, std::min(kLpScoreBytes, 4096 * slot), slot);
+}
+
+sl::LanePeelArgs lanepeel_args(const sl_ctx* c, const PeelProgram& P) {
+    sl::LanePeelArgs A{};
     A.n_ops = P.n_ops;
-    A.arena_cells = P.l64_arena;
-    A.adj_cells = P.l64_adj;
+    A.arena_cells = P.lp_arena;
+    A.adj_cells = P.lp_adj;
     A.N = c->N;
     A.F = c->F;
     A.M = c->M;
@@ -396,11 +434,43 @@ sl::Lane64Args lane64_args(const sl_ctx* c, const PeelProgram& P) {
     A.partial_theta = c->d_ptheta;
     A.log_theta = c->d_logt;
     A.log_anti = c->d_loga;
-    A.scratch = c->d_l64;
+    A.scratch = c->d_lp;
     return A;
 }
 
-hipError_t launch_scoring(sl_ctx* c, sl::LodArgs A, int nchunks) {
+// One scoring launch of the lane peel over A.graphs.
+hipError_t launch_lane_scoring(sl_ctx* c, int form, const sl::LodArgs& A) {
+    sl::LanePeelArgs B = lanepeel_args(c, c->prog);
+    B.hdr = c->d_lp_hdr;
+    B.fwd = c->d_lp_fwd;
+    B.graphs = A.graphs;
+    B.G = A.G;
+    B.partial = A.partial;
+    B.terms = A.terms;
+    B.gate_sweep = A.gate_sweep;
+    B.gate_burnin = A.gate_burnin;
+    B.gate_period = A.gate_period;
+    const size_t nacc = (size_t)(c->M - 1) * c->npos;
+    const sl::LanePeelForm f = (sl::LanePeelForm)form;
+    B.chunked = f == sl::kLpFloatLanes ? 1 : 0;
+    const bool flat = f == sl::kLpFloatLanesFlat;
+    if (flat) {
+        // terms first, into the caller's array or behind the partials
+        B.partial = nullptr;
+        if (!B.terms) B.terms = A.partial + nacc * ((A.G + 63) / 64);
+    }
+    const int64_t E = sl::lanepeel_lanes(f, A.G, c->M - 1, c->npos);
+    const size_t slot = sl::lanepeel_slot_bytes(c->prog.lp_arena, 0, c->precision == SL_FP64);
+    const hipError_t e = sl::launch_lanepeel(B, f, sl::lanepeel_waves(f, E, slot, c->lp_bytes),
+                                             sl::lanepeel_lds_bytes(c->W), c->stream);
+    if (e != hipSuccess || !flat || A.terms) return e;
+    return sl::launch_chunk_sums(B.terms, A.partial, A.G, (int)nacc, A.gate_sweep, A.gate_burnin, A.gate_period,
+                                 c->stream);
+}
+
+// form: lanepeel_form of the call's graphs
+hipError_t launch_scoring(sl_ctx* c, sl::LodArgs A, int nchunks, int form) {
+    if (form >= 0) return launch_lane_scoring(c, form, A);
     if (lane_mode(c, A.G)) return sl::launch_lane_lod(A, c->precision, c->lane_lds, nchunks, c->stream);
     const int nl = c->M - 1;
     if (!c->lod_global) return sl::launch_lod(A, c->precision, c->block, c->lds, nl, nchunks, c->stream);
@@ -486,7 +556,7 @@ int release_all(sl_ctx* c) {
                     c->g_sched_off, c->g_sched_ops, c->d_gdp, c->d_jac, c->d_gterms, c->d_gstate, c->d_sweep,
                     c->d_imp_graphs, c->d_imp_draw, c->d_imp_weight, c->d_imp_status, c->d_elod_pairs,
                     c->d_gtables, c->d_lgt, c->d_lstream, c->d_trace,
-                    c->d_task, c->d_task_base, c->d_level_task, c->d_rrec, c->d_l64_hdr, c->d_l64_fwd, c->g_l64_hdr, c->g_l64_fwd, c->g_l64_rev, c->d_l64};
+                    c->d_task, c->d_task_base, c->d_level_task, c->d_rrec, c->d_lp_hdr, c->d_lp_fwd, c->g_lp_hdr, c->g_lp_fwd, c->g_lp_rev, c->d_lp};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& e : c->ev_pool) (void)hipEventDestroy(e);
@@ -781,8 +851,8 @@ int sl_create(const sl_pedigree_desc* ped, const sl_map_desc* map, const sl_peel
         (rc = upload(c, &c->d_sched_ops, c->prog.sched_ops.data(), c->prog.sched_ops.size())) ||
         (rc = upload(c, &c->d_seq, c->prog.seq.data(), c->prog.seq.size())) ||
         (rc = upload(c, &c->d_lstream, c->prog.lstream.data(), c->prog.lstream.size())) ||
-        (rc = upload(c, &c->d_l64_hdr, c->prog.l64_hdr.data(), c->prog.l64_hdr.size())) ||
-        (rc = upload(c, &c->d_l64_fwd, c->prog.l64_fwd.data(), c->prog.l64_fwd.size())) ||
+        (rc = upload(c, &c->d_lp_hdr, c->prog.lp_hdr.data(), c->prog.lp_hdr.size())) ||
+        (rc = upload(c, &c->d_lp_fwd, c->prog.lp_fwd.data(), c->prog.lp_fwd.size())) ||
         (rc = upload(c, &c->d_trait_d, ped->disease_prob, 4 * (size_t)c->N)) ||
         (rc = upload(c, &c->d_trait_f, tf.data(), tf.size())) ||
         (rc = upload(c, &c->d_ptheta, c->ptheta.data(), c->ptheta.size())) ||
@@ -795,6 +865,7 @@ int sl_create(const sl_pedigree_desc* ped, const sl_map_desc* map, const sl_peel
         delete c;
         return fail(nullptr, rc, m);
     }
+    ensure_scoring_slots(c);
     // arrays both samplers read
     c->mother_h.assign(ped->mother, ped->mother + c->N);
     c->father_h.assign(ped->father, ped->father + c->N);
@@ -937,9 +1008,8 @@ static int lod_run(sl_ctx* c, const uint32_t* dev_graphs, int G, double* terms_d
                    int gate_burnin = 0, int gate_period = 1) {
     const int nchunks = lod_chunks(c, G);
     const size_t nacc = (size_t)(c->M - 1) * c->npos;
-    int rc = ensure(c, &c->d_partial, &c->partial_cap, nacc * nchunks);
+    int rc = ensure(c, &c->d_partial, &c->partial_cap, nacc * partial_rows(c, G));
     if (rc) return rc;
-    const int waves = lane64_mode(c, G) ? ensure_lane64(c, c->prog, (int64_t)nacc * G) : 0;
     sl::LodArgs A = lod_args(c);
     A.graphs = dev_graphs;
     A.G = G;
@@ -954,21 +1024,7 @@ static int lod_run(sl_ctx* c, const uint32_t* dev_graphs, int G, double* terms_d
         e1 = take_event(c);
         if (e0 && e1) SL_HIP(c, hipEventRecord(e0, c->stream));
     }
-    if (waves) {
-        sl::Lane64Args B = lane64_args(c, c->prog);
-        B.hdr = c->d_l64_hdr;
-        B.fwd = c->d_l64_fwd;
-        B.graphs = dev_graphs;
-        B.G = G;
-        B.partial = c->d_partial;
-        B.terms = terms_dev;
-        B.gate_sweep = gate;
-        B.gate_burnin = gate_burnin;
-        B.gate_period = gate_period;
-        SL_HIP(c, sl::launch_lane64(B, false, waves, sl::lane64_lds_bytes(c->W), c->stream));
-    } else {
-        SL_HIP(c, launch_scoring(c, A, nchunks));
-    }
+    SL_HIP(c, launch_scoring(c, A, nchunks, lanepeel_form(c, G)));
     if (c->prof && e0 && e1) {
         SL_HIP(c, hipEventRecord(e1, c->stream));
         c->ev_used.push_back({SL_KERNEL_LOD, e0, e1, 1});
@@ -1024,7 +1080,9 @@ int sl_lod_accumulate_packed_noalloc(sl_ctx* c, const uint32_t* dev_graphs, int3
                     "allocation-free LOD: one chunk's partials ((M-1) x positions x 8 bytes = " +
                         std::to_string(nacc * sizeof(double)) + " bytes) exceed the " +
                         std::to_string((size_t)SL_NOALLOC_SCRATCH_BYTES) + "-byte scratch array");
-    const int per = lane_mode(c, G) ? sl::kLaneGraphs : c->gpw;
+    const int per = graphs_per_chunk(c, G);
+    int form = lanepeel_form(c, G);
+    if (form == sl::kLpFloatLanesFlat) form = sl::kLpFloatLanes;  // the same sums without the terms' array
     const int group = (int)std::min<size_t>((size_t)G, std::min<size_t>(max_chunks, 65535) * (size_t)per);
     sl::LodArgs A = lod_args(c);
     A.partial = c->scratch;
@@ -1034,7 +1092,7 @@ int sl_lod_accumulate_packed_noalloc(sl_ctx* c, const uint32_t* dev_graphs, int3
         const int nchunks = (n + per - 1) / per;
         A.graphs = dev_graphs + (size_t)g0 * c->M * c->W;
         A.G = n;
-        SL_HIP(c, launch_scoring(c, A, nchunks));
+        SL_HIP(c, launch_scoring(c, A, nchunks, form));
         SL_HIP(c, sl::launch_lod_merge(c->d_acc, c->scratch, nchunks, (int)nacc, c->stream));
     }
     c->count += G;
@@ -2002,9 +2060,7 @@ int sl_batch_run(sl_batch* b, const sl_schedule* sch, sl_mcmc_stats* stats) {
             st[i].m_sweeps += C - nl;
             if (sl::gate_open(s, sch->burnin, sch->period)) st[i].scored += C;
         }
-        const int nchunks = lod_chunks(c, C);
-        int rc = ensure(c, &c->d_partial, &c->partial_cap, (size_t)(c->M - 1) * c->npos * nchunks);
-        if (!rc && lane64_mode(c, C)) (void)ensure_lane64(c, c->prog, (int64_t)(c->M - 1) * c->npos * C);
+        int rc = ensure(c, &c->d_partial, &c->partial_cap, (size_t)(c->M - 1) * c->npos * partial_rows(c, C));
         if (!rc && c->m_ready) rc = ensure(c, &c->d_order, &c->order_cap, c->meioses_h.size() * (size_t)C);
         if (!rc && c->samp_ready) rc = ensure_gtables(c);
         if (rc) return rc;
@@ -2129,7 +2185,7 @@ int install_lod_program(sl_ctx* c) {
     void** bufs[] = {(void**)&c->d_ops, (void**)&c->d_prevs, (void**)&c->d_children, (void**)&c->d_tasks,
                      (void**)&c->d_tinfo, (void**)&c->d_idx, (void**)&c->d_level_base, (void**)&c->d_sched_off,
                      (void**)&c->d_sched_ops, (void**)&c->d_trait_d, (void**)&c->d_trait_f, (void**)&c->d_seq,
-                     (void**)&c->d_lstream, (void**)&c->d_l64_hdr, (void**)&c->d_l64_fwd};
+                     (void**)&c->d_lstream, (void**)&c->d_lp_hdr, (void**)&c->d_lp_fwd};
     for (void** b : bufs) {
         if (*b) SL_HIP(c, hipFree(*b));
         *b = nullptr;
@@ -2143,6 +2199,7 @@ int install_lod_program(sl_ctx* c) {
     c->lane_ok = c->precision == SL_FP32_RESCALED && c->prog.lane_stream_ok && lane_lds <= 160 * 1024;
     SL_HIP(c, sl::configure_lod_lds(c->precision, c->lds, c->lod_global));
     if (int rc2 = ensure_lod_slots(c)) return rc2;
+    ensure_scoring_slots(c);
     if (c->lane_ok) SL_HIP(c, sl::configure_lane_lds(c->precision, c->lane_lds));
     std::vector<float> tf(c->dp_h.size());
     for (size_t i = 0; i < tf.size(); ++i) tf[i] = (float)c->dp_h[i];
@@ -2158,8 +2215,8 @@ int install_lod_program(sl_ctx* c) {
         (rc = upload(c, &c->d_sched_ops, c->prog.sched_ops.data(), c->prog.sched_ops.size())) ||
         (rc = upload(c, &c->d_seq, c->prog.seq.data(), c->prog.seq.size())) ||
         (rc = upload(c, &c->d_lstream, c->prog.lstream.data(), c->prog.lstream.size())) ||
-        (rc = upload(c, &c->d_l64_hdr, c->prog.l64_hdr.data(), c->prog.l64_hdr.size())) ||
-        (rc = upload(c, &c->d_l64_fwd, c->prog.l64_fwd.data(), c->prog.l64_fwd.size())) ||
+        (rc = upload(c, &c->d_lp_hdr, c->prog.lp_hdr.data(), c->prog.lp_hdr.size())) ||
+        (rc = upload(c, &c->d_lp_fwd, c->prog.lp_fwd.data(), c->prog.lp_fwd.size())) ||
         (rc = upload(c, &c->d_trait_d, c->dp_h.data(), c->dp_h.size())) ||
         (rc = upload(c, &c->d_trait_f, tf.data(), tf.size())))
         return rc;
@@ -2171,12 +2228,12 @@ int install_lod_program(sl_ctx* c) {
 // its headers (the program itself does not depend on them).
 int upload_grad_lanes(sl_ctx* c) {
     PeelProgram& P = c->gprog;
-    if (!P.l64_ok) return SL_OK;
+    if (!P.lp_ok) return SL_OK;
     for (int i = 0; i < P.n_ops; ++i) {
-        uint32_t* h = P.l64_hdr.data() + (size_t)i * sl::kL64Header;
+        uint32_t* h = P.lp_hdr.data() + (size_t)i * sl::kLpHeader;
         memcpy(h + sl::kHTrait, c->dp_h.data() + 4 * (size_t)h[sl::kHPerson], 4 * sizeof(double));
     }
-    SL_HIP(c, hipMemcpyAsync(c->g_l64_hdr, P.l64_hdr.data(), P.l64_hdr.size() * sizeof(uint32_t),
+    SL_HIP(c, hipMemcpyAsync(c->g_lp_hdr, P.lp_hdr.data(), P.lp_hdr.size() * sizeof(uint32_t),
                              hipMemcpyHostToDevice, c->stream));
     SL_HIP(c, hipStreamSynchronize(c->stream));
     return SL_OK;
@@ -2207,9 +2264,9 @@ int ensure_grad_program(sl_ctx* c) {
         (rc = upload(c, &c->g_level_base, P.level_base.data(), P.level_base.size())) ||
         (rc = upload(c, &c->g_sched_off, P.sched_off.data(), P.sched_off.size())) ||
         (rc = upload(c, &c->g_sched_ops, P.sched_ops.data(), P.sched_ops.size())) ||
-        (rc = upload<uint32_t>(c, &c->g_l64_hdr, nullptr, P.l64_hdr.size())) ||
-        (rc = upload(c, &c->g_l64_fwd, P.l64_fwd.data(), P.l64_fwd.size())) ||
-        (rc = upload(c, &c->g_l64_rev, P.l64_rev.data(), P.l64_rev.size())) || (rc = upload_grad_lanes(c)))
+        (rc = upload<uint32_t>(c, &c->g_lp_hdr, nullptr, P.lp_hdr.size())) ||
+        (rc = upload(c, &c->g_lp_fwd, P.lp_fwd.data(), P.lp_fwd.size())) ||
+        (rc = upload(c, &c->g_lp_rev, P.lp_rev.data(), P.lp_rev.size())) || (rc = upload_grad_lanes(c)))
         return rc;
     SL_HIP(c, hipStreamSynchronize(c->stream));
     c->g_ready = true;
@@ -2243,27 +2300,29 @@ sl::LodArgs grad_args(sl_ctx* c) {
 }
 
 // One launch of the adjoint over A.graphs (A.G of them) into out: one
-// evaluation per lane from kL64MinGradEvals evaluations, else one workgroup
+// evaluation per lane from kLpMinGradEvals evaluations, else one workgroup
 // each (a lane's reverse pass takes milliseconds, however few there are: at 30,
 // 77 and 150 people the two cross at 6 to 7 k evaluations).
 int launch_adjoint(sl_ctx* c, const sl::LodArgs& A, double* out) {
     const int64_t E = (int64_t)A.G * (c->M - 1) * c->npos;
-    const bool lanes = c->gprog.l64_ok && E >= kL64MinGradEvals && sl::lane64_lds_bytes(c->W) <= 64 * 1024;
-    const int waves = lanes ? ensure_lane64(c, c->gprog, E) : 0;
-    if (!waves) {
+    const size_t slot = sl::lanepeel_slot_bytes(c->gprog.lp_arena, c->gprog.lp_adj, true);
+    const bool lanes = c->gprog.lp_ok && E >= kLpMinGradEvals && sl::lanepeel_lds_bytes(c->W) <= 64 * 1024;
+    if (lanes) ensure_lanepeel(c, sl::lanepeel_waves(sl::kLpAdjoint, E, slot, kLpGradBytes) * slot, slot);
+    if (!lanes || c->lp_bytes < std::min<size_t>(kLpLeastWaves, (size_t)((E + 63) / 64)) * slot) {
         sl::GradArgs Gd{c->d_jac, out, c->npos};
         SL_HIP(c, sl::launch_grad(A, Gd, 0, c->g_lds, c->stream));
         return SL_OK;
     }
-    sl::Lane64Args B = lane64_args(c, c->gprog);
-    B.hdr = c->g_l64_hdr;
-    B.fwd = c->g_l64_fwd;
-    B.rev = c->g_l64_rev;
+    sl::LanePeelArgs B = lanepeel_args(c, c->gprog);
+    B.hdr = c->g_lp_hdr;
+    B.fwd = c->g_lp_fwd;
+    B.rev = c->g_lp_rev;
     B.graphs = A.graphs;
     B.G = A.G;
     B.jac = c->d_jac;
     B.out = out;
-    SL_HIP(c, sl::launch_lane64(B, true, waves, sl::lane64_lds_bytes(c->W), c->stream));
+    SL_HIP(c, sl::launch_lanepeel(B, sl::kLpAdjoint, sl::lanepeel_waves(sl::kLpAdjoint, E, slot, c->lp_bytes),
+                                  sl::lanepeel_lds_bytes(c->W), c->stream));
     return SL_OK;
 }
 

@@ -100,33 +100,33 @@ int place(const std::vector<int>& ids, const std::vector<int>& size, const std::
 // The FP64 lane program (program.h) of the compiled ops in the order `post`.
 // tape: every table keeps a cell range of its own (the adjoint reads them all)
 // and the generic ops get their reverse lists.
-std::string build_lane64(const PedigreeView& ped, const PeelView& pv, const std::vector<std::vector<int>>& cuts,
+std::string build_lanepeel(const PedigreeView& ped, const PeelView& pv, const std::vector<std::vector<int>>& cuts,
                          const std::vector<int>& post, const std::vector<int>& born, const std::vector<int>& dies,
                          bool tape, PeelProgram& P) {
     const int n = P.n_ops;
     auto has = [](const std::vector<int>& v, int x) { return std::find(v.begin(), v.end(), x) != v.end(); };
-    std::vector<int> kind(n, kL64Generic), consumer(n, -1), size(n);
+    std::vector<int> kind(n, kLpGeneric), consumer(n, -1), size(n);
     std::vector<std::vector<int>> cls(n);
     for (int o = 0; o < n; ++o) {
         const OpDesc& d = P.ops[o];
         size[o] = d.size;
-        if (d.n_prev > kL64MaxPrev || d.n_child > kL64MaxKids) return "";  // l64_ok stays false
+        if (d.n_prev > kLpMaxPrev || d.n_child > kLpMaxKids) return "";  // lp_ok stays false
         for (int q = pv.prev_off[o]; q < pv.prev_off[o + 1]; ++q) consumer[pv.prev[q]] = o;
         if (d.type == kChild && d.k == 2 && d.n_prev <= 2) {
             bool ok = ped.mother[d.peel] != ped.father[d.peel];
             for (int q = 0; q < d.n_prev; ++q) {
                 const std::vector<int>& c = cuts[pv.prev[pv.prev_off[o] + q]];
-                int k = kL64None;
-                if (c.size() == 1 && c[0] == d.peel) k = kL64K;
-                if (c.size() == 2 && has(c, cuts[o][0]) && has(c, cuts[o][1])) k = kL64M;
+                int k = kLpNone;
+                if (c.size() == 1 && c[0] == d.peel) k = kLpK;
+                if (c.size() == 2 && has(c, cuts[o][0]) && has(c, cuts[o][1])) k = kLpM;
                 cls[o].push_back(k);
-                ok &= k != kL64None;
+                ok &= k != kLpNone;
             }
-            if (ok) kind[o] = kL64Child;
+            if (ok) kind[o] = kLpChild;
         }
         if (d.type == kPartner && d.k == 1 && d.n_prev == 1) {
             const std::vector<int>& c = cuts[pv.prev[pv.prev_off[o]]];
-            if (c.size() == 2 && has(c, d.peel) && has(c, cuts[o][0])) kind[o] = kL64Founder;
+            if (c.size() == 2 && has(c, d.peel) && has(c, cuts[o][0])) kind[o] = kLpFounder;
         }
     }
     // tables handed on in registers: to the next op, when both ends work in
@@ -135,9 +135,9 @@ std::string build_lane64(const PedigreeView& ped, const PeelView& pv, const std:
     std::vector<char> chained(n, 0);
     for (int i = 0; i + 1 < n; ++i) {
         const int o = post[i], x = post[i + 1];
-        if (consumer[o] != x || kind[o] == kL64Generic || kind[x] == kL64Generic) continue;
-        if (kind[x] == kL64Founder) chained[o] = kind[o] == kL64Child;
-        else chained[o] = kind[o] == kL64Founder ||
+        if (consumer[o] != x || kind[o] == kLpGeneric || kind[x] == kLpGeneric) continue;
+        if (kind[x] == kLpFounder) chained[o] = kind[o] == kLpChild;
+        else chained[o] = kind[o] == kLpFounder ||
                           (ped.mother[P.ops[o].peel] == ped.mother[P.ops[x].peel] &&
                            ped.father[P.ops[o].peel] == ped.father[P.ops[x].peel]);
     }
@@ -152,16 +152,16 @@ std::string build_lane64(const PedigreeView& ped, const PeelView& pv, const std:
             off[o] = top;
             top += size[o];
         }
-        P.l64_arena = top;
+        P.lp_arena = top;
         // a table's adjoint lives from its consumer's reverse step to its own
         std::vector<int> rb(n), rd(n);
         for (int o = 0; o < n; ++o) {
             rb[o] = n - 1 - std::min(dies[o], n - 1);
             rd[o] = n - 1 - born[o];
         }
-        P.l64_adj = place(stored, size, rb, rd, &adj);
+        P.lp_adj = place(stored, size, rb, rd, &adj);
     } else {
-        P.l64_arena = place(stored, size, born, dies, &off);
+        P.lp_arena = place(stored, size, born, dies, &off);
     }
     // compact cell of table o at (a: value of person pa, b: of pb), or 0xFF
     auto cell_of = [&](int o, int pa, int a, int pb, int b) -> uint32_t {
@@ -176,11 +176,11 @@ std::string build_lane64(const PedigreeView& ped, const PeelView& pv, const std:
         (void)pb;
         return ix;
     };
-    P.l64_hdr.assign((size_t)n * kL64Header, 0u);
+    P.lp_hdr.assign((size_t)n * kLpHeader, 0u);
     for (int i = 0; i < n; ++i) {
         const int o = post[i];
         const OpDesc& d = P.ops[o];
-        uint32_t* h = P.l64_hdr.data() + (size_t)i * kL64Header;
+        uint32_t* h = P.lp_hdr.data() + (size_t)i * kLpHeader;
         h[kHKind] = (uint32_t)kind[o];
         h[kHType] = (uint32_t)d.type;
         h[kHPrevs] = (uint32_t)d.n_prev;
@@ -189,11 +189,12 @@ std::string build_lane64(const PedigreeView& ped, const PeelView& pv, const std:
         h[kHAdj] = (uint32_t)adj[o];
         h[kHPeel] = (uint32_t)(d.peel - ped.F);
         h[kHPerson] = (uint32_t)d.peel;
+        h[kHIntoLast] = consumer[o] == P.last_op ? 1u : 0u;
         h[kHKids] = (uint32_t)d.n_child;
         memcpy(h + kHTrait, ped.disease_prob + 4 * (size_t)d.peel, 4 * sizeof(double));
         const int mat = d.type == kChild ? ped.mother[d.peel] : -1, pat = d.type == kChild ? ped.father[d.peel] : -1;
         int axis_m = mat, axis_p = pat;  // the axes of a 4 x 4 register table of this op's consumed table
-        if (kind[o] == kL64Founder) {
+        if (kind[o] == kLpFounder) {
             // a table over a couple: its axes are the parents of the kid it peeled, when it
             // comes in registers; otherwise the peel node takes the maternal axis
             const int p = pv.prev[pv.prev_off[o]];
@@ -205,10 +206,12 @@ std::string build_lane64(const PedigreeView& ped, const PeelView& pv, const std:
                 h[kHPeelIsPat] = 1u;
             }
         }
+        if (kind[o] == kLpChild) h[kHMask] = (uint32_t)P.lod_mask[mat] | ((uint32_t)P.lod_mask[pat] << 4);
+        if (kind[o] == kLpFounder) h[kHMask] = (uint32_t)P.lod_mask[cuts[o][0]];
         for (int v = 0; v < 16; ++v) {
             uint32_t ix = 0xFFu;
-            if (kind[o] == kL64Child) ix = cell_of(o, mat, v >> 2, pat, v & 3);
-            if (kind[o] == kL64Founder && v < 4) ix = cell_of(o, cuts[o][0], v, -1, 0);
+            if (kind[o] == kLpChild) ix = cell_of(o, mat, v >> 2, pat, v & 3);
+            if (kind[o] == kLpFounder && v < 4) ix = cell_of(o, cuts[o][0], v, -1, 0);
             h[kHMap + (v >> 2)] |= ix << (8 * (v & 3));
         }
         for (int q = 0; q < d.n_prev; ++q) {
@@ -217,11 +220,11 @@ std::string build_lane64(const PedigreeView& ped, const PeelView& pv, const std:
             hp[kPOff] = chained[p] && !tape ? 0xFFFFFFFFu : (uint32_t)off[p];
             hp[kPAdj] = chained[p] ? 0xFFFFFFFFu : (uint32_t)adj[p];
             hp[kPSize] = (uint32_t)size[p];
-            hp[kPClass] = kind[o] == kL64Child ? (uint32_t)cls[o][q] : 0u;
-            if (kind[o] == kL64Generic) continue;
+            hp[kPClass] = kind[o] == kLpChild ? (uint32_t)cls[o][q] : 0u;
+            if (kind[o] == kLpGeneric) continue;
             for (int v = 0; v < 16; ++v) {
                 uint32_t ix = 0xFFu;
-                if (kind[o] == kL64Child && cls[o][q] == kL64K) ix = v < 4 ? cell_of(p, d.peel, v, -1, 0) : 0xFFu;
+                if (kind[o] == kLpChild && cls[o][q] == kLpK) ix = v < 4 ? cell_of(p, d.peel, v, -1, 0) : 0xFFu;
                 else ix = cell_of(p, axis_m, v >> 2, axis_p, v & 3);
                 hp[kPMap + (v >> 2)] |= ix << (8 * (v & 3));
             }
@@ -229,24 +232,24 @@ std::string build_lane64(const PedigreeView& ped, const PeelView& pv, const std:
         }
         for (int ch = 0; ch < d.n_child; ++ch)
             h[kHKid + ch] = (uint32_t)(P.children[d.child_off + ch].person - ped.F);
-        if (kind[o] != kL64Generic) continue;
+        if (kind[o] != kLpGeneric) continue;
         // generic cells: four terms [info, consumed cells]; info: trait value
         // (bits 0-1), non-zero probability (bit 2), per child the allowed
         // transmitted alleles (bits 4.., maternal pair then paternal pair)
-        h[kHStream] = (uint32_t)P.l64_fwd.size();
+        h[kHStream] = (uint32_t)P.lp_fwd.size();
         std::vector<uint32_t> info(4 * (size_t)d.size);
         for (int ct = 0; ct < 4 * d.size; ++ct) {
             const uint32_t ti = P.tinfo[(size_t)d.task_base * 4 + ct];
             uint32_t w = ti & 7u;
             for (int ch = 0; ch < d.n_child; ++ch) w |= ((ti >> (4 + 4 * ch)) & 15u) << (4 + 4 * ch);
             info[ct] = w;
-            P.l64_fwd.push_back(w);
-            for (int q = 0; q < kL64MaxPrev; ++q) {
+            P.lp_fwd.push_back(w);
+            for (int q = 0; q < kLpMaxPrev; ++q) {
                 uint32_t c = 0;
                 if (q < d.n_prev)
                     c = (uint32_t)off[pv.prev[pv.prev_off[o] + q]] +
                         ((w & 4u) ? P.idx[(size_t)d.idx_base + (size_t)ct * d.n_prev + q] : 0u);
-                P.l64_fwd.push_back(c);
+                P.lp_fwd.push_back(c);
             }
         }
         if (!tape) continue;
@@ -257,22 +260,22 @@ std::string build_lane64(const PedigreeView& ped, const PeelView& pv, const std:
                 if (!(info[ct] & 4u)) return "";  // the adjoint's program has no pruned terms
                 into[P.idx[(size_t)d.idx_base + (size_t)ct * d.n_prev + q]].push_back(ct);
             }
-            h[kHRev + q] = (uint32_t)P.l64_rev.size();
+            h[kHRev + q] = (uint32_t)P.lp_rev.size();
             // a cell nothing reads (a kid's trait its parent cannot give) gets
             // one contribution without the probability bit, a zero; so does
             // the padding to whole groups of four
             size_t entries = 0;
             auto put = [&](int ct, bool last, bool real) {
-                P.l64_rev.push_back((uint32_t)(adj[o] + ct / 4) | (last ? kRevLast : 0u));
-                P.l64_rev.push_back(real ? info[ct] | ((uint32_t)(ct & 3) << 30) : 0u);
+                P.lp_rev.push_back((uint32_t)(adj[o] + ct / 4) | (last ? kRevLast : 0u));
+                P.lp_rev.push_back(real ? info[ct] | ((uint32_t)(ct & 3) << 30) : 0u);
                 int n_other = 0;
                 for (int r = 0; r < d.n_prev; ++r)
                     if (r != q) {
-                        P.l64_rev.push_back((uint32_t)off[pv.prev[pv.prev_off[o] + r]] +
+                        P.lp_rev.push_back((uint32_t)off[pv.prev[pv.prev_off[o] + r]] +
                                             P.idx[(size_t)d.idx_base + (size_t)ct * d.n_prev + r]);
                         ++n_other;
                     }
-                for (; n_other < 2; ++n_other) P.l64_rev.push_back(0u);
+                for (; n_other < 2; ++n_other) P.lp_rev.push_back(0u);
                 ++entries;
             };
             for (auto& v : into) {
@@ -283,7 +286,7 @@ std::string build_lane64(const PedigreeView& ped, const PeelView& pv, const std:
             h[kHGroups + q] = (uint32_t)(entries / 4);
         }
     }
-    P.l64_ok = true;
+    P.lp_ok = true;
     return "";
 }
 
@@ -712,7 +715,7 @@ std::string compile_lod_program(const PedigreeView& ped, const PeelView& pv, int
         }
         if (!P.lane_stream_ok) S.clear();
         S.resize(S.size() + 3 * 64, 0u);
-        if (std::string why = build_lane64(ped, pv, cuts, post, born, dies, !reuse, P); !why.empty()) return why;
+        if (std::string why = build_lanepeel(ped, pv, cuts, post, born, dies, !reuse, P); !why.empty()) return why;
     }
     P.flops_per_eval = flops;
     P.lds_bytes_per_eval = lds;  // in elements; scaled by the element size by the caller

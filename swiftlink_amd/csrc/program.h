@@ -37,37 +37,39 @@ constexpr int kLaneMaxPrev = 7;  // consumed tables of an op the lane kernel tak
 inline int lane_cell_stride(int n_prev) { return n_prev <= 1 ? 8 : n_prev <= 3 ? 16 : 32; }
 inline int lane_cells_per_block(int n_prev) { return 32 / lane_cell_stride(n_prev); }
 
-// FP64 lane program.  An op is kL64Child (a CHILD peel over just its two
+// Lane peel program.  An op is kLpChild (a CHILD peel over just its two
 // parents, consuming tables over the kid (class K) or over the parents (class
-// M)), kL64Founder (a PARTNER peel of one of the two people of the one table
+// M)), kLpFounder (a PARTNER peel of one of the two people of the one table
 // it consumes, leaving the other) or generic.  A Child's or Founder's table
 // goes to the next op in registers when that op consumes it and is one of the
 // two; otherwise it is stored in the lane's arena.
-constexpr int kL64Header = 64;
-constexpr int kL64MaxPrev = 3, kL64MaxKids = 3;
+constexpr int kLpHeader = 64;
+constexpr int kLpMaxPrev = 3, kLpMaxKids = 3;
 constexpr uint32_t kRevLast = 0x80000000u;
-enum L64Kind : int32_t { kL64Generic = 0, kL64Child = 1, kL64Founder = 2 };
-enum L64Class : int32_t { kL64None = 0, kL64K = 1, kL64M = 2 };
+enum LpKind : int32_t { kLpGeneric = 0, kLpChild = 1, kLpFounder = 2 };
+enum LpClass : int32_t { kLpNone = 0, kLpK = 1, kLpM = 2 };
 // header words
-enum L64Word : int32_t {
+enum LpWord : int32_t {
     kHKind = 0, kHType = 1, kHPrevs = 2, kHSize = 3,
     kHOut = 4,        // arena cell of the table, or -1: registers only
     kHAdj = 5,        // adjoint arena cell of the table, or -1: registers only
     kHPeel = 6,       // peel node's non-founder index (person - F, negative for founders)
     kHKids = 7,       // PARENT children
-    kHStream = 8,     // generic: first word in l64_fwd
+    kHStream = 8,     // generic: first word in lp_fwd
     kHPerson = 9,     // the peel node
+    kHMask = 11,      // legal traits of the parents (bits 0-3 maternal, 4-7 paternal); Founder: of the one left
     kHPeelIsPat = 10, // Founder: 1 when the peel node is the table's paternal axis
     kHMap = 12,       // 4 words: compact cell of (mat, pat) byte 4 mat + pat, 0xFF illegal (Founder: of the trait)
     kHPrev = 16,      // 8 words per consumed table:
     kHKid = 40,       // 3 words: children's non-founder index
     kHTrait = 44,     // 8 words: the peel node's four disease probabilities
-    kHRev = 52,       // 3 words: first word in l64_rev of each consumed table
-    kHGroups = 55     // 3 words: its groups of four contributions
+    kHRev = 52,       // 3 words: first word in lp_rev of each consumed table
+    kHGroups = 55,    // 3 words: its groups of four contributions
+    kHIntoLast = 58   // 1 when the last op consumes the table
 };
 // of a consumed table: arena cell (-1: registers), class, size, adjoint arena
 // cell (-1: registers), 4 words of byte map ((mat, pat), or K: the trait's)
-enum L64Prev : int32_t { kPOff = 0, kPClass = 1, kPSize = 2, kPAdj = 3, kPMap = 4 };
+enum LpPrev : int32_t { kPOff = 0, kPClass = 1, kPSize = 2, kPAdj = 3, kPMap = 4 };
 
 enum OpType : int32_t { kChild = 1, kParent = 2, kPartner = 3, kLast = 4 };
 
@@ -159,16 +161,16 @@ struct PeelProgram {
     // lane_stream_ok false, when an op consumes more than kLaneMaxPrev tables.
     std::vector<uint32_t> lstream;
     bool lane_stream_ok = false;
-    // The FP64 lane program (lane64.hip): the ops in sequential order, each a
-    // header of kL64Header words (L64* offsets), and the generic ops' cells.
-    // l64_ok false when an op is outside what the kernel takes.
-    // l64_rev: per consumed table, cell by cell, each contribution to the cell's
+    // The lane peel's program (lanepeel.hip): the ops in sequential order, each a
+    // header of kLpHeader words (Lp* offsets), and the generic ops' cells.
+    // lp_ok false when an op is outside what the kernel takes.
+    // lp_rev: per consumed table, cell by cell, each contribution to the cell's
     // adjoint: [adjoint cell | kRevLast at the cell's last, info | term << 30,
     // the other consumed tables' cells].
-    std::vector<uint32_t> l64_hdr, l64_fwd, l64_rev;
-    int l64_arena = 0;                  // cells of a lane's stored tables
-    int l64_adj = 0;                    // cells of their adjoints (programs without reuse)
-    bool l64_ok = false;
+    std::vector<uint32_t> lp_hdr, lp_fwd, lp_rev;
+    int lp_arena = 0;                  // cells of a lane's stored tables
+    int lp_adj = 0;                    // cells of their adjoints (programs without reuse)
+    bool lp_ok = false;
     double flops_per_eval = 0.0;        // algorithmic flops per (graph, interval, position)
     double lds_bytes_per_eval = 0.0;    // table reads per evaluation, in elements
 };

@@ -1,4 +1,4 @@
-"""The FP64 peel with one evaluation per lane (scoring from 16384 evaluations,
+"""The peel with one evaluation per lane (scoring from 16384 evaluations,
 the adjoint from 6144) against the workgroup kernels that serve smaller
 launches and explicit requests: scoring terms and accumulators bit for bit,
 the adjoint's value bit for bit up to the final subtraction and its derivatives
@@ -89,3 +89,41 @@ def test_captured_scoring(tmp_path):
                 ctx.mcmc_run(6, 0, 2, 0.5, 11)
             accs.append(ctx.lod_results()[0])
     assert np.array_equal(accs[0], accs[1])
+
+
+# FP32: in the workgroup kernel's arithmetic and exponents (fewer than 32
+# graphs): equal bit for bit; and in the FP32 lane kernel's (whole wavefronts of
+# graphs, and evaluations in a row), whose tables may take their powers of two
+# elsewhere, which moves the rounding of ln L + E ln 2 (|ln L| below 1e3: 1e-12)
+@pytest.mark.parametrize("config,markers,nlod,graphs,kernel", (
+    ("ped30_snp100", 200, 5, 20, native.SL_LOD_WORKGROUP), ("ped150_snp1000", 66, 16, 17, native.SL_LOD_WORKGROUP),
+    ("ped150_snp1000", 300, 5, 64, native.SL_LOD_LANES), ("ped150_snp1000", 300, 5, 63, native.SL_LOD_LANES),
+    ("ped150_snp1000", 150, 5, 129, native.SL_LOD_LANES), ("ped150_snp1000", 300, 5, 33, native.SL_LOD_LANES)))
+def test_fp32_scoring_is_the_other_kernels(tmp_path, config, markers, nlod, graphs, kernel):
+    case, data = synth.make_case(config, str(tmp_path), nlod=nlod, n_markers=markers)
+    assert graphs * (markers - 1) * nlod >= 16384
+    g = _graphs(case, data, graphs)
+    out = []
+    for k in (native.SL_LOD_AUTO, kernel):
+        with native.Context(case, native.SL_FP32_RESCALED, lod_kernel=k) as ctx:
+            assert ctx.lod_kernel_for(graphs) == kernel
+            terms = ctx.lod_terms(g)
+            ctx.lod_accumulate(g)
+            out.append((terms, ctx.lod_results()[0]))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b) if kernel == native.SL_LOD_WORKGROUP else np.abs(a - b).max() < 1e-12
+
+
+def test_allocation_free_sums_are_the_same(tmp_path):
+    """96 graphs: summed in the wavefronts without an array for the terms."""
+    import torch
+    from swiftlink_amd.case import pack_graphs
+    case, data = synth.make_case("ped150_snp1000", str(tmp_path), n_markers=300)
+    g = _graphs(case, data, 96)
+    dev = torch.from_numpy(pack_graphs(case, g).reshape(-1).view(np.int32)).cuda()
+    with native.Context(case, native.SL_FP32_RESCALED) as ctx:
+        ctx.lod_accumulate_packed(dev.data_ptr(), 96)
+        a = ctx.lod_results()[0]
+        ctx.lod_reset()
+        ctx.lod_accumulate_packed_noalloc(dev.data_ptr(), 96)
+        assert np.array_equal(a, ctx.lod_results()[0])
