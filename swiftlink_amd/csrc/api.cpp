@@ -1186,7 +1186,7 @@ static sl::SampArgs samp_args(sl_ctx* c);
 // decoded in the kernel).
 static int setup_flat(sl_ctx* c) {
     const sl::SampProgram& P = c->sprog;
-    c->flat_lds = sl::lsampler_flat_lds_bytes(c->precision, c->cells_cap, P.n_ops, P.n_levels, c->N, c->F);
+    c->flat_lds = sl::lsampler_flat_lds_bytes(c->precision, c->cells_cap, P.n_ops, c->N, c->F);
     if (P.max_prev > sl::kFlatMaxPrev || P.max_child > sl::kFlatMaxKids || P.cell_base.empty() || c->N >= 8000 ||
         c->flat_lds > 160 * 1024 || sl::lsampler_build_lds_bytes(P.n_ops, c->N) > 64 * 1024)
         return SL_OK;

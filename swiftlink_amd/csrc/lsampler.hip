@@ -722,14 +722,20 @@ __global__ void __launch_bounds__(kLsamplerBlockWide) lsampler_kernel(SampArgs A
 // Which products a locus's peel forms depends on its legal masks only, not on
 // the chain: the builder writes them down once per context, one record per
 // (cell, value of the peel node), and a locus step reads each level's records
-// with one coalesced load per lane, issued a level ahead.  A level is then one
-// pass over its records by the whole workgroup, whatever ops they belong to, a
-// product of a handful of LDS entries per lane.  The kernel above decodes every
-// cell of every op again for each chain, op after op within a wavefront: one
-// chain's parity launch at ped150 took 105 us of dependent instructions, now 36;
-// 64 chains' (half of them) 1907 us, now 345; 1000 imputation replicates 164 us a
-// step, now 41; 65535 ELOD replicates in FP64 16.4 ms a step, now 7.4 (its 2550
-// cells per locus leave one workgroup per CU).
+// with one coalesced load per lane.  A level is then one pass over its records
+// by the whole workgroup, whatever ops they belong to, a product of a handful of
+// LDS entries per lane.  The kernel above decodes every cell of every op again
+// for each chain, op after op within a wavefront.
+//
+// A locus step is bound by the latency of its levels (22 forward and 14 reverse
+// at ped150), each behind a barrier, so nothing else may wait in one: the
+// records are kFlatAhead chunks ahead in registers (one chunk ahead, copied
+// down at the level's end, every level waited for its own load: 0.93 us), and
+// a lane's LDS reads come without a branch between them.  Measured: one chain's
+// parity launch at ped150 105 us with the kernel above, 36 one chunk ahead, 23
+// now; 64 chains' 1907, 345, 258 us; an imputation step of 1000 replicates 164,
+// 41, 29 us; 65535 ELOD replicates in FP64 16.4, 7.4, 6.6 ms (their 2550 cells
+// per locus leave one workgroup per CU).
 // Products, sums and scales are those of sampler_op, in its order, so tables,
 // draws and graphs are the same bit for bit.
 
@@ -884,7 +890,6 @@ struct FlatArea {
     T* dist;            // [8NF+2] transmission entries, then 1 and 0
     T* f4;              // [16] the entries by neighbour bits
     uint32_t* maxbits;  // [n_ops]
-    uint32_t* lvl;      // [n_levels+1]
     uint32_t* cnt;      // [kFlatBlock/64]
     uint8_t* pmk;       // [N]
     uint8_t* cmb;       // [2NF] neighbour bits: left | right << 1
@@ -898,8 +903,7 @@ struct FlatArea {
         dist = pre + 4 * (size_t)A.cells_cap;
         f4 = dist + 8 * NF + 4;
         maxbits = reinterpret_cast<uint32_t*>(f4 + 16);
-        lvl = maxbits + A.n_ops;
-        cnt = lvl + A.n_levels + 1;
+        cnt = maxbits + A.n_ops;
         pmk = reinterpret_cast<uint8_t*>(cnt + kFlatBlock / 64);
         cmb = pmk + A.N;
     }
@@ -913,40 +917,40 @@ __device__ __forceinline__ void flat_task(const SampArgs& A, const FlatArea<T>& 
     T x;
     if constexpr (sizeof(T) == 4) x = __uint_as_float(lo.x);
     else x = __longlong_as_double((long long)(((unsigned long long)hi.w << 32) | lo.x));
-    // consumed cells and their scales, all read before the products
-    T pv[kFlatMaxPrev];
+    // everything the product takes, read before it without a branch between
+    // the reads: a branch per operand made each wait for the one before
     const uint32_t cell[3] = {hi.y & 0xFFFFu, hi.y >> 16, hi.z & 0xFFFFu};
     const uint32_t pop[3] = {hi.w & 0xFFFFu, hi.w >> 16, hi.z >> 16};
+    const uint32_t fw[3] = {lo.z, lo.w, hi.x};
+    T pv[3] = {S.tab[cell[0]], S.tab[cell[1]], (T)1};
+    uint32_t mb[3] = {0, 0, 0};
+    if (RESCALE) {
+        mb[0] = S.maxbits[pop[0]];
+        mb[1] = S.maxbits[pop[1]];
+    }
+    T fa[3] = {S.dist[fw[0] & 0xFFFFu] * S.dist[fw[0] >> 16], (T)1, (T)1};
+    if (__any(np > 2u || nf > 2u)) {
+        pv[2] = S.tab[cell[2]];
+        if (RESCALE) mb[2] = S.maxbits[pop[2]];
+        fa[1] = S.dist[fw[1] & 0xFFFFu] * S.dist[fw[1] >> 16];
+        fa[2] = S.dist[fw[2] & 0xFFFFu] * S.dist[fw[2] >> 16];
+    }
     int se = 0;
 #pragma unroll
     for (uint32_t q = 0; q < 3; ++q) {
-        pv[q] = (T)1;
-        if (q < np) {
-            pv[q] = S.tab[cell[q]];
-            if (RESCALE) {
-                const uint32_t mb = S.maxbits[pop[q]];
-                pv[q] *= (T)scale_from_bits(mb);
-                const int ef = (int)((mb >> 23) & 0xFFu);
-                se += ef ? 126 - ef : 0;
-            }
+        if (RESCALE) {
+            pv[q] *= (T)scale_from_bits(mb[q]);
+            const int ef = (int)((mb[q] >> 23) & 0xFFu);
+            se += q < np && ef ? 126 - ef : 0;
         }
-    }
-    T fa[3];
-    const uint32_t fw[3] = {lo.z, lo.w, hi.x};
-#pragma unroll
-    for (uint32_t j = 0; j < 3; ++j) {
-        fa[j] = (T)1;
-        if (2 * j < nf) fa[j] = S.dist[fw[j] & 0xFFFFu] * S.dist[fw[j] >> 16];
+        pv[q] = q < np ? pv[q] : (T)1;
+        fa[q] = 2 * q < nf ? fa[q] : (T)1;
     }
     if (RESCALE && A.impute && (lo.y & 512u) && se != 0) atomicAdd(scale_exp, se);
-    if (x != (T)0) {
-        const bool parent = (lo.y & 256u) != 0u;
-        if (!parent && nf) x *= fa[0];
-#pragma unroll
-        for (uint32_t q = 0; q < 3; ++q)
-            if (q < np) x *= pv[q];
-        if (parent) x *= (fa[0] * fa[1]) * fa[2];
-    }
+    const bool parent = (lo.y & 256u) != 0u;
+    const T fp = (fa[0] * fa[1]) * fa[2];
+    const T y = ((((x * (parent ? (T)1 : fa[0])) * pv[0]) * pv[1]) * pv[2]) * (parent ? fp : (T)1);
+    x = x != (T)0 ? y : (T)0;
     S.pre[t] = x;
     const T s0 = quad_lane<T, 0x00>(x), s1 = quad_lane<T, 0x55>(x), s2 = quad_lane<T, 0xAA>(x), s3 = quad_lane<T, 0xFF>(x);
     const T total = ((s0 + s1) + s2) + s3;
@@ -969,14 +973,23 @@ __device__ __forceinline__ void flat_sample(const SampArgs& A, const FlatArea<T>
     const uint32_t k = hi.z & 255u, op = hi.z >> 8, m = lo.x;
     const uint32_t who[7] = {lo.z & 0xFFFFu, lo.z >> 16, lo.w & 0xFFFFu, lo.w >> 16,
                              hi.x & 0xFFFFu, hi.x >> 16, hi.y & 0xFFFFu};
+    // beyond the cut set the masks are empty: they add nothing
     uint32_t base = lo.y, st = 1;
-#pragma unroll
-    for (uint32_t q = 0; q < 7; ++q) {
-        if (q < k) {
-            const uint32_t mq = (m >> (4 * q)) & 15u;
-            base += rank_in(mq, S.pmk[who[q]]) * st;
-            st *= (uint32_t)__popc(mq);
-        }
+    const auto index = [&](uint32_t q, uint32_t v) {
+        const uint32_t mq = (m >> (4 * q)) & 15u;
+        base += rank_in(mq, v) * st;
+        st *= (uint32_t)__popc(mq);
+    };
+    const uint32_t v0 = S.pmk[who[0]], v1 = S.pmk[who[1]], v2 = S.pmk[who[2]];
+    index(0, v0);
+    index(1, v1);
+    index(2, v2);
+    if (__any(k > 3u)) {
+        const uint32_t v3 = S.pmk[who[3]], v4 = S.pmk[who[4]], v5 = S.pmk[who[5]], v6 = S.pmk[who[6]];
+        index(3, v3);
+        index(4, v4);
+        index(5, v5);
+        index(6, v6);
     }
     const T* pc = S.pre + 4 * (size_t)base;
     T pdv[4] = {pc[0], pc[1], pc[2], pc[3]};
@@ -1032,16 +1045,34 @@ __global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
     }
     const uint32_t base = A.task_base[locus];
     const uint4* task = reinterpret_cast<const uint4*>(A.task + (size_t)4 * base * kTaskWords);
-    const uint32_t* lt = A.level_task + (size_t)locus * (A.n_levels + 1);
-    // the first level's records, in flight during the set-up
-    uint4 lo = make_uint4(0, 0, 0, 0), hi = lo;
-    if ((uint32_t)tid < lt[1]) {
-        lo = task[2 * tid];
-        hi = task[2 * tid + 1];
-    }
+    const cint_p lt = (cint_p)(A.level_task + (size_t)locus * (A.n_levels + 1));
     uint32_t* g = A.graphs + (size_t)chain * M * A.W;
     const uint32_t* colL = locus > 0 && use_left ? g + (size_t)(locus - 1) * A.W : nullptr;
     const uint32_t* colR = locus < M - 1 && use_right ? g + (size_t)(locus + 1) * A.W : nullptr;
+    // one meiosis's neighbour words and parent, used after the set-up and at the end
+    const bool in0 = tid < 2 * NF;
+    const uint32_t word_l = in0 && colL ? colL[tid >> 5] : 0u, word_r = in0 && colR ? colR[tid >> 5] : 0u;
+    const int parent0 = in0 ? (tid & 1 ? A.father : A.mother)[F + (tid >> 1)] : 0;
+    // the forward peel's records: kFlatAhead chunks of a level's in flight
+    uint4 lo[kFlatAhead], hi[kFlatAhead];
+    const int t_end = lt[A.n_levels];
+    int from[kFlatAhead], to[kFlatAhead];  // a chunk's first record, its level's end
+    int pl = 0, pt = 0, pe = lt[1];
+    const auto fetch = [&](uint4& l, uint4& h, int& f, int& e) {
+        const int t = pt + tid < t_end ? pt + tid : t_end - 1;
+        l = task[2 * t];
+        h = task[2 * t + 1];
+        f = pt;
+        e = pe;
+        pt += kFlatBlock;
+        if (pt >= pe) {
+            pt = pe;
+            pl = pl + 1 < A.n_levels ? pl + 1 : pl;
+            pe = lt[pl + 1];
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < kFlatAhead; ++d) fetch(lo[d], hi[d], from[d], to[d]);
     // 1. what depends on the neighbours' bits of one meiosis: four cases
     if (tid < 4) {
         const double thL = locus > 0 ? A.theta[locus - 1] : 1.0, thR = locus < M - 1 ? A.theta[locus] : 1.0;
@@ -1072,7 +1103,6 @@ __global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
         S.dist[8 * NF] = (T)1;
         S.dist[8 * NF + 1] = (T)0;
     }
-    for (int L = tid; L <= A.n_levels; L += kFlatBlock) S.lvl[L] = lt[L];
     for (int o = tid; o < n_ops; o += kFlatBlock) {
         S.uop[o] = philox_uniform(A.seed, rng_chain, sweep, step_id, draw0 + (uint32_t)(n_ops - 1 - o));
         S.maxbits[o] = 0u;
@@ -1080,37 +1110,28 @@ __global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
     __syncthreads();
     for (int b = tid; b < 2 * NF; b += kFlatBlock) {
         uint32_t c = 0;
-        if (colL) c |= (colL[b >> 5] >> (b & 31)) & 1u;
-        if (colR) c |= ((colR[b >> 5] >> (b & 31)) & 1u) << 1;
+        if (colL) c |= ((b == tid ? word_l : colL[b >> 5]) >> (b & 31)) & 1u;
+        if (colR) c |= (((b == tid ? word_r : colR[b >> 5]) >> (b & 31)) & 1u) << 1;
         S.cmb[b] = (uint8_t)c;
 #pragma unroll
         for (int e = 0; e < 4; ++e) S.dist[4 * b + e] = S.f4[4 * c + e];
     }
     __syncthreads();
-    // 2. forward peel, a level per pass
-    for (int L = 0; L < A.n_levels; ++L) {
-        const int t0 = uni((int)S.lvl[L]), t1 = uni((int)S.lvl[L + 1]);
-        uint4 nlo = make_uint4(0, 0, 0, 0), nhi = nlo;
-        if (L + 1 < A.n_levels) {
-            const int tn = t1 + tid;
-            if (tn < uni((int)S.lvl[L + 2])) {
-                nlo = task[2 * tn];
-                nhi = task[2 * tn + 1];
+    // 2. forward peel, a barrier behind each level's last chunk
+    for (int left = A.n_levels; left > 0;) {
+#pragma unroll
+        for (int d = 0; d < kFlatAhead; ++d) {
+            const bool last = from[d] + kFlatBlock >= to[d];
+            if (from[d] + tid < to[d]) flat_task<T, RESCALE>(A, S, from[d] + tid, lo[d], hi[d], &s_scale_exp);
+            fetch(lo[d], hi[d], from[d], to[d]);
+            if (last) {
+                __syncthreads();
+                --left;
             }
         }
-        for (int t = t0 + tid; t < t1; t += kFlatBlock) {
-            if (t != t0 + tid) {
-                lo = task[2 * t];
-                hi = task[2 * t + 1];
-            }
-            flat_task<T, RESCALE>(A, S, t, lo, hi, &s_scale_exp);
-        }
-        lo = nlo;
-        hi = nhi;
-        __syncthreads();
     }
     // likelihood of the locus (locus_sampler2.cc:137-142): the last cell
-    const T like = S.tab[S.lvl[A.n_levels] / 4 - 1];
+    const T like = S.tab[t_end / 4 - 1];
     if (!(like > (T)0)) {
         if (tid == 0) A.status[chain] = -4;
         return;
@@ -1135,33 +1156,35 @@ __global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
             for (int i = tid; i < 2 * NF; i += kFlatBlock)
                 S.um[i] = philox_uniform(A.seed, rng_chain, sweep, step_id, draw0 + (uint32_t)(n_ops + i));
         const int stride = narrow ? 64 : kFlatBlock;
-        int r1 = ((cint_p)A.rlevel_off)[1];
-        uint4 rl = make_uint4(0, 0, 0, 0), rh = rl;
-        if (tid < r1) {
-            rl = rrec[2 * tid];
-            rh = rrec[2 * tid + 1];
-        }
-        int r0 = 0;
-        for (int R = 0; R < A.n_rlevels; ++R) {
-            const int r2 = R + 1 < A.n_rlevels ? ((cint_p)A.rlevel_off)[R + 2] : r1;
-            uint4 nl = make_uint4(0, 0, 0, 0), nh = nl;
-            if (r1 + tid < r2) {
-                nl = rrec[2 * (r1 + tid)];
-                nh = rrec[2 * (r1 + tid) + 1];
+        const cint_p off = (cint_p)A.rlevel_off;
+        int rl = 0, pt = 0, pe = off[1];
+        const auto fetch = [&](uint4& l, uint4& h, int& f, int& e) {
+            const int i = pt + tid < n_ops ? pt + tid : n_ops - 1;
+            l = rrec[2 * i];
+            h = rrec[2 * i + 1];
+            f = pt;
+            e = pe;
+            pt += stride;
+            if (pt >= pe) {
+                pt = pe;
+                rl = rl + 1 < A.n_rlevels ? rl + 1 : rl;
+                pe = uni(off[uni(rl + 1)]);
             }
-            for (int i = r0 + tid; i < r1; i += stride) {
-                if (i != r0 + tid) {
-                    rl = rrec[2 * i];
-                    rh = rrec[2 * i + 1];
+        };
+#pragma unroll
+        for (int d = 0; d < kFlatAhead; ++d) fetch(lo[d], hi[d], from[d], to[d]);
+        for (int left = A.n_rlevels; left > 0;) {
+#pragma unroll
+            for (int d = 0; d < kFlatAhead; ++d) {
+                const bool last = from[d] + stride >= to[d];
+                if (from[d] + tid < to[d]) flat_sample<T>(A, S, chain, locus, lo[d], hi[d]);
+                fetch(lo[d], hi[d], from[d], to[d]);
+                if (last) {
+                    if (narrow) lds_wave_sync();
+                    else __syncthreads();
+                    --left;
                 }
-                flat_sample<T>(A, S, chain, locus, rl, rh);
             }
-            rl = nl;
-            rh = nh;
-            r0 = r1;
-            r1 = r2;
-            if (narrow) lds_wave_sync();
-            else __syncthreads();
         }
     }
     __syncthreads();
@@ -1176,7 +1199,7 @@ __global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
         const int side = b & 1;
         if (in) {
             const int person = F + (b >> 1);
-            pt = S.pmk[side ? A.father[person] : A.mother[person]];
+            pt = S.pmk[b == tid ? parent0 : side ? A.father[person] : A.mother[person]];
             t = S.pmk[person];
         }
         const bool homo = in && (pt == PT_UU || pt == PT_AA);
@@ -1252,12 +1275,12 @@ hipError_t launch_lsampler(const SampArgs& A, int precision, int block, size_t l
 
 size_t lsampler_build_lds_bytes(int n_ops, int N) { return 4 * (2 * (size_t)n_ops + 2) + (size_t)N; }
 
-size_t lsampler_flat_lds_bytes(int precision, int cells_cap, int n_ops, int n_levels, int N, int F) {
+size_t lsampler_flat_lds_bytes(int precision, int cells_cap, int n_ops, int N, int F) {
     const size_t esz = precision == 0 ? 8 : 4;
     const int NF = N - F;
     size_t b = 8 * ((size_t)n_ops + 2 * NF + 4);                              // uop, um, thr
     b += esz * (5 * (size_t)cells_cap + 8 * NF + 4 + 16);                     // tab, pre, dist, f4
-    b += 4 * ((size_t)n_ops + n_levels + 1 + kFlatBlock / 64) + N + 2 * NF;   // maxbits, lvl, cnt, pmk, cmb
+    b += 4 * ((size_t)n_ops + kFlatBlock / 64) + N + 2 * NF;                  // maxbits, cnt, pmk, cmb
     return (b + 15) / 16 * 16;
 }
 

@@ -80,12 +80,15 @@ constexpr int kFlatMaxPrev = 3, kFlatMaxKids = 3;
 // word 5) | 6 cutset size | op << 8
 constexpr int kRevWords = 8;
 constexpr int kFlatBlock = 256;
+// Chunks of records in flight: 4 cover a load from beyond L2 (0.8 us) at 0.3 us a
+// level; 32 registers.
+constexpr int kFlatAhead = 4;
 
 // Fills task, level_task and rrec of every locus.
 hipError_t launch_lsampler_build(const SampArgs& A, int precision, uint32_t* task, uint32_t* level_task, uint32_t* rrec,
                                  size_t lds, hipStream_t s);
 size_t lsampler_build_lds_bytes(int n_ops, int N);
-size_t lsampler_flat_lds_bytes(int precision, int cells_cap, int n_ops, int n_levels, int N, int F);
+size_t lsampler_flat_lds_bytes(int precision, int cells_cap, int n_ops, int N, int F);
 hipError_t configure_lsampler_flat_lds(int precision, size_t lds);
 hipError_t launch_lsampler_flat(const SampArgs& A, int precision, size_t lds, int blocks_x, int blocks_y,
                                 hipStream_t s);

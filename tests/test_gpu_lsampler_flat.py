@@ -61,3 +61,11 @@ def test_wide_levels(tmp_path, people, missing):
             continue
         return _check(case, data)
     raise AssertionError("no family")
+
+
+@pytest.mark.parametrize("people", (4, 6, 9))
+def test_fewer_levels_than_chunks_in_flight(tmp_path, people):
+    """Nuclear families: one to a few levels, fewer than the records' look-ahead."""
+    spec = synth.SynthSpec(people, 2, 0, 6, 0.25, missing=0.3, seed=3200 + people)
+    data = synth.generate(spec, max_drops=2)
+    _check(linkage.load(*synth.write_linkage(data, str(tmp_path))), data)
