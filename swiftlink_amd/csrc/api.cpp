@@ -170,7 +170,7 @@ struct sl_ctx {
     bool samp_ready = false;
     // the flat L-sampler's per-locus records (unset when the tables are outside what it takes)
     bool flat_ok = false;
-    size_t flat_lds = 0;
+    size_t flat_lds[2] = {0, 0};  // of the recomputing and the keeping form
     uint32_t* d_task = nullptr;
     uint32_t* d_task_base = nullptr;
     uint32_t* d_level_task = nullptr;
@@ -1181,14 +1181,15 @@ static sl::SampArgs samp_args(sl_ctx* c);
 
 // The flat L-sampler's records (lsampler.hip).  Leaves flat_ok false where it
 // does not apply: an op consumes more than three tables or has more than three
-// children, an index passes 16 bits, the workgroup does not fit LDS, or the
+// children, an index passes 16 bits, the tables alone do not fit LDS, or the
 // records pass kFlatMaxBytes or the memory there is (the loci's steps are then
 // decoded in the kernel).
 static int setup_flat(sl_ctx* c) {
     const sl::SampProgram& P = c->sprog;
-    c->flat_lds = sl::lsampler_flat_lds_bytes(c->precision, c->cells_cap, P.n_ops, c->N, c->F);
+    for (int keep = 0; keep < 2; ++keep)
+        c->flat_lds[keep] = sl::lsampler_flat_lds_bytes(c->precision, c->cells_cap, P.n_ops, c->N, c->F, keep != 0);
     if (P.max_prev > sl::kFlatMaxPrev || P.max_child > sl::kFlatMaxKids || P.cell_base.empty() || c->N >= 8000 ||
-        c->flat_lds > 160 * 1024 || sl::lsampler_build_lds_bytes(P.n_ops, c->N) > 64 * 1024)
+        c->flat_lds[0] > 160 * 1024 || sl::lsampler_build_lds_bytes(P.n_ops, c->N) > 64 * 1024)
         return SL_OK;
     const size_t words = 4 * (size_t)P.cell_base[c->M] * sl::kTaskWords;
     if (words * sizeof(uint32_t) > kFlatMaxBytes) return SL_OK;
@@ -1210,7 +1211,9 @@ static int setup_flat(sl_ctx* c) {
     sl::SampArgs A = samp_args(c);
     SL_HIP(c, sl::launch_lsampler_build(A, c->precision, c->d_task, c->d_level_task, c->d_rrec,
                                         sl::lsampler_build_lds_bytes(P.n_ops, c->N), c->stream));
-    SL_HIP(c, sl::configure_lsampler_flat_lds(c->precision, c->flat_lds));
+    for (int keep = 0; keep < 2; ++keep)
+        if (c->flat_lds[keep] <= 160 * 1024)
+            SL_HIP(c, sl::configure_lsampler_flat_lds(c->precision, keep != 0, c->flat_lds[keep]));
     SL_HIP(c, hipStreamSynchronize(c->stream));
     c->flat_ok = true;
     return SL_OK;
@@ -1378,6 +1381,20 @@ static int ensure_gtables(sl_ctx* c) {
     return ensure(c, reinterpret_cast<unsigned char**>(&c->d_gtables), &c->gtables_cap, bytes);
 }
 
+// Whether the flat L-sampler keeps every cell's products in LDS for the reverse
+// pass (five entries a cell) or forms the sampled cells' again (one entry a
+// cell, a dependent record load in each reverse level).  Forming them again
+// pays where the kept products leave at most three workgroups to a CU and the
+// launch has more than fit at once: 65535 ELOD replicates in FP64, one
+// workgroup a CU, 6.6 -> 2.3 ms; 32 chains of 600 people, two, 1168 -> 936 us;
+// 3200 loci of 200 people in FP64, three, 108 -> 89 us.  At four it is even or
+// slower (3200 loci, 86 against 88 us; 1600, 71 against 80), and so it is for
+// launches that fit (500 loci of 600 people, 48 against 63 us).
+static bool flat_keeps(const sl_ctx* c, int64_t groups) {
+    const int64_t per_cu = (int64_t)(160 * 1024 / c->flat_lds[1]);
+    return per_cu > 3 || (per_cu > 0 && groups <= kCus * per_cu);
+}
+
 // One L-sampler launch over a grid of gx loci blocks by gy chains; with the
 // tables in global memory, as several launches of at most kGlobalTableSlots
 // workgroups, one slot each.
@@ -1385,7 +1402,8 @@ static int launch_samp(sl_ctx* c, sl::SampArgs A, int block, int gx, int gy) {
     A.block0 = A.chain0 = 0;
     A.gtables = nullptr;
     if (c->flat_ok) {
-        SL_HIP(c, sl::launch_lsampler_flat(A, c->precision, c->flat_lds, gx, gy, c->stream));
+        const bool keep = flat_keeps(c, (int64_t)gx * gy);
+        SL_HIP(c, sl::launch_lsampler_flat(A, c->precision, keep, c->flat_lds[keep], gx, gy, c->stream));
         return SL_OK;
     }
     if (!c->samp_global) {
@@ -1826,7 +1844,7 @@ int sl_mcmc_run(sl_ctx* c, const sl_schedule* sch, sl_mcmc_stats* stats) {
         const int nmei = (int)c->meioses_h.size();
         int rc = SL_OK;
         if (!c->d_sweep) SL_HIP(c, hipMalloc((void**)&c->d_sweep, sizeof(uint32_t)));
-        if ((any_l || any_both) && c->samp_global) rc = ensure_gtables(c);
+        if ((any_l || any_both) && !c->flat_ok) rc = ensure_gtables(c);
         if (!rc && (any_m || any_both) && nmei)
             rc = ensure(c, &c->d_order, &c->order_cap, (size_t)nmei * C);
         if (rc) return rc;

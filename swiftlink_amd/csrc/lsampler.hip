@@ -734,8 +734,14 @@ __global__ void __launch_bounds__(kLsamplerBlockWide) lsampler_kernel(SampArgs A
 // a lane's LDS reads come without a branch between them.  Measured: one chain's
 // parity launch at ped150 105 us with the kernel above, 36 one chunk ahead, 23
 // now; 64 chains' 1907, 345, 258 us; an imputation step of 1000 replicates 164,
-// 41, 29 us; 65535 ELOD replicates in FP64 16.4, 7.4, 6.6 ms (their 2550 cells
-// per locus leave one workgroup per CU).
+// 41, 29 us; 65535 ELOD replicates in FP64 16.4, 7.4, 6.6 ms.
+//
+// Those 2550 cells per locus, with their products kept for the reverse pass,
+// leave one workgroup per CU, four wavefronts to hide LDS and barrier latency
+// behind each other.  The recomputing form (KEEP false) holds the tables alone,
+// a fifth of it, and forms the products of the sampled cells again, a quad of
+// lanes per op: 2.3 ms, and 32 chains of 600 people 936 us a parity launch
+// against 1168.  The rule is flat_keeps' in api.cpp.
 // Products, sums and scales are those of sampler_op, in its order, so tables,
 // draws and graphs are the same bit for bit.
 
@@ -886,21 +892,21 @@ struct FlatArea {
     double* um;         // [2NF] meiosis draws by index
     double* thr;        // [4] draw threshold of a homozygous parent's meiosis by neighbour bits
     T* tab;             // [cells_cap]
-    T* pre;             // [4 cells_cap]
+    T* pre;             // [4 cells_cap], not in the recomputing form
     T* dist;            // [8NF+2] transmission entries, then 1 and 0
     T* f4;              // [16] the entries by neighbour bits
     uint32_t* maxbits;  // [n_ops]
     uint32_t* cnt;      // [kFlatBlock/64]
     uint8_t* pmk;       // [N]
     uint8_t* cmb;       // [2NF] neighbour bits: left | right << 1
-    __device__ FlatArea(unsigned char* p, const SampArgs& A) {
+    __device__ FlatArea(unsigned char* p, const SampArgs& A, bool keep) {
         const int NF = A.N - A.F;
         uop = reinterpret_cast<double*>(p);
         um = uop + A.n_ops;
         thr = um + 2 * NF;
         tab = reinterpret_cast<T*>(thr + 4);
         pre = tab + A.cells_cap;
-        dist = pre + 4 * (size_t)A.cells_cap;
+        dist = pre + (keep ? 4 * (size_t)A.cells_cap : 0);
         f4 = dist + 8 * NF + 4;
         maxbits = reinterpret_cast<uint32_t*>(f4 + 16);
         cnt = maxbits + A.n_ops;
@@ -909,10 +915,9 @@ struct FlatArea {
     }
 };
 
-// One record's product, the sum over its cell's quad, and their stores.
+// One record's product, and the exponent its op's consumed scales add (se).
 template <typename T, bool RESCALE>
-__device__ __forceinline__ void flat_task(const SampArgs& A, const FlatArea<T>& S, int t, const uint4& lo,
-                                          const uint4& hi, int* scale_exp) {
+__device__ __forceinline__ T flat_product(const FlatArea<T>& S, const uint4& lo, const uint4& hi, int& se) {
     const uint32_t np = lo.y & 15u, nf = (lo.y >> 4) & 15u;
     T x;
     if constexpr (sizeof(T) == 4) x = __uint_as_float(lo.x);
@@ -935,7 +940,7 @@ __device__ __forceinline__ void flat_task(const SampArgs& A, const FlatArea<T>& 
         fa[1] = S.dist[fw[1] & 0xFFFFu] * S.dist[fw[1] >> 16];
         fa[2] = S.dist[fw[2] & 0xFFFFu] * S.dist[fw[2] >> 16];
     }
-    int se = 0;
+    se = 0;
 #pragma unroll
     for (uint32_t q = 0; q < 3; ++q) {
         if (RESCALE) {
@@ -946,12 +951,20 @@ __device__ __forceinline__ void flat_task(const SampArgs& A, const FlatArea<T>& 
         pv[q] = q < np ? pv[q] : (T)1;
         fa[q] = 2 * q < nf ? fa[q] : (T)1;
     }
-    if (RESCALE && A.impute && (lo.y & 512u) && se != 0) atomicAdd(scale_exp, se);
     const bool parent = (lo.y & 256u) != 0u;
     const T fp = (fa[0] * fa[1]) * fa[2];
     const T y = ((((x * (parent ? (T)1 : fa[0])) * pv[0]) * pv[1]) * pv[2]) * (parent ? fp : (T)1);
-    x = x != (T)0 ? y : (T)0;
-    S.pre[t] = x;
+    return x != (T)0 ? y : (T)0;
+}
+
+// One record's product, the sum over its cell's quad, and their stores.
+template <typename T, bool RESCALE, bool KEEP>
+__device__ __forceinline__ void flat_task(const SampArgs& A, const FlatArea<T>& S, int t, const uint4& lo,
+                                          const uint4& hi, int* scale_exp) {
+    int se;
+    const T x = flat_product<T, RESCALE>(S, lo, hi, se);
+    if (RESCALE && A.impute && (lo.y & 512u) && se != 0) atomicAdd(scale_exp, se);
+    if (KEEP) S.pre[t] = x;
     const T s0 = quad_lane<T, 0x00>(x), s1 = quad_lane<T, 0x55>(x), s2 = quad_lane<T, 0xAA>(x), s3 = quad_lane<T, 0xFF>(x);
     const T total = ((s0 + s1) + s2) + s3;
     if ((t & 3) == 0) {
@@ -966,10 +979,12 @@ __device__ __forceinline__ void lds_wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Reverse step of one op (SamplerRfunction::sample, sampler_rfunction.cc:159-188)
-template <typename T>
-__device__ __forceinline__ void flat_sample(const SampArgs& A, const FlatArea<T>& S, int chain, int locus, const uint4& lo,
-                                            const uint4& hi) {
+// Reverse step of one op (SamplerRfunction::sample, sampler_rfunction.cc:159-188).
+// The recomputing form has a quad of lanes at each op: each forms the product
+// of one value of the peel node again, from the op's record and the tables.
+template <typename T, bool RESCALE, bool KEEP>
+__device__ __forceinline__ void flat_sample(const SampArgs& A, const FlatArea<T>& S, const uint4* task, int chain,
+                                            int locus, const uint4& lo, const uint4& hi) {
     const uint32_t k = hi.z & 255u, op = hi.z >> 8, m = lo.x;
     const uint32_t who[7] = {lo.z & 0xFFFFu, lo.z >> 16, lo.w & 0xFFFFu, lo.w >> 16,
                              hi.x & 0xFFFFu, hi.x >> 16, hi.y & 0xFFFFu};
@@ -991,8 +1006,20 @@ __device__ __forceinline__ void flat_sample(const SampArgs& A, const FlatArea<T>
         index(5, v5);
         index(6, v6);
     }
-    const T* pc = S.pre + 4 * (size_t)base;
-    T pdv[4] = {pc[0], pc[1], pc[2], pc[3]};
+    T pdv[4];
+    if (KEEP) {
+        const T* pc = S.pre + 4 * (size_t)base;
+        for (int v = 0; v < 4; ++v) pdv[v] = pc[v];
+    } else {
+        const size_t t = 4 * (size_t)base + (threadIdx.x & 3u);
+        const uint4 tl = task[2 * t], th = task[2 * t + 1];
+        int se;
+        const T x = flat_product<T, RESCALE>(S, tl, th, se);
+        pdv[0] = quad_lane<T, 0x00>(x);
+        pdv[1] = quad_lane<T, 0x55>(x);
+        pdv[2] = quad_lane<T, 0xAA>(x);
+        pdv[3] = quad_lane<T, 0xFF>(x);
+    }
     const T tot = pdv[0] + pdv[1] + pdv[2] + pdv[3];
     if (tot != (T)0)
         for (int v = 0; v < 4; ++v) pdv[v] /= tot;
@@ -1007,19 +1034,20 @@ __device__ __forceinline__ void flat_sample(const SampArgs& A, const FlatArea<T>
         if (pdv[v] != (T)0) last = v;
         if (v < 3 && pdv[v] != (T)0 && fabs(u - (double)run) < kEdgeTol<T>) edge = true;
     }
-    S.pmk[hi.y >> 16] = (uint8_t)(chosen >= 0 ? chosen : last);
-    if (A.near_edge && edge) {
+    const bool writer = KEEP || (threadIdx.x & 3u) == 0;
+    if (writer) S.pmk[hi.y >> 16] = (uint8_t)(chosen >= 0 ? chosen : last);
+    if (A.near_edge && edge && writer) {
         atomicAdd(&A.near_edge[chain], 1u);
         atomicOr(&A.near_loci[(size_t)chain * A.near_words + (locus >> 5)], 1u << (locus & 31));
     }
 }
 
-template <typename T, bool RESCALE>
+template <typename T, bool RESCALE, bool KEEP>
 __global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int s_scale_exp;
     const int N = A.N, F = A.F, M = A.M, n_ops = A.n_ops, NF = N - F, tid = threadIdx.x;
-    const FlatArea<T> S(smem, A);
+    const FlatArea<T> S(smem, A, KEEP);
     const int chain = (int)blockIdx.y;
     const uint32_t sweep = A.impute ? A.sweep : sweep_of(A);
     int locus;
@@ -1122,7 +1150,7 @@ __global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
 #pragma unroll
         for (int d = 0; d < kFlatAhead; ++d) {
             const bool last = from[d] + kFlatBlock >= to[d];
-            if (from[d] + tid < to[d]) flat_task<T, RESCALE>(A, S, from[d] + tid, lo[d], hi[d], &s_scale_exp);
+            if (from[d] + tid < to[d]) flat_task<T, RESCALE, KEEP>(A, S, from[d] + tid, lo[d], hi[d], &s_scale_exp);
             fetch(lo[d], hi[d], from[d], to[d]);
             if (last) {
                 __syncthreads();
@@ -1145,9 +1173,10 @@ __global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
     }
     // 3. reverse sampling by reverse levels: the first wavefront while the
     // others draw the meioses' uniforms (by draw index; not all are used), or
-    // the whole workgroup where levels are wide
+    // the whole workgroup where levels are wide or a quad of lanes takes an op
     const uint4* rrec = reinterpret_cast<const uint4*>(A.rrec + (size_t)locus * n_ops * kRevWords);
-    const bool narrow = A.max_rlevel_ops <= 64;
+    const bool narrow = KEEP && A.max_rlevel_ops <= 64;
+    const int item = KEEP ? tid : tid >> 2;
     if (narrow && tid >= 64) {
         for (int i = tid - 64; i < 2 * NF; i += kFlatBlock - 64)
             S.um[i] = philox_uniform(A.seed, rng_chain, sweep, step_id, draw0 + (uint32_t)(n_ops + i));
@@ -1155,11 +1184,11 @@ __global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
         if (!narrow)
             for (int i = tid; i < 2 * NF; i += kFlatBlock)
                 S.um[i] = philox_uniform(A.seed, rng_chain, sweep, step_id, draw0 + (uint32_t)(n_ops + i));
-        const int stride = narrow ? 64 : kFlatBlock;
+        const int stride = narrow || !KEEP ? 64 : kFlatBlock;
         const cint_p off = (cint_p)A.rlevel_off;
         int rl = 0, pt = 0, pe = off[1];
         const auto fetch = [&](uint4& l, uint4& h, int& f, int& e) {
-            const int i = pt + tid < n_ops ? pt + tid : n_ops - 1;
+            const int i = pt + item < n_ops ? pt + item : n_ops - 1;
             l = rrec[2 * i];
             h = rrec[2 * i + 1];
             f = pt;
@@ -1177,7 +1206,8 @@ __global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
 #pragma unroll
             for (int d = 0; d < kFlatAhead; ++d) {
                 const bool last = from[d] + stride >= to[d];
-                if (from[d] + tid < to[d]) flat_sample<T>(A, S, chain, locus, lo[d], hi[d]);
+                if (from[d] + item < to[d])
+                    flat_sample<T, RESCALE, KEEP>(A, S, task, chain, locus, lo[d], hi[d]);
                 fetch(lo[d], hi[d], from[d], to[d]);
                 if (last) {
                     if (narrow) lds_wave_sync();
@@ -1275,20 +1305,27 @@ hipError_t launch_lsampler(const SampArgs& A, int precision, int block, size_t l
 
 size_t lsampler_build_lds_bytes(int n_ops, int N) { return 4 * (2 * (size_t)n_ops + 2) + (size_t)N; }
 
-size_t lsampler_flat_lds_bytes(int precision, int cells_cap, int n_ops, int N, int F) {
+size_t lsampler_flat_lds_bytes(int precision, int cells_cap, int n_ops, int N, int F, bool keep) {
     const size_t esz = precision == 0 ? 8 : 4;
     const int NF = N - F;
-    size_t b = 8 * ((size_t)n_ops + 2 * NF + 4);                              // uop, um, thr
-    b += esz * (5 * (size_t)cells_cap + 8 * NF + 4 + 16);                     // tab, pre, dist, f4
-    b += 4 * ((size_t)n_ops + kFlatBlock / 64) + N + 2 * NF;                  // maxbits, cnt, pmk, cmb
+    size_t b = 8 * ((size_t)n_ops + 2 * NF + 4);                                     // uop, um, thr
+    b += esz * ((keep ? 5 : 1) * (size_t)cells_cap + 8 * NF + 4 + 16);               // tab, pre, dist, f4
+    b += 4 * ((size_t)n_ops + kFlatBlock / 64) + N + 2 * NF;                         // maxbits, cnt, pmk, cmb
     return (b + 15) / 16 * 16;
 }
 
-hipError_t configure_lsampler_flat_lds(int precision, size_t lds) {
+namespace {
+using FlatKernel = void (*)(SampArgs);
+FlatKernel flat_kernel(int precision, bool keep) {
+    if (precision == 0) return keep ? lsampler_flat_kernel<double, false, true> : lsampler_flat_kernel<double, false, false>;
+    return keep ? lsampler_flat_kernel<float, true, true> : lsampler_flat_kernel<float, true, false>;
+}
+}  // namespace
+
+hipError_t configure_lsampler_flat_lds(int precision, bool keep, size_t lds) {
     if (lds <= 64 * 1024) return hipSuccess;
-    const void* k = precision == 0 ? (const void*)lsampler_flat_kernel<double, false>
-                                   : (const void*)lsampler_flat_kernel<float, true>;
-    return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    return hipFuncSetAttribute((const void*)flat_kernel(precision, keep), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)lds);
 }
 
 hipError_t launch_lsampler_build(const SampArgs& A, int precision, uint32_t* task, uint32_t* level_task, uint32_t* rrec,
@@ -1298,11 +1335,9 @@ hipError_t launch_lsampler_build(const SampArgs& A, int precision, uint32_t* tas
     return hipGetLastError();
 }
 
-hipError_t launch_lsampler_flat(const SampArgs& A, int precision, size_t lds, int blocks_x, int blocks_y,
+hipError_t launch_lsampler_flat(const SampArgs& A, int precision, bool keep, size_t lds, int blocks_x, int blocks_y,
                                 hipStream_t s) {
-    const dim3 grid(blocks_x, blocks_y), block(kFlatBlock);
-    if (precision == 0) hipLaunchKernelGGL((lsampler_flat_kernel<double, false>), grid, block, lds, s, A);
-    else hipLaunchKernelGGL((lsampler_flat_kernel<float, true>), grid, block, lds, s, A);
+    hipLaunchKernelGGL(flat_kernel(precision, keep), dim3(blocks_x, blocks_y), dim3(kFlatBlock), lds, s, A);
     return hipGetLastError();
 }
 

@@ -88,9 +88,11 @@ constexpr int kFlatAhead = 4;
 hipError_t launch_lsampler_build(const SampArgs& A, int precision, uint32_t* task, uint32_t* level_task, uint32_t* rrec,
                                  size_t lds, hipStream_t s);
 size_t lsampler_build_lds_bytes(int n_ops, int N);
-size_t lsampler_flat_lds_bytes(int precision, int cells_cap, int n_ops, int N, int F);
-hipError_t configure_lsampler_flat_lds(int precision, size_t lds);
-hipError_t launch_lsampler_flat(const SampArgs& A, int precision, size_t lds, int blocks_x, int blocks_y,
+// keep: the products of every cell stay in LDS for the reverse pass; otherwise
+// the ops' sampled cells form theirs again
+size_t lsampler_flat_lds_bytes(int precision, int cells_cap, int n_ops, int N, int F, bool keep);
+hipError_t configure_lsampler_flat_lds(int precision, bool keep, size_t lds);
+hipError_t launch_lsampler_flat(const SampArgs& A, int precision, bool keep, size_t lds, int blocks_x, int blocks_y,
                                 hipStream_t s);
 
 // L-sampler workgroup: four wavefronts share each peel level; launches of

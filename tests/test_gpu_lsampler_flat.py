@@ -69,3 +69,16 @@ def test_fewer_levels_than_chunks_in_flight(tmp_path, people):
     spec = synth.SynthSpec(people, 2, 0, 6, 0.25, missing=0.3, seed=3200 + people)
     data = synth.generate(spec, max_drops=2)
     _check(linkage.load(*synth.write_linkage(data, str(tmp_path))), data)
+
+
+@pytest.mark.parametrize("people,missing,chains,markers", ((150, 0.97, 300, 4), (300, 0.97, 3, 4)))
+def test_products_formed_again(tmp_path, people, missing, chains, markers):
+    """Sparsely typed families: kept products of one workgroup fill a CU and the
+    launch has more than fit at once (91 KB, 600 workgroups); they do not fit."""
+    for seed in range(3300, 3330):
+        try:
+            case, data = _case(tmp_path, people, missing, seed, loops=1, markers=markers)
+        except RuntimeError:
+            continue
+        return _check(case, data, chains)
+    raise AssertionError("no family")
