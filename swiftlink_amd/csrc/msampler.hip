@@ -24,7 +24,7 @@
 //    exactly the reference's; the likelihood agrees with its products to
 //    rounding.  With a union-find over every edge of every locus a launch for
 //    64 chains at ped150 (half of them on an M-sweep) took 41 us and one for 32
-//    at 600 people and 2000 loci 169 us; now 19 us and 67 us, a third of the
+//    at 600 people and 2000 loci 169 us; now 19 us and 53 us, a third of the
 //    loci being evaluated (next point).
 //  * Of the flips of a step only those whose outcome depends on the descent
 //    graph are evaluated: where the meiosis's parent cannot be heterozygous the
@@ -112,11 +112,14 @@ struct WaveArea {
     uint32_t* acc;    // [2F] fixed to allele A (bit 0), to B (bit 1), touched (bit 2);
                       //      a free component's root: n0 (bits 3-13), n1 (bits 14-24)
     uint32_t* edges;  // [N] x (bits 0-9) | y (bits 10-19) | kEdge, 0 once settled
-    uint16_t* lab;    // [2(N-F)] founder allele of (person, parent)
+    uint16_t* lab;    // [2(N-F)] founder allele of (person, parent); founders first, [2N],
+                      //      for the register-resident likelihood
 };
 
 // an edge word in use (its nodes may both be node 0 only when it is illegal)
 constexpr uint32_t kEdge = 1u << 20;
+// a node's word once its component's root has counted it (above the counts)
+constexpr uint32_t kCounted = 1u << 25;
 
 __device__ __forceinline__ WaveArea wave_area(const MsampArgs& A, unsigned char* base) {
     WaveArea w;
@@ -321,14 +324,16 @@ __device__ double fag_log_likelihood(const MsampArgs& A, const uint2* ptab, cons
 }
 
 // The same likelihood for pedigrees of at most 64*KC people and 32*KC
-// founders, with the wave's
-// working set in registers: lane j holds people j, j+64, ... (genotype, edge,
-// the union-find words of the edge's two nodes) and slots j, j+64, ... of the
-// generation-ordered person table.  A round reads the union-find words of
-// every edge before it writes any hook, so after a compression every find is
-// a single LDS read, and the first round that hooks nothing has read exactly
-// what the consistency check needs.  The per-root terms and their order of
-// summation are those of fag_log_likelihood, so the result is the same.
+// founders: lane j holds people j, j+64, ... (genotype, edge) and slots j,
+// j+64, ... of the generation-ordered person table.  One pass over the edges
+// settles nearly all of them (at 600 people 187 heterozygous people leave 0 to
+// 31 edges, at 150 people 0 or 1), so the rest are packed into a list, which
+// the later rounds and the union-find go through 64 at a time (32 chains of 600
+// people and 2000 loci: 66.5 -> 53 us a launch; before, every round went over
+// every person's edge and the union-find over every founder allele).  Their
+// launches are bound by instruction issue; one chain waits for its slowest job.
+// The per-root terms and their order of summation are those of
+// fag_log_likelihood, so the result is the same.
 // A job's global inputs for the register-resident likelihood, loaded at once
 // at its start: lane j's genotypes and person-table slots j, j+64, ..., and
 // the locus's log allele-frequency terms.
@@ -350,54 +355,43 @@ struct JobInputs {
     }
 };
 
+// Chunks up to which every round goes over all edges, in registers (a launch of
+// one chain of 150 people waits for its slowest job: 7.47 us a step against 7.61
+// through the list).
+constexpr int kRegisterRounds = 3;
+
+// lanes of m below this one
+__device__ __forceinline__ uint32_t count_below(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
 template <int KC>
 __device__ double fag_log_likelihood_r(const MsampArgs& A, const JobInputs<KC>& in, const WaveArea& w, int l) {
-    constexpr int KN = KC;  // node chunks: the chunk class covers 2F too
     const int lane = lane_id();
-    const int F = A.F, NF = A.N - A.F, nodes = 2 * A.F;
-    int g[KC];
-#pragma unroll
-    for (int c = 0; c < KC; ++c) g[c] = in.g[c];
+    const int N = A.N, F = A.F, NF = A.N - A.F, nodes = 2 * A.F;
     const double lmaj = in.lmaj, lmin = in.lmin;
-    // (the nodes' words were reset by fag_job while the job's loads were in
-    // flight)
-    // label slots (reset, founder_allele_graph4.cc:543-569): the source of
-    // each of a slot's two labels, a founder allele (bit 31 set) or the label
-    // slot of the parent it came from
-    uint32_t src0[KC], src1[KC];
-    int sgen[KC], sb[KC];
-#pragma unroll
-    for (int c = 0; c < KC; ++c) {
-        const int k = 64 * c + lane;
-        sgen[c] = -1;
-        sb[c] = 0;
-        src0[c] = src1[c] = 0u;
-        if (k < NF) {
-            const uint2 e = in.pt[c];
-            const int i = (int)(e.x & 0xFFFFu), mo = (int)(e.y & 0xFFFFu), fa = (int)(e.y >> 16);
-            const int b = 2 * (i - F);
-            const uint32_t bm = (w.colw[b >> 5] >> (b & 31)) & 1u;
-            const uint32_t bp = (w.colw[(b + 1) >> 5] >> ((b + 1) & 31)) & 1u;
-            sgen[c] = (int)(e.x >> 16);
-            sb[c] = b;
-            src0[c] = (mo < F ? (0x80000000u | (uint32_t)(2 * mo)) : (uint32_t)(2 * (mo - F))) | bm;
-            src1[c] = (fa < F ? (0x80000000u | (uint32_t)(2 * fa)) : (uint32_t)(2 * (fa - F))) | bp;
-        }
-    }
-    // the slots are in generation order and a parent's generation is below
-    // its child's, so a chunk's slots only read slots of earlier chunks or of
-    // earlier generations of their own chunk: each chunk runs just the
-    // generations it spans (its first and last slot's)
+    // (the nodes' words and the founders' labels were written by fag_job while
+    // the job's loads were in flight)
+    // label slots (reset, founder_allele_graph4.cc:543-569): where each of a
+    // person's two labels comes from.  The slots are in generation order and a
+    // parent's generation is below its child's, so a chunk's slots only read
+    // slots of earlier chunks or of earlier generations of their own chunk:
+    // each chunk runs just the generations it spans (its first and last slot's)
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
         if (64 * c < NF) {
+            const bool in_use = 64 * c + lane < NF;
+            const uint2 e = in.pt[c];
+            const uint32_t i = in_use ? e.x & 0xFFFFu : (uint32_t)F, b = 2u * (i - (uint32_t)F);
+            const uint32_t bits = w.colw[b >> 5] >> (b & 31u);
+            const uint32_t s0 = 2u * (e.y & 0xFFFFu) + (bits & 1u), s1 = 2u * (e.y >> 16) + ((bits >> 1) & 1u);
+            const int gen = in_use ? (int)(e.x >> 16) : -1;
             const int last = NF - 64 * c > 64 ? 63 : NF - 1 - 64 * c;
-            const int g1 = __builtin_amdgcn_readlane(sgen[c], last);
-            for (int gen = __builtin_amdgcn_readlane(sgen[c], 0); gen <= g1; ++gen) {
-                if (sgen[c] == gen) {
-                    const uint32_t l0 = (src0[c] >> 31) ? (src0[c] & 0xFFFFu) : (uint32_t)w.lab[src0[c]];
-                    const uint32_t l1 = (src1[c] >> 31) ? (src1[c] & 0xFFFFu) : (uint32_t)w.lab[src1[c]];
-                    *reinterpret_cast<uint32_t*>(w.lab + sb[c]) = l0 | (l1 << 16);
+            const int g1 = __builtin_amdgcn_readlane(gen, last);
+            for (int g = __builtin_amdgcn_readlane(gen, 0); g <= g1; ++g) {
+                if (gen == g) {
+                    const uint32_t l0 = w.lab[s0], l1 = w.lab[s1];
+                    *reinterpret_cast<uint32_t*>(w.lab + 2 * i) = l0 | (l1 << 16);
                 }
                 wave_sync();
             }
@@ -409,133 +403,166 @@ __device__ double fag_log_likelihood_r(const MsampArgs& A, const JobInputs<KC>& 
     bool bad = false;
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
-        const int i = 64 * c + lane;
         e[c] = 0u;
-        if (g[c]) {
-            uint32_t x = (uint32_t)(2 * i), y = (uint32_t)(2 * i + 1);
-            if (i >= F) {
-                const uint32_t xy = *reinterpret_cast<const uint32_t*>(w.lab + 2 * (i - F));
-                x = xy & 0xFFFFu;
-                y = xy >> 16;
+        if (64 * c < N) {
+            if (in.g[c]) {
+                const uint32_t xy = *reinterpret_cast<const uint32_t*>(w.lab + 2 * (64 * c + lane));
+                const uint32_t x = xy & 0xFFFFu, y = xy >> 16;
+                if (in.g[c] == G_HETERO) {
+                    bad |= x == y;  // an autozygous heterozygote (:77-81)
+                    e[c] = x | (y << 10) | kEdge;
+                }
+                mark_person(w, in.g[c], x, y);
             }
-            if (g[c] == G_HETERO) {
-                bad |= x == y;  // an autozygous heterozygote (:77-81)
-                e[c] = x | (y << 10) | kEdge;
-            }
-            mark_person(w, g[c], x, y);
         }
     }
     if (__ballot(bad)) return -INFINITY;
-    // fixed alleles pass along the edges until nothing changes
-    bool conflict = false, pending;
-    for (;;) {
-        wave_sync();
-        uint32_t fa[KC], fb[KC];
+    // fixed alleles pass along the edges; those with neither side fixed are
+    // packed into w.edges
+    bool conflict = false, changed = false;
+    int listed = 0;
+    const auto list_edges = [&](bool pend, uint32_t word) {
+        const uint64_t m = __ballot(pend);
+        if (m) {
+            if (pend) w.edges[listed + (int)count_below(m)] = word;
+            listed += __popcll(m);
+        }
+    };
+    if constexpr (KC <= kRegisterRounds) {
+        do {
+            wave_sync();
+            changed = false;
+            uint32_t fa[KC], fb[KC];
 #pragma unroll
-        for (int c = 0; c < KC; ++c) {
-            fa[c] = fb[c] = 0u;
-            if (e[c]) {
+            for (int c = 0; c < KC; ++c) {
                 fa[c] = w.acc[e[c] & 0x3FFu] & 3u;
                 fb[c] = w.acc[(e[c] >> 10) & 0x3FFu] & 3u;
             }
-        }
-        bool changed = false;
-        pending = false;
 #pragma unroll
-        for (int c = 0; c < KC; ++c)
-            if (e[c]) {
-                if (pass_fixed(w, e[c], fa[c], fb[c], &changed, &conflict)) e[c] = 0u;
-                else pending = true;
+            for (int c = 0; c < KC; ++c)
+                if (e[c] && pass_fixed(w, e[c], fa[c], fb[c], &changed, &conflict)) e[c] = 0u;
+        } while (__ballot(changed));
+#pragma unroll
+        for (int c = 0; c < KC; ++c) list_edges(e[c] != 0u, e[c]);
+    } else {
+        wave_sync();
+#pragma unroll
+        for (int c0 = 0; c0 < KC; c0 += 4) {
+            if (64 * c0 < N) {
+                uint32_t fa[4] = {0, 0, 0, 0}, fb[4] = {0, 0, 0, 0};
+#pragma unroll
+                for (int c = c0; c < KC && c < c0 + 4; ++c) {
+                    fa[c - c0] = w.acc[e[c] & 0x3FFu] & 3u;
+                    fb[c - c0] = w.acc[(e[c] >> 10) & 0x3FFu] & 3u;
+                }
+#pragma unroll
+                for (int c = c0; c < KC && c < c0 + 4; ++c)
+                    list_edges(e[c] != 0u && !pass_fixed(w, e[c], fa[c - c0], fb[c - c0], &changed, &conflict), e[c]);
             }
-        if (!__ballot(changed)) break;
+        }
     }
-    uint32_t t[KN];
-#pragma unroll
-    for (int n = 0; n < KN; ++n) {
-        const int x = 64 * n + lane;
-        t[n] = 0u;
-        if (x < nodes) t[n] = w.acc[x];
+    // round after round over the list until nothing changes
+    bool pending = listed > 0;
+    while (pending && __ballot(changed)) {
+        wave_sync();
+        changed = pending = false;
+        for (int k0 = 0; k0 < listed; k0 += 64) {
+            const uint32_t x = k0 + lane < listed ? w.edges[k0 + lane] : 0u;
+            bool pend = false;
+            if (x) {
+                const uint32_t a = w.acc[x & 0x3FFu] & 3u, b = w.acc[(x >> 10) & 0x3FFu] & 3u;
+                if (pass_fixed(w, x, a, b, &changed, &conflict)) w.edges[k0 + lane] = 0u;
+                else pend = true;
+            }
+            pending |= __ballot(pend) != 0;
+        }
     }
+    wave_sync();
     int nA = 0, nB = 0;
 #pragma unroll
-    for (int n = 0; n < KN; ++n) {
-        conflict |= (t[n] & 3u) == 3u;
-        nA += __popcll(__ballot((t[n] & 3u) == 1u));
-        nB += __popcll(__ballot((t[n] & 3u) == 2u));
+    for (int n = 0; n < KC; ++n) {
+        if (64 * n < nodes) {
+            const int x = 64 * n + lane;
+            const uint32_t t = x < nodes ? w.acc[x] & 3u : 0u;
+            conflict |= t == 3u;
+            nA += __popcll(__ballot(t == 1u));
+            nB += __popcll(__ballot(t == 2u));
+        }
     }
     if (__ballot(conflict)) return -INFINITY;
     const double ll = (double)nA * lmaj + (double)nB * lmin;
-    if (!__ballot(pending)) return ll;
-    // components no homozygous person reaches: rounds of hooking and
-    // compression until a round hooks nothing (each hooking round removes a
-    // component, so at most 2F rounds hook); the alleles of an edge differ
-    uint32_t ux[KC], uy[KC];
-    // every node's compressed word (root | parity << 16), as the LDS holds it
-    uint32_t r[KN];
-#pragma unroll
-    for (int n = 0; n < KN; ++n) {
-        const int x = 64 * n + lane;
-        r[n] = (uint32_t)x;
-        if (x < nodes) w.uf[x] = (uint32_t)x;
+    if (!pending) return ll;
+    if (listed <= 64) {
+        // one edge left (half of the rest, nearly all of it at 150 people): its
+        // two alleles are a component of their own
+        const uint64_t m = __ballot(lane < listed && w.edges[lane] != 0u);
+        if (__popcll(m) == 1) return ll + free_term(A, l, (1u << 3) | (1u << 14), lmaj, lmin);
     }
-    bool converged = false;
-    for (int round = 0; round <= nodes; ++round) {
-        wave_sync();
-#pragma unroll
-        for (int c = 0; c < KC; ++c) {
-            ux[c] = uy[c] = 0u;
-            if (e[c]) {
-                ux[c] = w.uf[e[c] & 0x3FFu];
-                uy[c] = w.uf[(e[c] >> 10) & 0x3FFu];
-            }
+    // components no homozygous person reaches.  Their nodes are the ends of the
+    // edges left; rounds of hooking larger roots onto smaller ones until a round
+    // hooks nothing (each hooking round removes a component, so at most 2F
+    // rounds hook); the alleles of an edge differ
+    for (int k0 = 0; k0 < listed; k0 += 64) {
+        const uint32_t e0 = k0 + lane < listed ? w.edges[k0 + lane] : 0u;
+        if (e0) {
+            const uint32_t x = e0 & 0x3FFu, y = (e0 >> 10) & 0x3FFu;
+            w.uf[x] = x;
+            w.uf[y] = y;
         }
-        wave_sync();
+    }
+    bool converged = false, illegal = false;
+    for (int round = 0; round <= nodes; ++round) {
         bool hooked = false;
-#pragma unroll
-        for (int c = 0; c < KC; ++c) {
-            const uint32_t rx = ux[c] & 0xFFFFu, ry = uy[c] & 0xFFFFu;
-            if (e[c] && rx != ry) {
-                const uint32_t par = (((ux[c] ^ uy[c]) >> 16) ^ 1u) & 1u;
-                w.uf[rx > ry ? rx : ry] = (rx < ry ? rx : ry) | (par << 16);
-                hooked = true;
+        illegal = false;
+        for (int k0 = 0; k0 < listed; k0 += 64) {
+            wave_sync();
+            const uint32_t e0 = k0 + lane < listed ? w.edges[k0 + lane] : 0u;
+            uint32_t rx = 0, ry = 0, px = 0, py = 0;
+            if (e0) {
+                rx = uf_find(w.uf, e0 & 0x3FFu, &px);
+                ry = uf_find(w.uf, (e0 >> 10) & 0x3FFu, &py);
+            }
+            wave_sync();
+            if (e0) {
+                if (rx != ry) {
+                    w.uf[rx > ry ? rx : ry] = (rx < ry ? rx : ry) | ((px ^ py ^ 1u) << 16);
+                    hooked = true;
+                } else {
+                    illegal |= (px ^ py) != 1u;
+                }
             }
         }
         if (!__ballot(hooked)) {
             converged = true;
             break;
         }
-        wave_sync();
+    }
+    // the last round found every edge's ends in one component: their parities
+    if (!converged || __ballot(illegal)) return -INFINITY;
+    // each end once, counted at its root by parity
+    for (int k0 = 0; k0 < listed; k0 += 64) {
+        const uint32_t e0 = k0 + lane < listed ? w.edges[k0 + lane] : 0u;
+        if (e0) {
 #pragma unroll
-        for (int n = 0; n < KN; ++n) {
-            const int x = 64 * n + lane;
-            if (x < nodes) {
-                uint32_t p;
-                r[n] = uf_find(w.uf, (uint32_t)x, &p) | (p << 16);
+            for (int s = 0; s < 2; ++s) {
+                const uint32_t x = (e0 >> (10 * s)) & 0x3FFu;
+                if (!(atomicOr(&w.acc[x], kCounted) & kCounted)) {
+                    uint32_t p;
+                    const uint32_t r = uf_find(w.uf, x, &p);
+                    atomicAdd(&w.acc[r], p ? (1u << 14) : (1u << 3));
+                }
             }
         }
-        wave_sync();
-#pragma unroll
-        for (int n = 0; n < KN; ++n) {
-            const int x = 64 * n + lane;
-            if (x < nodes) w.uf[x] = r[n];
-        }
     }
-    // the last round's words are compressed: check every edge's parity
-    bool illegal = !converged;
-#pragma unroll
-    for (int c = 0; c < KC; ++c)
-        if (e[c]) illegal |= (((ux[c] ^ uy[c]) >> 16) & 1u) != 1u;
-    if (__ballot(illegal)) return -INFINITY;
-    // touched nodes without a fixed allele, counted at their root by parity
-#pragma unroll
-    for (int n = 0; n < KN; ++n)
-        if ((t[n] & 7u) == 4u) atomicAdd(&w.acc[r[n] & 0xFFFFu], ((r[n] >> 16) & 1u) ? (1u << 14) : (1u << 3));
     wave_sync();
     double free_ll = 0.0;
 #pragma unroll
-    for (int n = 0; n < KN; ++n) {
-        const int x = 64 * n + lane;
-        if ((t[n] & 7u) == 4u && r[n] == (uint32_t)x) free_ll += free_term(A, l, w.acc[x], lmaj, lmin);
+    for (int n = 0; n < KC; ++n) {
+        if (64 * n < nodes) {
+            const int x = 64 * n + lane;
+            const uint32_t a = x < nodes ? w.acc[x] : 0u;
+            if ((a & (kCounted - 8u)) != 0u) free_ll += free_term(A, l, a, lmaj, lmin);
+        }
     }
     return ll + wave_sum(free_ll);
 }
@@ -739,12 +766,11 @@ __device__ void fag_job(const MsampArgs& A, int chain, int q, const uint2* ptab,
     JobInputs<KC> in;
     if constexpr (KC > 0) {
         in.load(A, l);
-        // no node fixed or touched, written while the loads above are in flight
-#pragma unroll
-        for (int n = 0; n < KC; ++n) {
-            const int x = 64 * n + lane;
-            if (x < 2 * A.F) w.acc[x] = 0u;
-        }
+        // no node fixed or touched, and the founders' labels, written while
+        // the loads above are in flight
+        for (int x = lane; x < 2 * A.F; x += 64) w.acc[x] = 0u;
+        for (int f = lane; f < A.F; f += 64)
+            *reinterpret_cast<uint32_t*>(w.lab + 2 * f) = (uint32_t)(2 * f) | ((uint32_t)(2 * f + 1) << 16);
     }
     for (int k = lane; k < A.W; k += 64) {
         uint32_t x = src[k];
@@ -1473,8 +1499,8 @@ int msampler_people_chunks(int N, int F) {
 }
 
 size_t msampler_wave_bytes(int N, int F, int W) {
-    const size_t b = 4 * (size_t)W + 2 * 4 * (size_t)(2 * F) + 4 * (size_t)N +
-                     2 * 2 * (size_t)(N - F);
+    const size_t labelled = msampler_people_chunks(N, F) ? (size_t)N : (size_t)(N - F);
+    const size_t b = 4 * (size_t)W + 2 * 4 * (size_t)(2 * F) + 4 * (size_t)N + 2 * 2 * labelled;
     return (b + 15) / 16 * 16;
 }
 

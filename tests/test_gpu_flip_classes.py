@@ -7,8 +7,8 @@ import numpy as np
 import pytest
 
 from oracle_lib import Oracle
-from swiftlink_amd import native, synth
-from test_gpu_msampler import shuffled_order
+from swiftlink_amd import linkage, native, synth
+from test_gpu_msampler import assert_likelihoods, shuffled_order
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("mode", (native.SL_MSAMPLER_AUTO, native.SL_MSAMPLER_TWO_LAUNCH,
@@ -60,3 +60,56 @@ def test_classes_hold_for_every_flip(tmp_path):
                     seen[1] += 1
                     assert o.fag(f, l) == 0.0
     assert min(seen) > 20
+
+
+def _open_edges_case(tmp_path, people, markers, seed):
+    """A family whose typed people are nearly all heterozygous: founders carry
+    both alleles and homozygous people are untyped, but for one of them at every
+    other locus.  Few founder alleles are fixed, so most edges stay open after a
+    pass over them, or for several."""
+    spec = synth.SynthSpec(people, 4 + people // 100, 1, markers, 0.25, missing=0.0, seed=seed)
+    data = synth.generate(spec, max_drops=2)
+    case = linkage.load(*synth.write_linkage(data, str(tmp_path / "a")))
+    g = synth.true_graph(data, case)
+    order = [data["ped"].ids.index(i) for i in case.ids]  # case person -> data person
+    rng = np.random.default_rng(seed)
+    for l in range(markers):
+        al = np.empty((case.N, 2), int)
+        for p in range(case.N):
+            if p < case.F:
+                al[p] = rng.permutation([1, 2])
+            else:
+                al[p] = [al[case.mother[p], g[l, 2 * p]], al[case.father[p], g[l, 2 * p + 1]]]
+        homo = [p for p in range(case.N) if al[p, 0] == al[p, 1]]
+        keep = homo[len(homo) // 2] if l % 2 and homo else -1
+        for p in range(case.N):
+            data["alleles"][order[p]][:, l] = al[p]
+            data["missing"][order[p], l] = p in homo and p != keep
+    return linkage.load(*synth.write_linkage(data, str(tmp_path / "b"))), g
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("people", (30, 150, 180, 400))
+def test_many_open_edges(tmp_path, people):
+    """More than 64 edges without a fixed allele, below and above the size where
+    the rounds leave the registers; legal graphs and flipped ones."""
+    case, g = _open_edges_case(tmp_path, people, 8, 4100 + people)
+    o = Oracle(case)
+    rng = np.random.default_rng(people)
+    gs = [g]
+    for n in (1, 1, 2, 3):
+        f = g.copy()
+        for l in range(case.M):
+            for b in rng.integers(2 * case.F, 2 * case.N, n):
+                f[l, b] ^= 1
+        gs.append(f)
+    gs = np.stack(gs)
+    lik = []
+    for graphs in (native.SL_MSAMPLER_AUTO, native.SL_MSAMPLER_LDS_GRAPHS):
+        with native.Context(case, native.SL_FP64, msampler_mode=graphs) as ctx:
+            ctx.mcmc_init(gs)
+            lik.append(ctx.mcmc_likelihood())
+    ref = np.array([[o.fag(x, l) for l in range(case.M)] for x in gs])
+    assert np.all(ref[0] > 0.0) and (ref == 0.0).any()
+    assert_likelihoods(lik[0], ref)
+    assert np.array_equal(lik[0], lik[1])
