@@ -30,6 +30,16 @@ thread_local std::string g_create_error;
 // speculative M-steps double the likelihood wavefronts; used while they fit
 // in about two wavefronts per SIMD of the device
 constexpr int64_t kSpecWaves = 8192;
+// Most wavefronts a planned M-step launch starts; more jobs share them.
+constexpr int64_t kPlanWaves = 16384;
+// Jobs of an average step, times the 64-person chunks of one, up to which the
+// forward-backward pass runs beside the next step's jobs, both variants of each:
+// a step then takes one launch, but up to twice the work.  A sweep, beside
+// against two launches: 150 people and 1000 loci, 12 chains 3.44 against 3.75 ms,
+// 16 chains 4.11 against 3.85; 200 people and 2000 loci in FP64, 8 chains 6.3
+// against 7.0, 16 chains 9.2 against 8.6; 30 people and 100 loci, 128 chains 0.62
+// against 0.66, 256 chains 0.94 against 0.77; 600 people, 2 chains even.
+constexpr int64_t kBesideWork = 12288;
 // graphs per adjoint launch (its grid's z extent)
 constexpr int kMaxGridZ = 65535;
 // graphs from which the lane kernel scores a launch by default (half its lanes busy)
@@ -179,6 +189,7 @@ struct sl_ctx {
     std::vector<int32_t> mother_h, father_h;
     // M-sampler
     int m_mode = SL_MSAMPLER_AUTO;
+    size_t m_beside_lds = 0;       // LDS of a pass beside the next step's jobs, 0: not used
     int m_wave_bytes = 0;
     size_t m_lds = 0;       // dynamic LDS of a likelihood-kernel workgroup
     size_t m_spec_lds = 0;  // and of a speculative-kernel workgroup (0: too large, no speculation)
@@ -197,6 +208,11 @@ struct sl_ctx {
     int32_t* d_joblist = nullptr;  // [2(N-F)][M] the loci whose flipped likelihood is computed
     int32_t* d_jobcnt = nullptr;   // [2(N-F)]
     int max_jobs = 0;              // the largest of d_jobcnt
+    double mean_jobs = 0;          // their mean over the sampled meioses
+    uint2* d_mplan = nullptr;      // MsampArgs::plan
+    size_t mplan_cap = 0;
+    uint32_t* d_mplan_total = nullptr;  // [meioses]
+    size_t mplan_total_cap = 0;
     int32_t* d_meioses = nullptr;
     int32_t* d_order = nullptr;
     size_t order_cap = 0;
@@ -545,7 +561,7 @@ int release_all(sl_ctx* c) {
                     c->d_rlevel_ops, c->d_mother, c->d_father, c->d_legal_t, c->d_gprob_d, c->d_gprob_f,
                     c->d_theta, c->d_chains, c->d_status,
                     c->d_gen_off, c->d_ptab, c->d_geno2, c->d_lfreq, c->d_lsum, c->d_meioses, c->d_mcls,
-                    c->d_joblist, c->d_jobcnt, c->d_order,
+                    c->d_joblist, c->d_jobcnt, c->d_mplan, c->d_mplan_total, c->d_order,
                     c->d_fixed_order, c->d_lcur, c->d_lflip, c->d_fbuf, c->d_maps, c->d_mu, c->d_near, c->d_near_loci,
                     c->d_ops, c->d_prevs, c->d_children, c->d_tasks, c->d_tinfo, c->d_idx, c->d_level_base,
                     c->d_sched_off,
@@ -646,7 +662,10 @@ int setup_msampler(sl_ctx* c, const sl_pedigree_desc* ped) {
     // speculative kernel, in the dynamic LDS its job workgroups use)
     c->m_ubuf = M <= sl::kFbUbufLoci;
     if (c->m_ubuf && c->m_spec_lds) c->m_spec_lds = std::max(c->m_spec_lds, sizeof(double) * (size_t)M);
-    SL_HIP(c, sl::configure_msampler_lds(c->m_lds, c->m_spec_lds));
+    c->m_beside_lds = sl::msampler_lds_bytes(A, sl::kFbBlock);
+    if (c->m_ubuf) c->m_beside_lds = std::max(c->m_beside_lds, sizeof(double) * (size_t)M);
+    if (c->m_beside_lds > 160 * 1024 || M > sl::kMaxBesideLoci) c->m_beside_lds = 0;
+    SL_HIP(c, sl::configure_msampler_lds(c->m_lds, c->m_spec_lds, c->m_beside_lds));
     // the founder-allele log terms of every locus, formed once here: ln of
     // each allele's frequency, and the term ln(e^l0 + e^l1) - max(l0, l1) =
     // ln(1 + e^-|l0 - l1|) of a component free to take either assignment,
@@ -691,6 +710,7 @@ int setup_msampler(sl_ctx* c, const sl_pedigree_desc* ped) {
     (void)hipFree(masks);
     SL_HIP(c, e);
     c->max_jobs = *std::max_element(cnt.begin(), cnt.end());
+    for (int32_t b : c->meioses_h) c->mean_jobs += (double)cnt[b] / (double)c->meioses_h.size();
     c->m_ready = true;
     return SL_OK;
 }
@@ -1673,11 +1693,20 @@ static int record_trace(sl_ctx* c, uint32_t s) {
     return SL_OK;
 }
 
+// The buffers of an M-sweep of nm steps.
+static int ensure_msweep(sl_ctx* c, size_t nm) {
+    const size_t C = (size_t)c->n_chains;
+    int rc = ensure(c, &c->d_order, &c->order_cap, nm * C);
+    if (!rc) rc = ensure(c, &c->d_mplan, &c->mplan_cap, nm * C);
+    if (!rc) rc = ensure(c, &c->d_mplan_total, &c->mplan_total_cap, nm);
+    return rc;
+}
+
 // One M-sweep: order, current-column likelihoods, one launch per meiosis step.
 static int run_msweep(sl_ctx* c, uint64_t seed, uint32_t sweep, const int32_t* dev_order, int nm, int check_kind,
                       double lprob, const uint32_t* sweep_dev = nullptr) {
     if (nm == 0) return SL_OK;
-    int rc = ensure(c, &c->d_order, &c->order_cap, (size_t)nm * c->n_chains);
+    int rc = ensure_msweep(c, (size_t)nm);
     if (rc) return rc;
     sl::MsampArgs A = msamp_args(c);
     A.seed = seed;
@@ -1688,7 +1717,8 @@ static int run_msweep(sl_ctx* c, uint64_t seed, uint32_t sweep, const int32_t* d
     A.lprob = lprob;
     SL_HIP(c, sl::launch_morder(A, dev_order, c->stream));
     // one launch per step when the doubled likelihood work still fits the
-    // device in one wave of workgroups (few chains), two launches otherwise
+    // device in one wave of workgroups (few chains); otherwise planned launches,
+    // the pass beside the next step's jobs or one after the other
     const int launch_mode = c->m_mode & 3;
     const bool spec = c->m_spec_lds != 0 &&
                       (launch_mode == SL_MSAMPLER_SPECULATIVE ||
@@ -1716,13 +1746,33 @@ static int run_msweep(sl_ctx* c, uint64_t seed, uint32_t sweep, const int32_t* d
             }
             return SL_OK;
         });
+    A.plan = c->d_mplan;
+    A.plan_total = c->d_mplan_total;
+    SL_HIP(c, sl::launch_mplan(A, c->stream));
+    // as many wavefronts as an average step has jobs, were every chain on an M-sweep
+    const int waves = (int)std::min<double>(std::ceil(c->mean_jobs * c->n_chains), (double)kPlanWaves);
+    const bool beside = c->m_beside_lds != 0 && launch_mode == SL_MSAMPLER_AUTO && A.people_chunks > 0 &&
+                        (int64_t)waves * A.people_chunks <= kBesideWork;
+    if (beside) {
+        A.spec = 1;
+        return timed_span(c, SL_KERNEL_MSAMPLER, nm, [&] {
+            for (int k = 0; k < nm; ++k) {
+                A.fb_step = k;
+                A.step = k + 1;
+                A.plan_waves = k + 1 < nm ? waves : 0;
+                A.draw_uniforms = k + 1 < nm ? 1 : 0;
+                SL_HIP(c, sl::launch_mbeside(A, c->m_beside_lds, c->stream));
+            }
+            return SL_OK;
+        });
+    }
+    A.plan_waves = waves;
     for (int k = 0; k < nm; ++k) {
         A.fb_step = k;
         A.step = k + 1;
         rc = timed_launch(c, SL_KERNEL_MSAMPLER_FB, [&] { return sl::launch_mfb(A, c->stream); });
-        A.n_jobs = k + 1 < nm ? jobs : 0;
         if (!rc && k + 1 < nm)
-            rc = timed_launch(c, SL_KERNEL_MSAMPLER, [&] { return sl::launch_mstep(A, c->m_lds, c->stream); });
+            rc = timed_launch(c, SL_KERNEL_MSAMPLER, [&] { return sl::launch_mplanned(A, c->m_lds, c->stream); });
         if (rc) return rc;
     }
     return SL_OK;
@@ -1846,7 +1896,7 @@ int sl_mcmc_run(sl_ctx* c, const sl_schedule* sch, sl_mcmc_stats* stats) {
         if (!c->d_sweep) SL_HIP(c, hipMalloc((void**)&c->d_sweep, sizeof(uint32_t)));
         if ((any_l || any_both) && !c->flat_ok) rc = ensure_gtables(c);
         if (!rc && (any_m || any_both) && nmei)
-            rc = ensure(c, &c->d_order, &c->order_cap, (size_t)nmei * C);
+            rc = ensure_msweep(c, (size_t)nmei);
         if (rc) return rc;
         SL_HIP(c, hipMemcpyAsync(c->d_sweep, &sch->first_sweep, sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
         SL_HIP(c, hipStreamSynchronize(c->stream));
@@ -2079,7 +2129,7 @@ int sl_batch_run(sl_batch* b, const sl_schedule* sch, sl_mcmc_stats* stats) {
             if (sl::gate_open(s, sch->burnin, sch->period)) st[i].scored += C;
         }
         int rc = ensure(c, &c->d_partial, &c->partial_cap, (size_t)(c->M - 1) * c->npos * partial_rows(c, C));
-        if (!rc && c->m_ready) rc = ensure(c, &c->d_order, &c->order_cap, c->meioses_h.size() * (size_t)C);
+        if (!rc && c->m_ready) rc = ensure_msweep(c, c->meioses_h.size());
         if (!rc && c->samp_ready) rc = ensure_gtables(c);
         if (rc) return rc;
         SL_HIP(c, hipMemcpyAsync(c->d_sweep, &sch->first_sweep, sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));

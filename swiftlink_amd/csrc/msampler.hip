@@ -24,7 +24,7 @@
 //    exactly the reference's; the likelihood agrees with its products to
 //    rounding.  With a union-find over every edge of every locus a launch for
 //    64 chains at ped150 (half of them on an M-sweep) took 41 us and one for 32
-//    at 600 people and 2000 loci 169 us; now 19 us and 53 us, a third of the
+//    at 600 people and 2000 loci 169 us; now 14.5 us and 51.5 us, a third of the
 //    loci being evaluated (next point).
 //  * Of the flips of a step only those whose outcome depends on the descent
 //    graph are evaluated: where the meiosis's parent cannot be heterozygous the
@@ -44,10 +44,13 @@
 // the one bit of m_k there.  With few chains (mspec_kernel) one launch runs
 // step k's forward-backward pass in one workgroup per chain and, in the other
 // workgroups, step k+1's likelihoods for both values of that bit, so a step
-// costs one launch; with many chains (mstep_kernel, mfb_kernel) each step is
-// a likelihood launch then a forward-backward launch.  The start of a sweep
-// also computes the current columns' likelihoods (MeiosisSampler::reset,
-// :17-40).
+// costs one launch.  With more chains the jobs of a step are planned at the
+// sweep's start over all of them (mplan_kernel) and shared by as many wavefronts
+// as an average step has jobs; while those are few, they run beside the
+// forward-backward passes (mbeside_kernel), otherwise each step is a
+// forward-backward launch (mfb_kernel) then a likelihood launch
+// (mplanned_kernel).  The start of a sweep (mstep_kernel) also computes the
+// current columns' likelihoods (MeiosisSampler::reset, :17-40).
 #include <hip/hip_runtime.h>
 #include <cmath>
 #include <cstdint>
@@ -71,6 +74,19 @@ constexpr int kGenoPrefetch = 4;  // genotype chunks of 64 persons loaded ahead
 __device__ __forceinline__ uint32_t sweep_of(const MsampArgs& A) { return A.sweep_dev ? *A.sweep_dev : A.sweep; }
 
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63u); }
+
+// x, and s, as values the compiler knows nothing about: what is formed from
+// them in a loop stays there.  A planned kernel's job loop otherwise kept every
+// address and comparison of a job in registers across jobs (208 registers and
+// 243 spilled scalars at 12 chunks).
+__device__ __forceinline__ int opaque_v(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+__device__ __forceinline__ int opaque_s(int x) {
+    asm volatile("" : "+s"(x));
+    return x;
+}
 
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -173,6 +189,11 @@ __device__ __forceinline__ bool pass_fixed(const WaveArea& w, uint32_t e, uint32
     return true;
 }
 
+// ln(1 + e^-x), out of line: its FP64 constants, kept in registers over a job
+// loop, took half of a planned kernel's; a count difference of kLsumK or more is
+// the only caller
+__device__ __attribute__((noinline)) double log1p_exp_minus(double x) { return log1p(exp(-x)); }
+
 // ln(e^l0 + e^l1) of a component free to take either assignment, from its
 // root's counts
 __device__ __forceinline__ double free_term(const MsampArgs& A, int l, uint32_t a, double lmaj, double lmin) {
@@ -180,7 +201,7 @@ __device__ __forceinline__ double free_term(const MsampArgs& A, int l, uint32_t 
     const double n0 = (double)c0, n1 = (double)c1;
     const double l0 = n0 * lmaj + n1 * lmin;  // root allele A
     const double l1 = n1 * lmaj + n0 * lmin;  // root allele B
-    return fmax(l0, l1) + (kd < (uint32_t)kLsumK ? A.lsum[(size_t)l * kLsumK + kd] : log1p(exp(-fabs(l0 - l1))));
+    return fmax(l0, l1) + (kd < (uint32_t)kLsumK ? A.lsum[(size_t)l * kLsumK + kd] : log1p_exp_minus(fabs(l0 - l1)));
 }
 
 // log of the founder-allele-graph likelihood of the column in w.colw at locus
@@ -343,12 +364,12 @@ struct JobInputs {
     uint2 pt[KC];
     double lmaj, lmin;
     __device__ __forceinline__ void load(const MsampArgs& A, int l) {
-        const int lane = lane_id();
+        const int lane = opaque_v(lane_id()), N = opaque_s(A.N), NF = N - opaque_s(A.F);
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
             const int i = 64 * c + lane;
-            g[c] = i < A.N ? genotype_at(A, l, i) : 0;
-            pt[c] = i < A.N - A.F ? A.ptab[i] : make_uint2(0u, 0u);
+            g[c] = i < N ? genotype_at(A, l, i) : 0;
+            pt[c] = i < NF ? A.ptab[i] : make_uint2(0u, 0u);
         }
         lmaj = A.lfreq[2 * (size_t)l];
         lmin = A.lfreq[2 * (size_t)l + 1];
@@ -367,8 +388,8 @@ __device__ __forceinline__ uint32_t count_below(uint64_t m) {
 
 template <int KC>
 __device__ double fag_log_likelihood_r(const MsampArgs& A, const JobInputs<KC>& in, const WaveArea& w, int l) {
-    const int lane = lane_id();
-    const int N = A.N, F = A.F, NF = A.N - A.F, nodes = 2 * A.F;
+    const int lane = opaque_v(lane_id());
+    const int N = opaque_s(A.N), F = opaque_s(A.F), NF = N - F, nodes = 2 * F;
     const double lmaj = in.lmaj, lmin = in.lmin;
     // (the nodes' words and the founders' labels were written by fag_job while
     // the job's loads were in flight)
@@ -1252,6 +1273,131 @@ __device__ __forceinline__ void run_jobs(const MsampArgs& A, int chain, int bloc
     if (q < A.n_jobs) fag_job<KC>(A, chain, q, ptab, smem + A.ptab_bytes + (size_t)wave * A.wave_bytes);
 }
 
+// The planned jobs of step A.step: the flips to compute over all chains, in the
+// plan's order, shared by n_waves wavefronts.  A grid of one job slot per chain
+// and locus of the longest list sized every step for its worst meiosis, and most
+// wavefronts only found out that they had nothing to do: 64 chains of 150 people
+// 19.1 us a launch, planned 14.5; 32 chains of 600 people, whose jobs fill the
+// device, 53 and 51.5.  With A.spec and k > 0 a job
+// gives both variants (fag_job), the second from the same inputs.
+template <int KC>
+__device__ __forceinline__ void planned_jobs(const MsampArgs& A, uint32_t wave, uint32_t n_waves, const uint2* ptab,
+                                             unsigned char* smem, int area) {
+    const int M = A.M;
+    const uint2* row = A.plan + (size_t)A.step * A.n_chains;
+    const uint32_t total = A.plan_total[A.step];
+    const bool two = A.spec && A.step > 0;
+    for (uint32_t q = wave; q < total; q += n_waves) {
+        const int lane = opaque_v(lane_id()), F = opaque_s(A.F);
+        const WaveArea w = wave_area(A, smem + opaque_s(area));
+        // its chain: the last whose first job is at or below q, 64 candidates a round
+        int chain = 0, n = A.n_chains, flip, stride;
+        uint32_t first;
+        do {
+            stride = (n + 63) >> 6;
+            const int i = lane * stride;
+            const uint2 r = i < n ? row[chain + i] : make_uint2(~0u, 0u);
+            const int at = __popcll(__ballot(r.x <= q)) - 1;
+            first = readlane_u32(r.x, at);
+            flip = (int)readlane_u32(r.y, at);
+            chain += at * stride;
+            n = n - at * stride < stride ? n - at * stride : stride;
+        } while (stride > 1);
+        const int l = A.joblist[(size_t)flip * M + (q - first)];
+        const int status = A.status[chain];
+        int force = two ? (int)A.plan[(size_t)(A.step - 1) * A.n_chains + chain].y : -1;
+        const int pc = two ? A.cls[(size_t)force * M + l] : kFlipSame;
+        if (pc == kFlipIllegal) force = -1;
+        const uint32_t* src = A.graphs + ((size_t)chain * M + l) * A.W;
+        double* const dst = A.lflip + lflip_index(A, A.step, 0, chain, l);
+        double* const dst1 = A.lflip + lflip_index(A, A.step, 1, chain, l);
+        JobInputs<KC> in;
+        if constexpr (KC > 0) {
+            in.load(A, l);
+            for (int f = lane; f < F; f += 64)
+                *reinterpret_cast<uint32_t*>(w.lab + 2 * f) = (uint32_t)(2 * f) | ((uint32_t)(2 * f + 1) << 16);
+        }
+        for (int k = lane; k < A.W; k += 64) {
+            uint32_t x = src[k];
+            if (force >= 0 && (force >> 5) == k) x &= ~(1u << (force & 31));
+            if ((flip >> 5) == k) x ^= 1u << (flip & 31);
+            w.colw[k] = x;
+        }
+        if (status != 0) continue;  // illegal since the plan was made
+        const int variants = two && pc == kFlipCompute ? 2 : 1;
+        for (int v = 0; v < variants; ++v) {
+            if (v && lane == 0) w.colw[force >> 5] ^= 1u << (force & 31);
+            if constexpr (KC > 0)
+                for (int x = lane; x < 2 * F; x += 64) w.acc[x] = 0u;
+            wave_sync();
+            double L;
+            if constexpr (KC > 0) L = fag_log_likelihood_r<KC>(A, in, w, l);
+            else L = fag_log_likelihood(A, ptab, w, l);
+            if (lane == 0) {
+                *(v ? dst1 : dst) = L;
+                if (two && variants == 1) *dst1 = L;
+            }
+            wave_sync();
+        }
+    }
+}
+
+// A workgroup of a planned launch: the first n_job_blocks take the jobs, the
+// others draw step A.step's uniforms.
+template <int KC>
+__device__ __forceinline__ void planned_block(const MsampArgs& A, int block, int n_job_blocks, unsigned char* smem) {
+    const int nw = blockDim.x >> 6, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (block >= n_job_blocks) {
+        const int per_chain = (A.M + (int)blockDim.x - 1) / (int)blockDim.x;
+        const int chain = (block - n_job_blocks) / per_chain;
+        const int i = (block - n_job_blocks) % per_chain * (int)blockDim.x + (int)threadIdx.x;
+        if (i < A.M && is_msweep(A, chain))
+            A.udev[udev_index(A, A.step, chain) + i] =
+                philox_uniform(A.seed, (uint32_t)chain, sweep_of(A), (uint32_t)A.step, (uint32_t)i);
+        return;
+    }
+    uint2* ptab = reinterpret_cast<uint2*>(smem);
+    if constexpr (KC == 0) {
+        for (int k = threadIdx.x; k < A.N - A.F; k += blockDim.x) ptab[k] = A.ptab[k];
+        __syncthreads();
+    }
+    planned_jobs<KC>(A, (uint32_t)(block * nw + wave), (uint32_t)(n_job_blocks * nw), ptab, smem,
+                     A.ptab_bytes + wave * A.wave_bytes);
+}
+
+// The plan of a sweep: for every step the chains' jobs, summed over the chains
+// before.  One workgroup per step.
+constexpr int kPlanBlock = 256;
+__global__ void __launch_bounds__(kPlanBlock) mplan_kernel(MsampArgs A) {
+    __shared__ uint32_t wsum[kPlanBlock / 64];
+    const int k = blockIdx.x, tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+    uint32_t before = 0;
+    for (int c0 = 0; c0 < A.n_chains; c0 += kPlanBlock) {
+        const int c = c0 + tid;
+        int flip = 0;
+        uint32_t cnt = 0;
+        if (c < A.n_chains && A.status[c] == 0 && is_msweep(A, c)) {
+            flip = order_at(A, c, k);
+            cnt = (uint32_t)A.jobcnt[flip];
+        }
+        uint32_t up = cnt;  // inclusive over the wavefront
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t x = (uint32_t)__shfl_up((int)up, d);
+            if (lane >= d) up += x;
+        }
+        if (lane == 63) wsum[wave] = up;
+        __syncthreads();
+        uint32_t mine = before + up - cnt;
+        for (int x = 0; x < kPlanBlock / 64; ++x) {
+            if (x < wave) mine += wsum[x];
+            before += wsum[x];
+        }
+        if (c < A.n_chains) A.plan[(size_t)k * A.n_chains + c] = make_uint2(mine, (uint32_t)flip);
+        __syncthreads();
+    }
+    if (tid == 0) A.plan_total[k] = before;
+}
+
 // What flipping a meiosis does to a legal column, for every meiosis and locus,
 // by genotype elimination (a descent graph only adds constraints, so what no
 // assignment of phased genotypes to the family allows, no column allows).  A
@@ -1369,6 +1515,28 @@ __global__ void __launch_bounds__(kSpecBlock) mspec_kernel(MsampArgs A) {
                                 A.fb_ubuf ? reinterpret_cast<double*>(smem) : nullptr);
     else
         run_jobs<KC>(A, blockIdx.y, blockIdx.x - 1, smem);
+}
+
+// planned jobs only
+template <int KC>
+__global__ void __launch_bounds__(kMsampBlock) mplanned_kernel(MsampArgs A) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    planned_block<KC>(A, blockIdx.x, (A.plan_waves * 64 + kMsampBlock - 1) / kMsampBlock, smem);
+}
+
+// the first workgroups run step fb_step's forward-backward pass, one chain each,
+// in mfb_kernel's shape (the same scans, the same rounding), the others the
+// planned jobs of step fb_step + 1
+template <int SM, int KC, typename T>
+__global__ void __launch_bounds__(kFbBlock) mbeside_kernel(MsampArgs A) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ MatT<T> wtot[kFbBlock / 64];
+    __shared__ uint32_t wcnt[kFbBlock / 64], wmap[kFbBlock / 64];
+    const int b = blockIdx.x;
+    if (b < A.n_chains)
+        forward_backward<SM, T>(A, b, A.fb_step, wtot, wcnt, wmap, A.fb_ubuf ? reinterpret_cast<double*>(smem) : nullptr);
+    else
+        planned_block<KC>(A, b - A.n_chains, (A.plan_waves * 64 + kFbBlock - 1) / kFbBlock, smem);
 }
 
 // this sweep's meiosis order: the given order, or a Fisher-Yates shuffle of the
@@ -1534,13 +1702,45 @@ hipError_t set_lds_spec(size_t spec) {
     return e;
 }
 
+template <int KC, typename T>
+hipError_t set_lds_beside(size_t beside) {
+    hipError_t e = set_lds((const void*)mbeside_kernel<1, KC, T>, beside);
+    if (e == hipSuccess) e = set_lds((const void*)mbeside_kernel<2, KC, T>, beside);
+    if (e == hipSuccess) e = set_lds((const void*)mbeside_kernel<4, KC, T>, beside);
+    return e;
+}
+
 template <int KC>
-hipError_t set_lds_kc(size_t job, size_t spec) {
+hipError_t set_lds_kc(size_t job, size_t spec, size_t beside) {
     hipError_t e = set_lds((const void*)mstep_kernel<KC>, job);
+    if (e == hipSuccess) e = set_lds((const void*)mplanned_kernel<KC>, job);
+    if (e == hipSuccess && beside) e = set_lds_beside<KC, double>(beside);
+    if (e == hipSuccess && beside) e = set_lds_beside<KC, float>(beside);
     if (spec == 0) return e;
     if (e == hipSuccess) e = set_lds_spec<KC, double>(spec);
     if (e == hipSuccess) e = set_lds_spec<KC, float>(spec);
     return e;
+}
+
+// workgroups of a planned launch: jobs, then the uniforms
+int planned_blocks(const MsampArgs& A, int block) {
+    return (A.plan_waves * 64 + block - 1) / block +
+           (A.fb_ubuf && A.draw_uniforms ? A.n_chains * ((A.M + block - 1) / block) : 0);
+}
+
+template <int KC, typename T>
+void launch_mbeside_kc(const MsampArgs& A, size_t lds, hipStream_t s) {
+    const int seg = (A.M + kFbBlock - 1) / kFbBlock;
+    const dim3 grid(A.n_chains + planned_blocks(A, kFbBlock)), block(kFbBlock);
+    if (seg <= 1) hipLaunchKernelGGL((mbeside_kernel<1, KC, T>), grid, block, lds, s, A);
+    else if (seg <= 2) hipLaunchKernelGGL((mbeside_kernel<2, KC, T>), grid, block, lds, s, A);
+    else hipLaunchKernelGGL((mbeside_kernel<4, KC, T>), grid, block, lds, s, A);
+}
+
+template <int KC>
+void launch_mbeside_kc(const MsampArgs& A, size_t lds, hipStream_t s) {
+    if (A.fp32) launch_mbeside_kc<KC, float>(A, lds, s);
+    else launch_mbeside_kc<KC, double>(A, lds, s);
 }
 
 template <int KC, typename T>
@@ -1574,15 +1774,15 @@ void launch_mfb_t(const MsampArgs& A, hipStream_t s) {
 
 }  // namespace
 
-hipError_t configure_msampler_lds(size_t job_lds, size_t spec_lds) {
-    hipError_t e = set_lds_kc<0>(job_lds, spec_lds);
-    if (e == hipSuccess) e = set_lds_kc<2>(job_lds, spec_lds);
-    if (e == hipSuccess) e = set_lds_kc<3>(job_lds, spec_lds);
-    if (e == hipSuccess) e = set_lds_kc<4>(job_lds, spec_lds);
-    if (e == hipSuccess) e = set_lds_kc<6>(job_lds, spec_lds);
-    if (e == hipSuccess) e = set_lds_kc<8>(job_lds, spec_lds);
-    if (e == hipSuccess) e = set_lds_kc<12>(job_lds, spec_lds);
-    if (e == hipSuccess) e = set_lds_kc<16>(job_lds, spec_lds);
+hipError_t configure_msampler_lds(size_t job_lds, size_t spec_lds, size_t beside_lds) {
+    hipError_t e = set_lds_kc<0>(job_lds, spec_lds, beside_lds);
+    if (e == hipSuccess) e = set_lds_kc<2>(job_lds, spec_lds, beside_lds);
+    if (e == hipSuccess) e = set_lds_kc<3>(job_lds, spec_lds, beside_lds);
+    if (e == hipSuccess) e = set_lds_kc<4>(job_lds, spec_lds, beside_lds);
+    if (e == hipSuccess) e = set_lds_kc<6>(job_lds, spec_lds, beside_lds);
+    if (e == hipSuccess) e = set_lds_kc<8>(job_lds, spec_lds, beside_lds);
+    if (e == hipSuccess) e = set_lds_kc<12>(job_lds, spec_lds, beside_lds);
+    if (e == hipSuccess) e = set_lds_kc<16>(job_lds, spec_lds, beside_lds);
     return e;
 }
 
@@ -1611,6 +1811,41 @@ hipError_t launch_mstep(const MsampArgs& A, size_t lds, hipStream_t s) {
         case 12: hipLaunchKernelGGL(mstep_kernel<12>, grid, dim3(kMsampBlock), lds, s, A); break;
         case 16: hipLaunchKernelGGL(mstep_kernel<16>, grid, dim3(kMsampBlock), lds, s, A); break;
         default: hipLaunchKernelGGL(mstep_kernel<0>, grid, dim3(kMsampBlock), lds, s, A); break;
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_mplan(const MsampArgs& A, hipStream_t s) {
+    hipLaunchKernelGGL(mplan_kernel, dim3(A.n_meioses), dim3(kPlanBlock), 0, s, A);
+    return hipGetLastError();
+}
+
+hipError_t launch_mplanned(const MsampArgs& A, size_t lds, hipStream_t s) {
+    const dim3 grid(planned_blocks(A, kMsampBlock)), block(kMsampBlock);
+    if (grid.x == 0) return hipSuccess;
+    switch (A.people_chunks) {
+        case 2: hipLaunchKernelGGL(mplanned_kernel<2>, grid, block, lds, s, A); break;
+        case 3: hipLaunchKernelGGL(mplanned_kernel<3>, grid, block, lds, s, A); break;
+        case 4: hipLaunchKernelGGL(mplanned_kernel<4>, grid, block, lds, s, A); break;
+        case 6: hipLaunchKernelGGL(mplanned_kernel<6>, grid, block, lds, s, A); break;
+        case 8: hipLaunchKernelGGL(mplanned_kernel<8>, grid, block, lds, s, A); break;
+        case 12: hipLaunchKernelGGL(mplanned_kernel<12>, grid, block, lds, s, A); break;
+        case 16: hipLaunchKernelGGL(mplanned_kernel<16>, grid, block, lds, s, A); break;
+        default: hipLaunchKernelGGL(mplanned_kernel<0>, grid, block, lds, s, A); break;
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_mbeside(const MsampArgs& A, size_t lds, hipStream_t s) {
+    switch (A.people_chunks) {
+        case 2: launch_mbeside_kc<2>(A, lds, s); break;
+        case 3: launch_mbeside_kc<3>(A, lds, s); break;
+        case 4: launch_mbeside_kc<4>(A, lds, s); break;
+        case 6: launch_mbeside_kc<6>(A, lds, s); break;
+        case 8: launch_mbeside_kc<8>(A, lds, s); break;
+        case 12: launch_mbeside_kc<12>(A, lds, s); break;
+        case 16: launch_mbeside_kc<16>(A, lds, s); break;
+        default: launch_mbeside_kc<0>(A, lds, s); break;
     }
     return hipGetLastError();
 }

@@ -13,7 +13,9 @@ namespace sl {
 constexpr int kMaxFagNodes = 1022;  // 2F
 constexpr int kMsampBlock = 256;    // threads per workgroup of the likelihood kernel (its launch bound)
 constexpr int kSpecBlock = 512;     // threads per workgroup of the speculative kernel
-constexpr int kFbBlock = 1024;      // threads per workgroup of the forward-backward kernel
+constexpr int kFbBlock = 1024;      // threads per workgroup of the forward-backward kernel, and of the planned
+                                    // kernel that runs it beside the next step's jobs
+constexpr int kMaxBesideLoci = 4 * kFbBlock;  // loci that kernel takes: segments of 1, 2 or 4 per thread
 
 struct MsampArgs {
     int N, F, M, W;
@@ -64,6 +66,10 @@ struct MsampArgs {
     int fp32;                     // 1: the forward-backward pass in FP32 (FP32-rescaled contexts)
     int fb_ubuf;                  // 1: forward-backward launches carry M doubles of dynamic LDS for the
                                   //    step's uniforms (mspec: within its dynamic LDS)
+    uint2* plan;                  // [n_meioses][chains] planned launches: (jobs of the step's launch in the
+                                  // chains before, the chain's meiosis); no jobs where it makes no M-sweep
+    uint32_t* plan_total;         // [n_meioses] the step's jobs over all chains
+    int plan_waves;               // wavefronts that share them
     int draw_uniforms;            // 1: this job launch also draws step `step`'s uniforms into udev
     double* udev;                 // [2 step parities][chains][M] uniforms of a step by draw index
 };
@@ -87,11 +93,18 @@ int msampler_people_chunks(int N, int F);  // register chunks for N people, F fo
 size_t msampler_wave_bytes(int N, int F, int W);
 size_t msampler_ptab_bytes(int N, int F);
 size_t msampler_lds_bytes(const MsampArgs& A, int block);
-hipError_t configure_msampler_lds(size_t job_lds, size_t spec_lds);  // spec_lds 0: no speculative launches
+// spec_lds, beside_lds 0: none of these launches
+hipError_t configure_msampler_lds(size_t job_lds, size_t spec_lds, size_t beside_lds);
 hipError_t launch_morder(const MsampArgs& A, const int32_t* fixed_order, hipStream_t s);
 hipError_t launch_mstep(const MsampArgs& A, size_t lds, hipStream_t s);
 hipError_t launch_mfb(const MsampArgs& A, hipStream_t s);
 hipError_t launch_mspec(const MsampArgs& A, size_t lds, hipStream_t s);
+// fills plan and plan_total from the sweep's orders
+hipError_t launch_mplan(const MsampArgs& A, hipStream_t s);
+// step A.step's planned jobs and uniforms
+hipError_t launch_mplanned(const MsampArgs& A, size_t lds, hipStream_t s);
+// step A.fb_step's forward-backward pass beside step A.step's planned jobs (none when A.plan_waves is 0)
+hipError_t launch_mbeside(const MsampArgs& A, size_t lds, hipStream_t s);
 // per chain: the CODA trace likelihood of its graph into out[chain], from
 // lcur holding the current columns' founder-allele log-likelihoods
 hipError_t launch_trace(const MsampArgs& A, const double* log_theta, const double* log_anti, double trans, double* out,

@@ -113,3 +113,27 @@ def test_many_open_edges(tmp_path, people):
     assert np.all(ref[0] > 0.0) and (ref == 0.0).any()
     assert_likelihoods(lik[0], ref)
     assert np.array_equal(lik[0], lik[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", (native.SL_MSAMPLER_AUTO, native.SL_MSAMPLER_TWO_LAUNCH))
+@pytest.mark.parametrize("chains,markers,missing", ((64, 65, 0.1), (70, 65, 0.7), (1100, 5, 0.3), (4200, 3, 0.1)))
+def test_planned_steps(tmp_path, chains, markers, missing, mode):
+    """Enough chains for planned launches, around the 64 candidates of a job's
+    search for its chain (one, two and three rounds), the forward-backward pass
+    beside the next step's jobs or before them."""
+    case, data = synth.make_case("ped30_snp100", str(tmp_path), n_markers=markers, missing=missing)
+    o = Oracle(case)
+    g0 = synth.true_graph(data, case)
+    with native.Context(case, native.SL_FP64, msampler_mode=mode) as ctx:
+        ctx.mcmc_init(np.repeat(g0[None], chains, axis=0))
+        ctx.msweep(41, 0)
+        ctx.msweep(41, 1)
+        out = ctx.mcmc_graphs()
+        assert np.all(ctx.mcmc_status() == 0)
+        near = ctx.mcmc_near_edge()
+    for c in sorted({0, 1, 63, 64 % chains, 65 % chains, chains // 2, chains - 2, chains - 1}):
+        assert near[c] == 0
+        g = o.msweep(g0, shuffled_order(o, 41, c, 0), 41, c, 0)
+        g = o.msweep(g, shuffled_order(o, 41, c, 1), 41, c, 1)
+        assert np.array_equal(out[c], g), c
