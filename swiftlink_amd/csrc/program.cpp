@@ -97,7 +97,7 @@ int place(const std::vector<int>& ids, const std::vector<int>& size, const std::
     return top;
 }
 
-// The FP64 lane program (program.h) of the compiled ops in the order `post`.
+// The lane-peel program (program.h) of the compiled ops in the order `post`.
 // tape: every table keeps a cell range of its own (the adjoint reads them all)
 // and the generic ops get their reverse lists.
 std::string build_lanepeel(const PedigreeView& ped, const PeelView& pv, const std::vector<std::vector<int>>& cuts,

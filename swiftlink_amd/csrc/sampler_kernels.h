@@ -80,7 +80,7 @@ constexpr int kFlatMaxPrev = 3, kFlatMaxKids = 3;
 // word 5) | 6 cutset size | op << 8
 constexpr int kRevWords = 8;
 constexpr int kFlatBlock = 256;
-// Chunks of records in flight: 4 cover a load from beyond L2 (0.8 us) at 0.3 us a
+// Chunks of records in flight: 4 cover a load from beyond L2 (0.8 us) at 0.5 us a
 // level; 32 registers.
 constexpr int kFlatAhead = 4;
 
