@@ -369,8 +369,8 @@ bool lane_mode(const sl_ctx* c, int G) {
 // (FP64, us, workgroup against lanes: 118/121 at 15840 and 30 people, 413/276 at
 // 19980 and 150, 1057/526 at 39980 and 200).
 int lanepeel_form(const sl_ctx* c, int G) {
-    if (!c->prog.lp_ok || c->lod_kernel != SL_LOD_AUTO || sl::lanepeel_lds_bytes(c->W) > 64 * 1024 ||
-        (int64_t)G * (c->M - 1) * c->npos < kLpMinEvals)
+    if ((int64_t)G * (c->M - 1) * c->npos < kLpMinEvals || !c->prog.lp_ok || c->lod_kernel != SL_LOD_AUTO ||
+        sl::lanepeel_lds_bytes(c->W) > 64 * 1024)
         return -1;
     const size_t slot = sl::lanepeel_slot_bytes(c->prog.lp_arena, 0, c->precision == SL_FP64);
     if (c->lp_bytes < std::max(slot, std::min(kLpScoreBytes, kLpLeastWaves * slot))) return -1;  // no memory for them
