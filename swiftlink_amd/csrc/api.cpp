@@ -207,8 +207,8 @@ struct sl_ctx {
     uint8_t* d_mcls = nullptr;     // [2(N-F)][M] classes of a meiosis's flip by locus
     int32_t* d_joblist = nullptr;  // [2(N-F)][M] the loci whose flipped likelihood is computed
     int32_t* d_jobcnt = nullptr;   // [2(N-F)]
-    int max_jobs = 0;              // the largest of d_jobcnt
-    double mean_jobs = 0;          // their mean over the sampled meioses
+    std::vector<int32_t> jobcnt_h;
+    int max_jobs = 0;              // the largest of them
     uint2* d_mplan = nullptr;      // MsampArgs::plan
     size_t mplan_cap = 0;
     uint32_t* d_mplan_total = nullptr;  // [meioses]
@@ -702,7 +702,8 @@ int setup_msampler(sl_ctx* c, const sl_pedigree_desc* ped) {
     K.ptab = c->d_ptab;
     K.geno2 = c->d_geno2;
     K.GW = GW;
-    std::vector<int32_t> cnt(nb);
+    std::vector<int32_t>& cnt = c->jobcnt_h;
+    cnt.resize(nb);
     hipError_t e = sl::launch_mclass(K, masks, c->d_mcls, c->d_joblist, c->d_jobcnt, c->stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(cnt.data(), c->d_jobcnt, nb * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream);
@@ -710,7 +711,6 @@ int setup_msampler(sl_ctx* c, const sl_pedigree_desc* ped) {
     (void)hipFree(masks);
     SL_HIP(c, e);
     c->max_jobs = *std::max_element(cnt.begin(), cnt.end());
-    for (int32_t b : c->meioses_h) c->mean_jobs += (double)cnt[b] / (double)c->meioses_h.size();
     c->m_ready = true;
     return SL_OK;
 }
@@ -1702,9 +1702,10 @@ static int ensure_msweep(sl_ctx* c, size_t nm) {
     return rc;
 }
 
-// One M-sweep: order, current-column likelihoods, one launch per meiosis step.
-static int run_msweep(sl_ctx* c, uint64_t seed, uint32_t sweep, const int32_t* dev_order, int nm, int check_kind,
-                      double lprob, const uint32_t* sweep_dev = nullptr) {
+// One M-sweep over the meioses `order` (in this order where dev_order holds them
+// too, else shuffled): current-column likelihoods, one launch per meiosis step.
+static int run_msweep(sl_ctx* c, uint64_t seed, uint32_t sweep, const int32_t* dev_order, const int32_t* order, int nm,
+                      int check_kind, double lprob, const uint32_t* sweep_dev = nullptr) {
     if (nm == 0) return SL_OK;
     int rc = ensure_msweep(c, (size_t)nm);
     if (rc) return rc;
@@ -1749,8 +1750,11 @@ static int run_msweep(sl_ctx* c, uint64_t seed, uint32_t sweep, const int32_t* d
     A.plan = c->d_mplan;
     A.plan_total = c->d_mplan_total;
     SL_HIP(c, sl::launch_mplan(A, c->stream));
-    // as many wavefronts as an average step has jobs, were every chain on an M-sweep
-    const int waves = (int)std::min<double>(std::ceil(c->mean_jobs * c->n_chains), (double)kPlanWaves);
+    // as many wavefronts as an average step of this sweep's meioses has jobs,
+    // were every chain on an M-sweep: none only where no step has one
+    double jobs_sum = 0.0;
+    for (int k = 0; k < nm; ++k) jobs_sum += (double)c->jobcnt_h[order[k]];
+    const int waves = (int)std::min<double>(std::ceil(jobs_sum * c->n_chains / nm), (double)kPlanWaves);
     const bool beside = c->m_beside_lds != 0 && launch_mode == SL_MSAMPLER_AUTO && A.people_chunks > 0 &&
                         (int64_t)waves * A.people_chunks <= kBesideWork;
     if (beside) {
@@ -1802,7 +1806,8 @@ int sl_msweep(sl_ctx* c, uint64_t seed, uint32_t sweep, const int32_t* order, in
             SL_HIP(c, hipStreamSynchronize(c->stream));
         }
     }
-    return run_msweep(c, seed, sweep, order ? c->d_fixed_order : nullptr, nm, 0, 0.0);
+    return run_msweep(c, seed, sweep, order ? c->d_fixed_order : nullptr, order ? order : c->meioses_h.data(), nm, 0,
+                      0.0);
 }
 
 }  // extern "C"
@@ -1911,7 +1916,7 @@ int sl_mcmc_run(sl_ctx* c, const sl_schedule* sch, sl_mcmc_stats* stats) {
             return r ? r : advance();
         });
         if (!rc && (any_m || any_both)) rc = capture_sweep(c, &g_ma, [&] {
-            const int r = run_msweep(c, sch->seed, 0u, nullptr, nmei, 1, sch->lprob, c->d_sweep);
+            const int r = run_msweep(c, sch->seed, 0u, nullptr, c->meioses_h.data(), nmei, 1, sch->lprob, c->d_sweep);
             return r ? r : advance();
         });
         if (rc) return rc;
@@ -1927,10 +1932,11 @@ int sl_mcmc_run(sl_ctx* c, const sl_schedule* sch, sl_mcmc_stats* stats) {
         } else if (C == 1) {
             // one chain: launch only the sweep it takes
             rc = nl ? run_lsweep(c, sch->seed, s, p0, 0, 0.0)
-                    : run_msweep(c, sch->seed, s, nullptr, (int)c->meioses_h.size(), 0, 0.0);
+                    : run_msweep(c, sch->seed, s, nullptr, c->meioses_h.data(), (int)c->meioses_h.size(), 0, 0.0);
         } else {
             if (nl) rc = run_lsweep(c, sch->seed, s, 0, 1, sch->lprob);
-            if (!rc && nm) rc = run_msweep(c, sch->seed, s, nullptr, (int)c->meioses_h.size(), 1, sch->lprob);
+            if (!rc && nm) rc = run_msweep(c, sch->seed, s, nullptr, c->meioses_h.data(), (int)c->meioses_h.size(), 1,
+                                       sch->lprob);
         }
         if (rc) return rc;
         st.l_sweeps += nl;
@@ -2094,7 +2100,7 @@ int enqueue_sweep(sl_ctx* c, const sl_schedule* sch) {
     int rc = SL_OK;
     if (c->samp_ready) rc = run_lsweep(c, sch->seed, 0u, 0, 1, sch->lprob, c->d_sweep);
     if (!rc && c->m_ready)
-        rc = run_msweep(c, sch->seed, 0u, nullptr, (int)c->meioses_h.size(), 1, sch->lprob, c->d_sweep);
+        rc = run_msweep(c, sch->seed, 0u, nullptr, c->meioses_h.data(), (int)c->meioses_h.size(), 1, sch->lprob, c->d_sweep);
     if (!rc) rc = lod_run(c, c->d_chains, c->n_chains, nullptr, c->d_sweep, sch->burnin, sch->period);
     if (!rc) SL_HIP(c, sl::launch_advance(c->d_sweep, c->stream));
     return rc;

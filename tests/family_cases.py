@@ -1,0 +1,39 @@
+"""Cases from a pedigree given as parent arrays, without going through files."""
+import numpy as np
+
+from swiftlink_amd import linkage, peelseq
+from swiftlink_amd.case import Case
+
+
+def family_case(mother, father, founders, markers, missing, seed, minor=None, spacing=0.5, nlod=2, untyped=(),
+                tries=16):
+    """(Case, descent graph [M][2N]) of genotypes dropped from `seed` down the
+    pedigree (internal order, founders first), a share `missing` of them and all
+    of the people `untyped` left out."""
+    mother, father = np.asarray(mother, np.int32), np.asarray(father, np.int32)
+    N, F, M = len(mother), founders, markers
+    rng = np.random.default_rng(seed)
+    maf = rng.uniform(0.1, 0.5, M) if minor is None else np.asarray(minor, float)
+    theta = np.full(M - 1, 0.5 * (1.0 - np.exp(-2.0 * spacing / 100.0)))
+    partial = 0.5 * (1.0 - np.exp(-2.0 * (-0.5 * np.log(1.0 - 2.0 * theta)) / (nlod + 1)))
+    graph = np.zeros((M, 2 * N), np.int32)
+    graph[0, 2 * F:] = rng.integers(0, 2, 2 * (N - F))
+    for l in range(1, M):
+        graph[l, 2 * F:] = graph[l - 1, 2 * F:] ^ (rng.random(2 * (N - F)) < theta[l - 1])
+    alleles = np.zeros((N, 2, M), np.int8)
+    alleles[:F] = rng.random((F, 2, M)) < maf
+    for p in range(F, N):  # parents come before children
+        for side, q in enumerate((mother[p], father[p])):
+            alleles[p, side] = np.where(graph[:, 2 * p + side] == 0, alleles[q, 0], alleles[q, 1])
+    geno = np.where(alleles[:, 0] != alleles[:, 1], linkage.HETERO,
+                    np.where(alleles[:, 0] == 0, linkage.HOMOZ_A, linkage.HOMOZ_B)).astype(np.uint8)
+    geno[rng.random((N, M)) < missing] = linkage.UNTYPED
+    geno[list(untyped)] = linkage.UNTYPED
+    aff = np.where(np.arange(N) >= F, 1 + rng.integers(0, 2, N), 1).astype(np.int32)
+    dprob = np.array([linkage.disease_probs(int(a), i < F, 0.05, [0.1, 0.4, 0.9]) for i, a in enumerate(aff)])
+    case = Case(N=N, F=F, M=M, nlod=nlod, mother=mother, father=father, sex=np.zeros(N, np.int32), affection=aff,
+                typed=(geno != 0).any(axis=1).astype(np.int32), geno=geno, disease_prob=dprob,
+                geno_prob=linkage.sampler_cache(geno, maf), legal=linkage.eliminate(geno, mother, father, F),
+                theta=theta, partial_theta=partial, minor=maf,
+                ops=peelseq.build(N, F, mother, father, seed=1, tries=tries))
+    return case, graph
