@@ -194,6 +194,12 @@ __device__ __forceinline__ bool pass_fixed(const WaveArea& w, uint32_t e, uint32
 // the only caller
 __device__ __attribute__((noinline)) double log1p_exp_minus(double x) { return log1p(exp(-x)); }
 
+// the share of nA and nB founder alleles fixed to A and to B; a count of 0 has
+// none, also where its allele's frequency is 0 and the log infinite
+__device__ __forceinline__ double fixed_term(int nA, int nB, double lmaj, double lmin) {
+    return (nA ? (double)nA * lmaj : 0.0) + (nB ? (double)nB * lmin : 0.0);
+}
+
 // ln(e^l0 + e^l1) of a component free to take either assignment, from its
 // root's counts
 __device__ __forceinline__ double free_term(const MsampArgs& A, int l, uint32_t a, double lmaj, double lmin) {
@@ -283,7 +289,7 @@ __device__ double fag_log_likelihood(const MsampArgs& A, const uint2* ptab, cons
     }
     if (__ballot(conflict)) return -INFINITY;
     const double lmaj = A.lfreq[2 * (size_t)l], lmin = A.lfreq[2 * (size_t)l + 1];
-    const double ll = (double)nA * lmaj + (double)nB * lmin;
+    const double ll = fixed_term(nA, nB, lmaj, lmin);
     if (!__ballot(pending)) return ll;
     // components no homozygous person reaches: hook the larger root under the
     // smaller one with the parity the edge implies (the alleles of an edge
@@ -511,7 +517,7 @@ __device__ double fag_log_likelihood_r(const MsampArgs& A, const JobInputs<KC>& 
         }
     }
     if (__ballot(conflict)) return -INFINITY;
-    const double ll = (double)nA * lmaj + (double)nB * lmin;
+    const double ll = fixed_term(nA, nB, lmaj, lmin);
     if (!pending) return ll;
     if (listed <= 64) {
         // one edge left (half of the rest, nearly all of it at 150 people): its
