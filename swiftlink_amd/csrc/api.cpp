@@ -657,14 +657,15 @@ int setup_msampler(sl_ctx* c, const sl_pedigree_desc* ped) {
         c->m_why = "M-sampler workgroup needs more than 160 KiB of LDS";
         return SL_OK;
     }
-    if (c->m_spec_lds > 160 * 1024) c->m_spec_lds = 0;  // steps then take two launches
     // forward-backward passes keep the step's uniforms in LDS (in the
     // speculative kernel, in the dynamic LDS its job workgroups use)
     c->m_ubuf = M <= sl::kFbUbufLoci;
-    if (c->m_ubuf && c->m_spec_lds) c->m_spec_lds = std::max(c->m_spec_lds, sizeof(double) * (size_t)M);
+    if (c->m_ubuf) c->m_spec_lds = std::max(c->m_spec_lds, sizeof(double) * (size_t)M);
+    // steps take two launches where a workgroup's LDS cannot hold both
+    if (c->m_spec_lds + sl::fb_static_lds(sl::kSpecBlock) > sl::kLdsBytes) c->m_spec_lds = 0;
     c->m_beside_lds = sl::msampler_lds_bytes(A, sl::kFbBlock);
     if (c->m_ubuf) c->m_beside_lds = std::max(c->m_beside_lds, sizeof(double) * (size_t)M);
-    if (c->m_beside_lds > 160 * 1024 || M > sl::kMaxBesideLoci) c->m_beside_lds = 0;
+    if (c->m_beside_lds + sl::fb_static_lds(sl::kFbBlock) > sl::kLdsBytes || M > sl::kMaxBesideLoci) c->m_beside_lds = 0;
     SL_HIP(c, sl::configure_msampler_lds(c->m_lds, c->m_spec_lds, c->m_beside_lds));
     // the founder-allele log terms of every locus, formed once here: ln of
     // each allele's frequency, and the term ln(e^l0 + e^l1) - max(l0, l1) =

@@ -604,6 +604,7 @@ struct MatT {
     T a, b, c, d;  // [[a, b], [c, d]]
 };
 using Mat = MatT<double>;
+static_assert(fb_static_lds(64) == sizeof(Mat) + 2 * sizeof(uint32_t), "LDS of the scans: wtot, wcnt, wmap");
 
 // product with an exact power-of-two rescale keeping the largest entry in
 // [0.5, 1): for a normal largest entry m with biased exponent E the factor is

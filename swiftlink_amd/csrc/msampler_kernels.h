@@ -16,6 +16,10 @@ constexpr int kSpecBlock = 512;     // threads per workgroup of the speculative 
 constexpr int kFbBlock = 1024;      // threads per workgroup of the forward-backward kernel, and of the planned
                                     // kernel that runs it beside the next step's jobs
 constexpr int kMaxBesideLoci = 4 * kFbBlock;  // loci that kernel takes: segments of 1, 2 or 4 per thread
+// LDS of a workgroup, and what a kernel with a forward-backward pass declares of
+// it besides its dynamic LDS: a 2x2 FP64 product and two words per wavefront
+constexpr size_t kLdsBytes = 160 * 1024;
+constexpr size_t fb_static_lds(int block) { return (size_t)(block / 64) * (4 * sizeof(double) + 2 * sizeof(uint32_t)); }
 
 struct MsampArgs {
     int N, F, M, W;

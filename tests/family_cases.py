@@ -37,3 +37,18 @@ def family_case(mother, father, founders, markers, missing, seed, minor=None, sp
                 theta=theta, partial_theta=partial, minor=maf,
                 ops=peelseq.build(N, F, mother, father, seed=1, tries=tries))
     return case, graph
+
+
+def line_family(people, founders):
+    """A line of couples: each one's first child marries the next founder.
+    `people - founders` children in all, spread evenly."""
+    mother, father = [-1] * founders, [-1] * founders
+    couples, kids = founders - 1, people - founders
+    ma, pa = 0, 1
+    for c in range(couples):
+        first = len(mother)
+        for _ in range(kids // couples + (c < kids % couples)):
+            mother.append(ma)
+            father.append(pa)
+        ma, pa = first, c + 2
+    return dict(mother=mother, father=father, founders=founders)
