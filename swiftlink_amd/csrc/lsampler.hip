@@ -897,6 +897,7 @@ struct FlatArea {
     T* f4;              // [16] the entries by neighbour bits
     uint32_t* maxbits;  // [n_ops]
     uint32_t* cnt;      // [kFlatBlock/64]
+    int* scale_exp;     // [1] sum of log2 of the table scale factors consumed
     uint8_t* pmk;       // [N]
     uint8_t* cmb;       // [2NF] neighbour bits: left | right << 1
     __device__ FlatArea(unsigned char* p, const SampArgs& A, bool keep) {
@@ -910,7 +911,8 @@ struct FlatArea {
         f4 = dist + 8 * NF + 4;
         maxbits = reinterpret_cast<uint32_t*>(f4 + 16);
         cnt = maxbits + A.n_ops;
-        pmk = reinterpret_cast<uint8_t*>(cnt + kFlatBlock / 64);
+        scale_exp = reinterpret_cast<int*>(cnt + kFlatBlock / 64);
+        pmk = reinterpret_cast<uint8_t*>(scale_exp + 1);
         cmb = pmk + A.N;
     }
 };
@@ -1045,7 +1047,6 @@ __device__ __forceinline__ void flat_sample(const SampArgs& A, const FlatArea<T>
 template <typename T, bool RESCALE, bool KEEP>
 __global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
     extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ int s_scale_exp;
     const int N = A.N, F = A.F, M = A.M, n_ops = A.n_ops, NF = N - F, tid = threadIdx.x;
     const FlatArea<T> S(smem, A, KEEP);
     const int chain = (int)blockIdx.y;
@@ -1127,7 +1128,7 @@ __global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
         S.thr[tid] = p0 / (p0 + p1);
     }
     if (tid == 4) {
-        s_scale_exp = 0;
+        *S.scale_exp = 0;
         S.dist[8 * NF] = (T)1;
         S.dist[8 * NF + 1] = (T)0;
     }
@@ -1150,7 +1151,7 @@ __global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
 #pragma unroll
         for (int d = 0; d < kFlatAhead; ++d) {
             const bool last = from[d] + kFlatBlock >= to[d];
-            if (from[d] + tid < to[d]) flat_task<T, RESCALE, KEEP>(A, S, from[d] + tid, lo[d], hi[d], &s_scale_exp);
+            if (from[d] + tid < to[d]) flat_task<T, RESCALE, KEEP>(A, S, from[d] + tid, lo[d], hi[d], S.scale_exp);
             fetch(lo[d], hi[d], from[d], to[d]);
             if (last) {
                 __syncthreads();
@@ -1168,7 +1169,7 @@ __global__ void __launch_bounds__(kFlatBlock) lsampler_flat_kernel(SampArgs A) {
         // ln of the locus likelihood (locus_sampler2.cc:221, 228, 235): the
         // rescaled last table divided by the scale factors it absorbed
         double w = log((double)like);
-        if (RESCALE) w -= (double)s_scale_exp * 0.69314718055994530942;
+        if (RESCALE) w -= (double)*S.scale_exp * 0.69314718055994530942;
         A.imp_weight[chain] += w;
     }
     // 3. reverse sampling by reverse levels: the first wavefront while the
@@ -1310,7 +1311,7 @@ size_t lsampler_flat_lds_bytes(int precision, int cells_cap, int n_ops, int N, i
     const int NF = N - F;
     size_t b = 8 * ((size_t)n_ops + 2 * NF + 4);                                     // uop, um, thr
     b += esz * ((keep ? 5 : 1) * (size_t)cells_cap + 8 * NF + 4 + 16);               // tab, pre, dist, f4
-    b += 4 * ((size_t)n_ops + kFlatBlock / 64) + N + 2 * NF;                         // maxbits, cnt, pmk, cmb
+    b += 4 * ((size_t)n_ops + kFlatBlock / 64 + 1) + N + 2 * NF;                     // maxbits, cnt, scale_exp, pmk, cmb
     return (b + 15) / 16 * 16;
 }
 
