@@ -18,6 +18,7 @@
 #include "philox.h"
 #include "program.h"
 #include "sampler_kernels.h"
+#include "slots.h"
 #include "sampler_program.h"
 
 using sl::PeelProgram;
@@ -96,9 +97,8 @@ struct sl_ctx {
     uint32_t* g_lp_hdr = nullptr;   // and the adjoint's
     uint32_t* g_lp_fwd = nullptr;
     uint32_t* g_lp_rev = nullptr;
-    void* d_lp = nullptr;            // its wavefronts' table slots
-    size_t lp_bytes = 0;
-    size_t lp_limit = SIZE_MAX;      // bytes past which an allocation has failed
+    sl::Slots lp;                    // its wavefronts' table slots when scoring
+    sl::Slots g_lp;                  // and in the adjoint
     bool lod_global = false;     // the workgroup kernel's arena in global-memory slots (too large for LDS)
     void* d_lgt = nullptr;       // kLodGlobalSlots slots of arena_bytes
     size_t lgt_cap = 0;
@@ -373,7 +373,7 @@ int lanepeel_form(const sl_ctx* c, int G) {
         sl::lanepeel_lds_bytes(c->W) > 64 * 1024)
         return -1;
     const size_t slot = sl::lanepeel_slot_bytes(c->prog.lp_arena, 0, c->precision == SL_FP64);
-    if (c->lp_bytes < std::max(slot, std::min(kLpScoreBytes, kLpLeastWaves * slot))) return -1;  // no memory for them
+    if (c->lp.bytes < std::max(slot, std::min(kLpScoreBytes, kLpLeastWaves * slot))) return -1;  // no memory for them
     if (lane_mode(c, G)) {
         // the FP32 lane kernel's wavefronts hold their tables in LDS; while all
         // of a launch's are on the device at once it is the faster (30 people,
@@ -406,26 +406,19 @@ size_t partial_rows(const sl_ctx* c, int G) {
     return (size_t)lod_chunks(c, G) + (lanepeel_form(c, G) == sl::kLpFloatLanesFlat ? (size_t)G : 0);
 }
 
-// The lane peel's table slots: at least `bytes`, or as much as the device gives
-// down to a quarter of its SIMDs' wavefronts of `slot` bytes each (none below
-// that: the other kernels then serve the calls).  A size that was refused is not
-// asked for again.
-void ensure_lanepeel(sl_ctx* c, size_t bytes, size_t slot) {
-    const size_t least = std::min(bytes, kLpLeastWaves * slot);
-    for (;;) {
-        const size_t want = std::min(bytes, c->lp_limit);
-        if (want <= c->lp_bytes || want < least) return;
-        if (c->d_lp) (void)hipFree(c->d_lp);
-        c->d_lp = nullptr;
-        c->lp_bytes = 0;
-        if (hipMalloc(&c->d_lp, want) == hipSuccess) {
-            c->lp_bytes = want;
-            return;
-        }
-        (void)hipGetLastError();
-        c->d_lp = nullptr;
-        c->lp_limit = want / 2;
-    }
+// Grows table slots of the lane peel to `bytes`, or as much as there is down to a
+// quarter of the SIMDs' wavefronts of `slot` bytes each (below that the other
+// kernels serve the calls).
+void ensure_lanepeel(sl::Slots* s, size_t bytes, size_t slot) {
+    sl::grow(
+        s, bytes, std::min(bytes, kLpLeastWaves * slot),
+        [](size_t n) {
+            void* p = nullptr;
+            if (hipMalloc(&p, n) == hipSuccess) return p;
+            (void)hipGetLastError();
+            return (void*)nullptr;
+        },
+        [](void* p) { (void)hipFree(p); });
 }
 
 // Scoring's slots are allocated with the program, so that scoring itself never
@@ -433,10 +426,10 @@ void ensure_lanepeel(sl_ctx* c, size_t bytes, size_t slot) {
 void ensure_scoring_slots(sl_ctx* c) {
     if (!c->prog.lp_ok || sl::lanepeel_lds_bytes(c->W) > 64 * 1024) return;
     const size_t slot = sl::lanepeel_slot_bytes(c->prog.lp_arena, 0, c->precision == SL_FP64);
-    ensure_lanepeel(c, std::min(kLpScoreBytes, 4096 * slot), slot);
+    ensure_lanepeel(&c->lp, std::min(kLpScoreBytes, 4096 * slot), slot);
 }
 
-sl::LanePeelArgs lanepeel_args(const sl_ctx* c, const PeelProgram& P) {
+sl::LanePeelArgs lanepeel_args(const sl_ctx* c, const PeelProgram& P, const sl::Slots& slots) {
     sl::LanePeelArgs A{};
     A.n_ops = P.n_ops;
     A.arena_cells = P.lp_arena;
@@ -450,13 +443,13 @@ sl::LanePeelArgs lanepeel_args(const sl_ctx* c, const PeelProgram& P) {
     A.partial_theta = c->d_ptheta;
     A.log_theta = c->d_logt;
     A.log_anti = c->d_loga;
-    A.scratch = c->d_lp;
+    A.scratch = slots.p;
     return A;
 }
 
 // One scoring launch of the lane peel over A.graphs.
 hipError_t launch_lane_scoring(sl_ctx* c, int form, const sl::LodArgs& A) {
-    sl::LanePeelArgs B = lanepeel_args(c, c->prog);
+    sl::LanePeelArgs B = lanepeel_args(c, c->prog, c->lp);
     B.hdr = c->d_lp_hdr;
     B.fwd = c->d_lp_fwd;
     B.graphs = A.graphs;
@@ -477,7 +470,7 @@ hipError_t launch_lane_scoring(sl_ctx* c, int form, const sl::LodArgs& A) {
     }
     const int64_t E = sl::lanepeel_lanes(f, A.G, c->M - 1, c->npos);
     const size_t slot = sl::lanepeel_slot_bytes(c->prog.lp_arena, 0, c->precision == SL_FP64);
-    const hipError_t e = sl::launch_lanepeel(B, f, sl::lanepeel_waves(f, E, slot, c->lp_bytes),
+    const hipError_t e = sl::launch_lanepeel(B, f, sl::lanepeel_waves(f, E, slot, c->lp.bytes),
                                              sl::lanepeel_lds_bytes(c->W), c->stream);
     if (e != hipSuccess || !flat || A.terms) return e;
     return sl::launch_chunk_sums(B.terms, A.partial, A.G, (int)nacc, A.gate_sweep, A.gate_burnin, A.gate_period,
@@ -572,7 +565,7 @@ int release_all(sl_ctx* c) {
                     c->g_sched_off, c->g_sched_ops, c->d_gdp, c->d_jac, c->d_gterms, c->d_gstate, c->d_sweep,
                     c->d_imp_graphs, c->d_imp_draw, c->d_imp_weight, c->d_imp_status, c->d_elod_pairs,
                     c->d_gtables, c->d_lgt, c->d_lstream, c->d_trace,
-                    c->d_task, c->d_task_base, c->d_level_task, c->d_rrec, c->d_lp_hdr, c->d_lp_fwd, c->g_lp_hdr, c->g_lp_fwd, c->g_lp_rev, c->d_lp};
+                    c->d_task, c->d_task_base, c->d_level_task, c->d_rrec, c->d_lp_hdr, c->d_lp_fwd, c->g_lp_hdr, c->g_lp_fwd, c->g_lp_rev, c->lp.p, c->g_lp.p};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& e : c->ev_pool) (void)hipEventDestroy(e);
@@ -2382,13 +2375,13 @@ int launch_adjoint(sl_ctx* c, const sl::LodArgs& A, double* out) {
     const int64_t E = (int64_t)A.G * (c->M - 1) * c->npos;
     const size_t slot = sl::lanepeel_slot_bytes(c->gprog.lp_arena, c->gprog.lp_adj, true);
     const bool lanes = c->gprog.lp_ok && E >= kLpMinGradEvals && sl::lanepeel_lds_bytes(c->W) <= 64 * 1024;
-    if (lanes) ensure_lanepeel(c, sl::lanepeel_waves(sl::kLpAdjoint, E, slot, kLpGradBytes) * slot, slot);
-    if (!lanes || c->lp_bytes < std::min<size_t>(kLpLeastWaves, (size_t)((E + 63) / 64)) * slot) {
+    if (lanes) ensure_lanepeel(&c->g_lp, sl::lanepeel_waves(sl::kLpAdjoint, E, slot, kLpGradBytes) * slot, slot);
+    if (!lanes || c->g_lp.bytes < std::min<size_t>(kLpLeastWaves, (size_t)((E + 63) / 64)) * slot) {
         sl::GradArgs Gd{c->d_jac, out, c->npos};
         SL_HIP(c, sl::launch_grad(A, Gd, 0, c->g_lds, c->stream));
         return SL_OK;
     }
-    sl::LanePeelArgs B = lanepeel_args(c, c->gprog);
+    sl::LanePeelArgs B = lanepeel_args(c, c->gprog, c->g_lp);
     B.hdr = c->g_lp_hdr;
     B.fwd = c->g_lp_fwd;
     B.rev = c->g_lp_rev;
@@ -2396,7 +2389,7 @@ int launch_adjoint(sl_ctx* c, const sl::LodArgs& A, double* out) {
     B.G = A.G;
     B.jac = c->d_jac;
     B.out = out;
-    SL_HIP(c, sl::launch_lanepeel(B, sl::kLpAdjoint, sl::lanepeel_waves(sl::kLpAdjoint, E, slot, c->lp_bytes),
+    SL_HIP(c, sl::launch_lanepeel(B, sl::kLpAdjoint, sl::lanepeel_waves(sl::kLpAdjoint, E, slot, c->g_lp.bytes),
                                   sl::lanepeel_lds_bytes(c->W), c->stream));
     return SL_OK;
 }

@@ -1,0 +1,69 @@
+"""The rule by which a context's optional device buffers grow (csrc/slots.h),
+compiled for the host with an allocator that refuses sizes."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+PROGRAM = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <map>
+#include "slots.h"
+
+static std::map<void*, size_t> live;
+static size_t largest;  // an allocation past it is refused
+static int asked;
+
+static void* take(size_t n) {
+    ++asked;
+    if (n > largest) return nullptr;
+    void* p = malloc(1);
+    live[p] = n;
+    return p;
+}
+static void drop(void* p) {
+    if (!live.count(p)) abort();
+    live.erase(p);
+    free(p);
+}
+static void grow(sl::Slots* s, size_t bytes, size_t least) { sl::grow(s, bytes, least, take, drop); }
+static void show(const sl::Slots& s) {
+    if (s.p && live.at(s.p) != s.bytes) abort();
+    printf("%zu %zu %d\n", s.bytes, live.size(), asked);
+    asked = 0;
+}
+
+int main() {
+    sl::Slots s;
+    largest = 1000;
+    grow(&s, 256, 64), show(s);    // given
+    grow(&s, 200, 64), show(s);    // there already
+    largest = 100;
+    grow(&s, 4000, 2000), show(s);  // refused down to the least: the 256 stay
+    grow(&s, 4000, 2000), show(s);  // not asked again
+    sl::Slots t;
+    largest = 600;
+    grow(&t, 4000, 64), show(t);   // halved until given, beside s
+    largest = 5000;
+    grow(&t, 4000, 64), show(t);   // what was refused is not asked again
+    sl::Slots u;
+    grow(&u, 4000, 64), show(u);
+    grow(&u, 5000, 64), show(u);   // replaced: the old one is released
+    return 0;
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+def test_growth(tmp_path):
+    src, exe = tmp_path / "slots.cpp", tmp_path / "slots"
+    src.write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", os.path.join(ROOT, "swiftlink_amd", "csrc"), str(src),
+                    "-o", str(exe)], check=True, timeout=300)
+    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True, timeout=60).stdout
+    assert [tuple(map(int, x.split())) for x in out.splitlines()] == [
+        (256, 1, 1), (256, 1, 0), (256, 1, 2), (256, 1, 0), (500, 2, 4), (500, 2, 0), (4000, 3, 1), (5000, 3, 1)]
