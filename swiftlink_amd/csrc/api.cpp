@@ -406,6 +406,13 @@ size_t partial_rows(const sl_ctx* c, int G) {
     return (size_t)lod_chunks(c, G) + (lanepeel_form(c, G) == sl::kLpFloatLanesFlat ? (size_t)G : 0);
 }
 
+size_t free_memory() {
+    size_t avail = 0, total = 0;
+    if (hipMemGetInfo(&avail, &total) == hipSuccess) return avail;
+    (void)hipGetLastError();
+    return 0;
+}
+
 // Grows table slots of the lane peel to `bytes`, or as much as there is down to a
 // quarter of the SIMDs' wavefronts of `slot` bytes each (below that the other
 // kernels serve the calls).
@@ -418,7 +425,7 @@ void ensure_lanepeel(sl::Slots* s, size_t bytes, size_t slot) {
             (void)hipGetLastError();
             return (void*)nullptr;
         },
-        [](void* p) { (void)hipFree(p); });
+        [](void* p) { (void)hipFree(p); }, free_memory);
 }
 
 // Scoring's slots are allocated with the program, so that scoring itself never
@@ -1196,8 +1203,8 @@ static sl::SampArgs samp_args(sl_ctx* c);
 // The flat L-sampler's records (lsampler.hip).  Leaves flat_ok false where it
 // does not apply: an op consumes more than three tables or has more than three
 // children, an index passes 16 bits, the tables alone do not fit LDS, or the
-// records pass kFlatMaxBytes or the memory there is (the loci's steps are then
-// decoded in the kernel).
+// records pass kFlatMaxBytes or their share of the memory there is (the loci's
+// steps are then decoded in the kernel).
 static int setup_flat(sl_ctx* c) {
     const sl::SampProgram& P = c->sprog;
     for (int keep = 0; keep < 2; ++keep)
@@ -1205,11 +1212,12 @@ static int setup_flat(sl_ctx* c) {
     if (P.max_prev > sl::kFlatMaxPrev || P.max_child > sl::kFlatMaxKids || P.cell_base.empty() || c->N >= 8000 ||
         c->flat_lds[0] > 160 * 1024 || sl::lsampler_build_lds_bytes(P.n_ops, c->N) > 64 * 1024)
         return SL_OK;
-    const size_t words = 4 * (size_t)P.cell_base[c->M] * sl::kTaskWords;
-    if (words * sizeof(uint32_t) > kFlatMaxBytes) return SL_OK;
     uint32_t** bufs[] = {&c->d_task, &c->d_level_task, &c->d_rrec, &c->d_task_base};
-    const size_t sizes[] = {words, (size_t)c->M * (P.n_levels + 1), (size_t)c->M * P.n_ops * sl::kRevWords,
-                            (size_t)c->M + 1};
+    const size_t sizes[] = {4 * (size_t)P.cell_base[c->M] * sl::kTaskWords, (size_t)c->M * (P.n_levels + 1),
+                            (size_t)c->M * P.n_ops * sl::kRevWords, (size_t)c->M + 1};
+    const size_t words = sizes[0] + sizes[1] + sizes[2] + sizes[3];
+    if (sizes[0] * sizeof(uint32_t) > kFlatMaxBytes || words * sizeof(uint32_t) > free_memory() / sl::kOptionalShare)
+        return SL_OK;
     for (int i = 0; i < 4; ++i)
         if (hipMalloc((void**)bufs[i], sizes[i] * sizeof(uint32_t)) != hipSuccess) {
             (void)hipGetLastError();

@@ -8,17 +8,24 @@
 
 namespace sl {
 
+// Share of the free memory one such buffer may take, so that contexts made one
+// after another leave room for the buffers they cannot do without.
+constexpr size_t kOptionalShare = 8;
+
 struct Slots {
     void* p = nullptr;
     size_t bytes = 0;
-    size_t limit = SIZE_MAX;  // bytes past which a request has been refused
+    size_t limit = SIZE_MAX;  // bytes past which a request has been refused or cut
 };
 
-// Grows s to `bytes`, or as much as alloc(size) gives (null: refused), down to
-// `least`.  A size that was refused is not asked for again.  The old buffer is
-// released once the new one is there.
-template <typename Alloc, typename Release>
-void grow(Slots* s, size_t bytes, size_t least, Alloc alloc, Release release) {
+// Grows s to `bytes`, or as much as alloc(size) (null when refused) and a share
+// of free_bytes() give, down to `least`.  A size that was refused is not asked
+// for again.  The old buffer is released once the new one is there.
+template <typename Alloc, typename Release, typename Free>
+void grow(Slots* s, size_t bytes, size_t least, Alloc alloc, Release release, Free free_bytes) {
+    if (std::min(bytes, s->limit) <= s->bytes) return;
+    const size_t share = free_bytes() / kOptionalShare;
+    if (bytes > share) s->limit = std::min(s->limit, share);
     for (;;) {
         const size_t want = std::min(bytes, s->limit);
         if (want <= s->bytes || want < least) return;

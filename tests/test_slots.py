@@ -16,6 +16,7 @@ PROGRAM = r"""
 
 static std::map<void*, size_t> live;
 static size_t largest;  // an allocation past it is refused
+static size_t unused = 1 << 20;
 static int asked;
 
 static void* take(size_t n) {
@@ -30,7 +31,7 @@ static void drop(void* p) {
     live.erase(p);
     free(p);
 }
-static void grow(sl::Slots* s, size_t bytes, size_t least) { sl::grow(s, bytes, least, take, drop); }
+static void grow(sl::Slots* s, size_t bytes, size_t least) { sl::grow(s, bytes, least, take, drop, [] { return unused; }); }
 static void show(const sl::Slots& s) {
     if (s.p && live.at(s.p) != s.bytes) abort();
     printf("%zu %zu %d\n", s.bytes, live.size(), asked);
@@ -53,6 +54,14 @@ int main() {
     sl::Slots u;
     grow(&u, 4000, 64), show(u);
     grow(&u, 5000, 64), show(u);   // replaced: the old one is released
+    sl::Slots v;
+    unused = 8000;
+    grow(&v, 4000, 64), show(v);   // cut to an eighth of the free memory
+    unused = 1 << 20;
+    grow(&v, 4000, 64), show(v);   // and stays so
+    sl::Slots w;
+    unused = 8000;
+    grow(&w, 4000, 2000), show(w);  // not asked for below the least
     return 0;
 }
 """
@@ -66,4 +75,5 @@ def test_growth(tmp_path):
                     "-o", str(exe)], check=True, timeout=300)
     out = subprocess.run([str(exe)], check=True, capture_output=True, text=True, timeout=60).stdout
     assert [tuple(map(int, x.split())) for x in out.splitlines()] == [
-        (256, 1, 1), (256, 1, 0), (256, 1, 2), (256, 1, 0), (500, 2, 4), (500, 2, 0), (4000, 3, 1), (5000, 3, 1)]
+        (256, 1, 1), (256, 1, 0), (256, 1, 2), (256, 1, 0), (500, 2, 4), (500, 2, 0), (4000, 3, 1), (5000, 3, 1),
+        (1000, 4, 1), (1000, 4, 0), (0, 4, 0)]
