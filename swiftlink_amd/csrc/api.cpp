@@ -272,10 +272,25 @@ int hip_fail(sl_ctx* c, hipError_t e, const char* where) {
         if (e_ != hipSuccess) return hip_fail((c), e_, #call); \
     } while (0)
 
+// Memory a call cannot do without; a context's adjoint slots make room for it.
+hipError_t device_alloc(sl_ctx* c, void** p, size_t bytes) {
+    hipError_t e = hipSuccess;
+    *p = sl::take(
+        &c->g_lp, bytes,
+        [&](size_t n) {
+            void* q = nullptr;
+            e = hipMalloc(&q, n);
+            if (e != hipSuccess) (void)hipGetLastError();
+            return e == hipSuccess ? q : nullptr;
+        },
+        [](void* q) { (void)hipFree(q); });
+    return e;
+}
+
 template <typename T>
 int upload(sl_ctx* c, T** dst, const T* src, size_t n) {
     if (n == 0) n = 1;
-    SL_HIP(c, hipMalloc((void**)dst, n * sizeof(T)));
+    SL_HIP(c, device_alloc(c, (void**)dst, n * sizeof(T)));
     if (src) SL_HIP(c, hipMemcpyAsync(*dst, src, n * sizeof(T), hipMemcpyHostToDevice, c->stream));
     return SL_OK;
 }
@@ -285,7 +300,7 @@ int ensure(sl_ctx* c, T** buf, size_t* cap, size_t n) {
     if (n <= *cap) return SL_OK;
     if (*buf) SL_HIP(c, hipFree(*buf));
     *buf = nullptr;
-    SL_HIP(c, hipMalloc((void**)buf, n * sizeof(T)));
+    SL_HIP(c, device_alloc(c, (void**)buf, n * sizeof(T)));
     *cap = n;
     return SL_OK;
 }
@@ -1260,15 +1275,15 @@ static int alloc_chains(sl_ctx* c, int n_chains) {
             *b = nullptr;
         }
         c->n_chains = 0;
-        SL_HIP(c, hipMalloc((void**)&c->d_chains, words * sizeof(uint32_t)));
-        SL_HIP(c, hipMalloc((void**)&c->d_status, (size_t)n_chains * sizeof(int32_t)));
-        SL_HIP(c, hipMalloc((void**)&c->d_lcur, cm * sizeof(double)));
-        SL_HIP(c, hipMalloc((void**)&c->d_lflip, 4 * cm * sizeof(double)));
-        SL_HIP(c, hipMalloc((void**)&c->d_fbuf, 2 * cm * sizeof(double)));
-        SL_HIP(c, hipMalloc((void**)&c->d_maps, cm));
-        SL_HIP(c, hipMalloc((void**)&c->d_mu, (c->m_ubuf ? 2 * cm : 1) * sizeof(double)));
-        SL_HIP(c, hipMalloc((void**)&c->d_near, (size_t)n_chains * sizeof(uint32_t)));
-        SL_HIP(c, hipMalloc((void**)&c->d_near_loci, (size_t)n_chains * near_words(c) * sizeof(uint32_t)));
+        SL_HIP(c, device_alloc(c, (void**)&c->d_chains, words * sizeof(uint32_t)));
+        SL_HIP(c, device_alloc(c, (void**)&c->d_status, (size_t)n_chains * sizeof(int32_t)));
+        SL_HIP(c, device_alloc(c, (void**)&c->d_lcur, cm * sizeof(double)));
+        SL_HIP(c, device_alloc(c, (void**)&c->d_lflip, 4 * cm * sizeof(double)));
+        SL_HIP(c, device_alloc(c, (void**)&c->d_fbuf, 2 * cm * sizeof(double)));
+        SL_HIP(c, device_alloc(c, (void**)&c->d_maps, cm));
+        SL_HIP(c, device_alloc(c, (void**)&c->d_mu, (c->m_ubuf ? 2 * cm : 1) * sizeof(double)));
+        SL_HIP(c, device_alloc(c, (void**)&c->d_near, (size_t)n_chains * sizeof(uint32_t)));
+        SL_HIP(c, device_alloc(c, (void**)&c->d_near_loci, (size_t)n_chains * near_words(c) * sizeof(uint32_t)));
         c->n_chains = n_chains;
     }
     SL_HIP(c, hipMemsetAsync(c->d_status, 0, (size_t)n_chains * sizeof(int32_t), c->stream));
@@ -1671,7 +1686,7 @@ static int grow_trace(sl_ctx* c, size_t n) {
     if (n <= c->trace_cap) return SL_OK;
     const size_t cap = std::max(n, 2 * c->trace_cap);
     double* nb = nullptr;
-    SL_HIP(c, hipMalloc((void**)&nb, cap * sizeof(double)));
+    SL_HIP(c, device_alloc(c, (void**)&nb, cap * sizeof(double)));
     const size_t used = c->trace_iter.size() * (size_t)c->n_chains;
     if (used) SL_HIP(c, hipMemcpyAsync(nb, c->d_trace, used * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
     SL_HIP(c, hipStreamSynchronize(c->stream));
@@ -1900,7 +1915,7 @@ int sl_mcmc_run(sl_ctx* c, const sl_schedule* sch, sl_mcmc_stats* stats) {
     if (captured) {
         const int nmei = (int)c->meioses_h.size();
         int rc = SL_OK;
-        if (!c->d_sweep) SL_HIP(c, hipMalloc((void**)&c->d_sweep, sizeof(uint32_t)));
+        if (!c->d_sweep) SL_HIP(c, device_alloc(c, (void**)&c->d_sweep, sizeof(uint32_t)));
         if ((any_l || any_both) && !c->flat_ok) rc = ensure_gtables(c);
         if (!rc && (any_m || any_both) && nmei)
             rc = ensure_msweep(c, (size_t)nmei);
@@ -2420,8 +2435,8 @@ int sl_set_trait_model(sl_ctx* c, const sl_trait_model* model) {
         c->dp_h = old;
         return rc;
     }
-    if (!c->d_gdp) SL_HIP(c, hipMalloc((void**)&c->d_gdp, dp.size() * sizeof(double)));
-    if (!c->d_jac) SL_HIP(c, hipMalloc((void**)&c->d_jac, jac.size() * sizeof(double)));
+    if (!c->d_gdp) SL_HIP(c, device_alloc(c, (void**)&c->d_gdp, dp.size() * sizeof(double)));
+    if (!c->d_jac) SL_HIP(c, device_alloc(c, (void**)&c->d_jac, jac.size() * sizeof(double)));
     SL_HIP(c, hipMemcpyAsync(c->d_gdp, dp.data(), dp.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
     SL_HIP(c, hipMemcpyAsync(c->d_jac, jac.data(), jac.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
     SL_HIP(c, hipStreamSynchronize(c->stream));

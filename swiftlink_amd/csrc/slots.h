@@ -39,4 +39,16 @@ void grow(Slots* s, size_t bytes, size_t least, Alloc alloc, Release release, Fr
     }
 }
 
+// alloc(n) for a buffer a call cannot do without: where it is refused and s holds
+// one that calls can do without, that one is released first.
+template <typename Alloc, typename Release>
+void* take(Slots* s, size_t n, Alloc alloc, Release release) {
+    void* p = alloc(n);
+    if (p || !s->p) return p;
+    release(s->p);
+    s->p = nullptr;
+    s->bytes = 0;
+    return alloc(n);
+}
+
 }  // namespace sl

@@ -19,7 +19,7 @@ static size_t largest;  // an allocation past it is refused
 static size_t unused = 1 << 20;
 static int asked;
 
-static void* take(size_t n) {
+static void* get(size_t n) {
     ++asked;
     if (n > largest) return nullptr;
     void* p = malloc(1);
@@ -31,7 +31,7 @@ static void drop(void* p) {
     live.erase(p);
     free(p);
 }
-static void grow(sl::Slots* s, size_t bytes, size_t least) { sl::grow(s, bytes, least, take, drop, [] { return unused; }); }
+static void grow(sl::Slots* s, size_t bytes, size_t least) { sl::grow(s, bytes, least, get, drop, [] { return unused; }); }
 static void show(const sl::Slots& s) {
     if (s.p && live.at(s.p) != s.bytes) abort();
     printf("%zu %zu %d\n", s.bytes, live.size(), asked);
@@ -62,6 +62,14 @@ int main() {
     sl::Slots w;
     unused = 8000;
     grow(&w, 4000, 2000), show(w);  // not asked for below the least
+    largest = 300;
+    void* a = sl::take(&u, 200, get, drop);  // given: u (5000) stays
+    printf("%d %zu\n", a != nullptr, u.bytes);
+    largest = 100;
+    void* b = sl::take(&u, 200, [](size_t n) { if (live.size() < 5) largest = 200; return get(n); }, drop);
+    printf("%d %zu\n", b != nullptr, u.bytes);  // refused at first: u is released
+    void* c = sl::take(&u, 300, get, drop);
+    printf("%d %zu\n", c != nullptr, u.bytes);  // nothing left to release
     return 0;
 }
 """
@@ -76,4 +84,5 @@ def test_growth(tmp_path):
     out = subprocess.run([str(exe)], check=True, capture_output=True, text=True, timeout=60).stdout
     assert [tuple(map(int, x.split())) for x in out.splitlines()] == [
         (256, 1, 1), (256, 1, 0), (256, 1, 2), (256, 1, 0), (500, 2, 4), (500, 2, 0), (4000, 3, 1), (5000, 3, 1),
-        (1000, 4, 1), (1000, 4, 0), (0, 4, 0)]
+        (1000, 4, 1), (1000, 4, 0), (0, 4, 0),
+        (1, 5000), (1, 0), (0, 0)]
