@@ -298,11 +298,13 @@ int upload(sl_ctx* c, T** dst, const T* src, size_t n) {
 template <typename T>
 int ensure(sl_ctx* c, T** buf, size_t* cap, size_t n) {
     if (n <= *cap) return SL_OK;
-    if (*buf) SL_HIP(c, hipFree(*buf));
-    *buf = nullptr;
-    SL_HIP(c, device_alloc(c, (void**)buf, n * sizeof(T)));
-    *cap = n;
-    return SL_OK;
+    return sl::replace(
+        buf, cap, n,
+        [c](T** p, size_t m) {
+            SL_HIP(c, device_alloc(c, (void**)p, m * sizeof(T)));
+            return SL_OK;
+        },
+        [](T* p) { (void)hipFree(p); });
 }
 
 sl::LodArgs lod_args(sl_ctx* c) {

@@ -51,4 +51,16 @@ void* take(Slots* s, size_t n, Alloc alloc, Release release) {
     return alloc(n);
 }
 
+// Replaces the buffer *p of *cap elements by one of n; alloc(p, n) is 0 when given.
+// Refused, it leaves none, of no elements, so that the next request asks again.
+template <typename T, typename Alloc, typename Release>
+int replace(T** p, size_t* cap, size_t n, Alloc alloc, Release release) {
+    if (*p) release(*p);
+    *p = nullptr;
+    *cap = 0;
+    const int rc = alloc(p, n);
+    if (rc == 0) *cap = n;
+    return rc;
+}
+
 }  // namespace sl

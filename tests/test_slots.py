@@ -70,6 +70,17 @@ int main() {
     printf("%d %zu\n", b != nullptr, u.bytes);  // refused at first: u is released
     void* c = sl::take(&u, 300, get, drop);
     printf("%d %zu\n", c != nullptr, u.bytes);  // nothing left to release
+    char* buf = nullptr;
+    size_t cap = 0;
+    const auto alloc = [](char** p, size_t n) { return (*p = (char*)get(n)) ? 0 : -3; };
+    const auto replace = [&](size_t n) {
+        const int rc = sl::replace(&buf, &cap, n, alloc, [](char* p) { drop(p); });
+        printf("%d %d %zu\n", rc, buf != nullptr, cap);
+    };
+    largest = 100;
+    replace(50);
+    replace(200);  // refused: no buffer, and none is said to be there
+    replace(40);
     return 0;
 }
 """
@@ -85,4 +96,5 @@ def test_growth(tmp_path):
     assert [tuple(map(int, x.split())) for x in out.splitlines()] == [
         (256, 1, 1), (256, 1, 0), (256, 1, 2), (256, 1, 0), (500, 2, 4), (500, 2, 0), (4000, 3, 1), (5000, 3, 1),
         (1000, 4, 1), (1000, 4, 0), (0, 4, 0),
-        (1, 5000), (1, 0), (0, 0)]
+        (1, 5000), (1, 0), (0, 0),
+        (0, 1, 50), (-3, 0, 0), (0, 1, 40)]
