@@ -398,8 +398,10 @@ int lanepeel_form(const sl_ctx* c, int G) {
         // graphs: 1328 us against 790; 77 people, 70 graphs: 318 against 227)
         const int64_t waves = (int64_t)(c->M - 1) * c->npos * ((G + 63) / 64);
         if (waves <= kCus * (int64_t)(160 * 1024 / c->lane_lds)) return -1;
-        // 64 graphs to a wavefront where that leaves few lanes empty
-        return (G + 63) / 64 * 64 > G + G / 16 ? sl::kLpFloatLanesFlat : sl::kLpFloatLanes;
+        // 64 graphs to a wavefront where that leaves few lanes empty, or where
+        // every graph's terms would take more than the slots may
+        const size_t terms = (size_t)G * (c->M - 1) * c->npos * sizeof(double);
+        return (G + 63) / 64 * 64 > G + G / 16 && terms <= kLpScoreBytes ? sl::kLpFloatLanesFlat : sl::kLpFloatLanes;
     }
     if (c->gpw != 1) return -1;
     return c->precision == SL_FP64 ? sl::kLpDouble : sl::kLpFloat;

@@ -25,3 +25,25 @@ def test_scoring_before_and_after_a_gradient(tmp_path):
     ok = np.isfinite(before)
     assert ok.any()
     np.testing.assert_allclose(grad[..., 0][ok], before[ok], rtol=1e-14)
+
+
+def test_terms_of_a_long_map_take_no_array(tmp_path):
+    """400 graphs of 100000 positions: 320 MB of terms, which the wavefronts sum
+    themselves, as the FP32 lane kernel's do (equal to the rounding of ln L + E ln 2,
+    |ln L| below 1e3)."""
+    import torch
+    from swiftlink_amd.case import pack_graphs
+    case, data = synth.make_case("ped30_snp100", str(tmp_path), n_markers=20001)
+    n = 400
+    g = _graphs(case, data, 20)
+    dev = torch.from_numpy(pack_graphs(case, g).reshape(20, -1).view(np.int32)).cuda()
+    dev = dev[torch.arange(n, device="cuda") % 20].contiguous()
+    torch.cuda.synchronize()
+    out = []
+    for kernel in (native.SL_LOD_AUTO, native.SL_LOD_LANES):
+        with native.Context(case, native.SL_FP32_RESCALED, lod_kernel=kernel) as ctx:
+            free = torch.cuda.mem_get_info()[0]
+            ctx.lod_accumulate_packed(dev.data_ptr(), n)
+            out.append(ctx.lod_results()[0])
+            assert free - torch.cuda.mem_get_info()[0] < 64 * MIB
+    assert np.abs(out[0] - out[1]).max() < 1e-12
