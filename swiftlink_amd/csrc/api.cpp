@@ -2157,7 +2157,7 @@ int sl_batch_run(sl_batch* b, const sl_schedule* sch, sl_mcmc_stats* stats) {
         }
         int rc = ensure(c, &c->d_partial, &c->partial_cap, (size_t)(c->M - 1) * c->npos * partial_rows(c, C));
         if (!rc && c->m_ready) rc = ensure_msweep(c, c->meioses_h.size());
-        if (!rc && c->samp_ready) rc = ensure_gtables(c);
+        if (!rc && c->samp_ready && !c->flat_ok) rc = ensure_gtables(c);
         if (rc) return rc;
         SL_HIP(c, hipMemcpyAsync(c->d_sweep, &sch->first_sweep, sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
         SL_HIP(c, hipStreamSynchronize(c->stream));

@@ -3,6 +3,7 @@ the same results as these come and go."""
 import numpy as np
 import pytest
 
+from family_cases import family_case, line_family
 from swiftlink_amd import native, synth
 from test_gpu_lanepeel import MODEL, _graphs
 
@@ -47,3 +48,28 @@ def test_terms_of_a_long_map_take_no_array(tmp_path):
             out.append(ctx.lod_results()[0])
             assert free - torch.cuda.mem_get_info()[0] < 64 * MIB
     assert np.abs(out[0] - out[1]).max() < 1e-12
+
+
+def test_batches_allocate_the_tables_they_use():
+    """300 people, hardly typed, in FP64: tables and kept products pass LDS, so the
+    decoding L-sampler would keep both in 2048 slots of global memory (at least
+    5 x 8 bytes x 3500 cells each, 286 MB); the record form that runs has no slots."""
+    import torch
+    case, g0 = family_case(markers=50, missing=0.95, seed=1, tries=1, **line_family(300, 80))
+    legal = np.array([bin(x).count("1") for x in range(16)])[case.legal & 15]
+    cells = sum(np.prod(legal[case.ops.cutset(o)], axis=0, dtype=int) for o in range(case.ops.n))
+    assert 5 * 8 * cells.max() > 160 * 1024
+    with native.Context(case, native.SL_FP64) as ctx:
+        ctx.mcmc_init(np.stack([g0, g0]))
+        ctx.lod_reset()
+        with native.Batch([ctx]) as b:
+            free = torch.cuda.mem_get_info()[0]
+            b.run(4, 0, 2, 0.5, 7)
+            assert free - torch.cuda.mem_get_info()[0] < 128 * MIB
+        out = ctx.mcmc_graphs()
+        assert np.all(ctx.mcmc_status() == 0)
+    with native.Context(case, native.SL_FP64) as ctx:
+        ctx.mcmc_init(np.stack([g0, g0]))
+        ctx.lod_reset()
+        ctx.mcmc_run(4, 0, 2, 0.5, 7)
+        assert np.array_equal(out, ctx.mcmc_graphs())
