@@ -1,8 +1,10 @@
 """Cases from a pedigree given as parent arrays, without going through files."""
+import dataclasses
+
 import numpy as np
 
 from swiftlink_amd import linkage, peelseq
-from swiftlink_amd.case import Case
+from swiftlink_amd.case import OP_CHILD, Case, PeelOps
 
 
 def family_case(mother, father, founders, markers, missing, seed, minor=None, spacing=0.5, nlod=2, untyped=(),
@@ -52,3 +54,27 @@ def line_family(people, founders):
             father.append(pa)
         ma, pa = first, c + 2
     return dict(mother=mother, father=father, founders=founders)
+
+
+def unchained(case):
+    """The case with a peel table in which a couple's children are peeled side by
+    side: a CHILD op that consumes another over the same parents leaves that table to
+    its own consumer, whose op then consumes as many tables as the couple has
+    children."""
+    ops = case.ops
+    prevs = [ops.prevs(o) for o in range(ops.n)]
+    for o in range(ops.n - 1, -1, -1):
+        for q in list(prevs[o]):
+            if ops.type[o] == OP_CHILD == ops.type[q] and set(ops.cutset(o)) == set(ops.cutset(q)):
+                up = next(u for u in range(o + 1, ops.n) if o in prevs[u])
+                prevs[o].remove(q)
+                prevs[up].append(q)
+                break
+    return dataclasses.replace(case, ops=PeelOps.from_lists(
+        ops.type, ops.peel, [ops.cutset(o) for o in range(ops.n)], prevs, [ops.children(o) for o in range(ops.n)]))
+
+
+def locus_cells(case):
+    """Cells of the L-sampler's tables at each locus."""
+    legal = np.array([bin(x).count("1") for x in range(16)])[case.legal & 15]
+    return sum(np.prod(legal[case.ops.cutset(o)], axis=0, dtype=int) for o in range(case.ops.n))

@@ -82,3 +82,19 @@ def test_products_formed_again(tmp_path, people, missing, chains, markers):
             continue
         return _check(case, data, chains)
     raise AssertionError("no family")
+
+
+def test_op_of_four_tables():
+    from family_cases import family_case, line_family, unchained
+    case, g = family_case(markers=9, missing=0.2, seed=6, tries=4, **line_family(26, 8))
+    case = unchained(case)
+    assert max(len(case.ops.prevs(o)) for o in range(case.ops.n)) == 4
+    o = Oracle(case)
+    with native.Context(case, native.SL_FP64) as ctx:
+        ctx.mcmc_init(np.stack([g, g]))
+        ctx.lsweep(5, 0, 0)
+        out = ctx.mcmc_graphs()
+        assert np.all(ctx.mcmc_status() == 0)
+        assert np.all(ctx.mcmc_near_edge() == 0)
+    for c in range(2):
+        assert np.array_equal(out[c], oracle_lsweep(o, g, case.M, 5, c, 0, 0)), c
