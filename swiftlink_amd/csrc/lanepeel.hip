@@ -648,7 +648,6 @@ __device__ __forceinline__ void founder_reverse(const LanePeelArgs& A, const Lan
     pass_adjoint<kLpM>(adj, hp, L.lane, g, cur);
 }
 
-// A term's factor besides its consumed tables
 // sum of a child's transmission factors over its allowed (i, j)
 __device__ __forceinline__ double allowed_sum(const double q[4], uint32_t m) {
     double s = 0.0;
@@ -658,6 +657,7 @@ __device__ __forceinline__ double allowed_sum(const double q[4], uint32_t m) {
     return s;
 }
 
+// a term's factor besides its consumed tables
 template <int TYPE, int NC>
 __device__ __forceinline__ double term_factor(const Trait<double>& tr, const double q[4], const double (*qk)[4], uint32_t info,
                                               uint32_t t) {

@@ -163,8 +163,8 @@ std::string build_lanepeel(const PedigreeView& ped, const PeelView& pv, const st
     } else {
         P.lp_arena = place(stored, size, born, dies, &off);
     }
-    // compact cell of table o at (a: value of person pa, b: of pb), or 0xFF
-    auto cell_of = [&](int o, int pa, int a, int pb, int b) -> uint32_t {
+    // compact cell of table o where person pa has value a and its other person b, or 0xFF
+    auto cell_of = [&](int o, int pa, int a, int b) -> uint32_t {
         uint32_t ix = 0, st = 1;
         for (int who : cuts[o]) {
             const int v = who == pa ? a : b;
@@ -173,7 +173,6 @@ std::string build_lanepeel(const PedigreeView& ped, const PeelView& pv, const st
             ix += st * (uint32_t)popc4(m & ((1u << v) - 1u));
             st *= (uint32_t)popc4(m);
         }
-        (void)pb;
         return ix;
     };
     P.lp_hdr.assign((size_t)n * kLpHeader, 0u);
@@ -193,16 +192,14 @@ std::string build_lanepeel(const PedigreeView& ped, const PeelView& pv, const st
         h[kHKids] = (uint32_t)d.n_child;
         memcpy(h + kHTrait, ped.disease_prob + 4 * (size_t)d.peel, 4 * sizeof(double));
         const int mat = d.type == kChild ? ped.mother[d.peel] : -1, pat = d.type == kChild ? ped.father[d.peel] : -1;
-        int axis_m = mat, axis_p = pat;  // the axes of a 4 x 4 register table of this op's consumed table
+        int axis_m = mat;  // who has the maternal axis of a 4 x 4 register table of this op's consumed table
         if (kind[o] == kLpFounder) {
             // a table over a couple: its axes are the parents of the kid it peeled, when it
             // comes in registers; otherwise the peel node takes the maternal axis
             const int p = pv.prev[pv.prev_off[o]];
             axis_m = d.peel;
-            axis_p = cuts[o][0];
             if (chained[p] && ped.mother[P.ops[p].peel] != d.peel) {
                 axis_m = cuts[o][0];
-                axis_p = d.peel;
                 h[kHPeelIsPat] = 1u;
             }
         }
@@ -210,8 +207,8 @@ std::string build_lanepeel(const PedigreeView& ped, const PeelView& pv, const st
         if (kind[o] == kLpFounder) h[kHMask] = (uint32_t)P.lod_mask[cuts[o][0]];
         for (int v = 0; v < 16; ++v) {
             uint32_t ix = 0xFFu;
-            if (kind[o] == kLpChild) ix = cell_of(o, mat, v >> 2, pat, v & 3);
-            if (kind[o] == kLpFounder && v < 4) ix = cell_of(o, cuts[o][0], v, -1, 0);
+            if (kind[o] == kLpChild) ix = cell_of(o, mat, v >> 2, v & 3);
+            if (kind[o] == kLpFounder && v < 4) ix = cell_of(o, cuts[o][0], v, 0);
             h[kHMap + (v >> 2)] |= ix << (8 * (v & 3));
         }
         for (int q = 0; q < d.n_prev; ++q) {
@@ -219,13 +216,12 @@ std::string build_lanepeel(const PedigreeView& ped, const PeelView& pv, const st
             uint32_t* hp = h + kHPrev + 8 * q;
             hp[kPOff] = chained[p] && !tape ? 0xFFFFFFFFu : (uint32_t)off[p];
             hp[kPAdj] = chained[p] ? 0xFFFFFFFFu : (uint32_t)adj[p];
-            hp[kPSize] = (uint32_t)size[p];
             hp[kPClass] = kind[o] == kLpChild ? (uint32_t)cls[o][q] : 0u;
             if (kind[o] == kLpGeneric) continue;
             for (int v = 0; v < 16; ++v) {
                 uint32_t ix = 0xFFu;
-                if (kind[o] == kLpChild && cls[o][q] == kLpK) ix = v < 4 ? cell_of(p, d.peel, v, -1, 0) : 0xFFu;
-                else ix = cell_of(p, axis_m, v >> 2, axis_p, v & 3);
+                if (kind[o] == kLpChild && cls[o][q] == kLpK) ix = v < 4 ? cell_of(p, d.peel, v, 0) : 0xFFu;
+                else ix = cell_of(p, axis_m, v >> 2, v & 3);
                 hp[kPMap + (v >> 2)] |= ix << (8 * (v & 3));
             }
             if (chained[p]) hp[kPClass] |= 16u;  // comes in registers

@@ -67,9 +67,9 @@ enum LpWord : int32_t {
     kHGroups = 55,    // 3 words: its groups of four contributions
     kHIntoLast = 58   // 1 when the last op consumes the table
 };
-// of a consumed table: arena cell (-1: registers), class, size, adjoint arena
+// of a consumed table (8 words): arena cell (-1: registers), class, adjoint arena
 // cell (-1: registers), 4 words of byte map ((mat, pat), or K: the trait's)
-enum LpPrev : int32_t { kPOff = 0, kPClass = 1, kPSize = 2, kPAdj = 3, kPMap = 4 };
+enum LpPrev : int32_t { kPOff = 0, kPClass = 1, kPAdj = 2, kPMap = 4 };
 
 enum OpType : int32_t { kChild = 1, kParent = 2, kPartner = 3, kLast = 4 };
 
