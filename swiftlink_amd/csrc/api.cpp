@@ -180,6 +180,7 @@ struct sl_ctx {
     bool samp_ready = false;
     // the flat L-sampler's per-locus records (unset when the tables are outside what it takes)
     bool flat_ok = false;
+    bool flat_tried = false;
     size_t flat_lds[2] = {0, 0};  // of the recomputing and the keeping form
     uint32_t* d_task = nullptr;
     uint32_t* d_task_base = nullptr;
@@ -707,31 +708,43 @@ int setup_msampler(sl_ctx* c, const sl_pedigree_desc* ped) {
         (rc = upload(c, &c->d_lsum, lsum.data(), lsum.size())) ||
         (rc = upload(c, &c->d_meioses, c->meioses_h.data(), c->meioses_h.size())))
         return rc;
-    // what each meiosis's flip does at each locus, and the loci left to compute
-    const size_t nb = 2 * (size_t)(N - F);
-    uint8_t* masks = nullptr;
-    if ((rc = upload<uint8_t>(c, &c->d_mcls, nullptr, nb * M)) ||
-        (rc = upload<int32_t>(c, &c->d_joblist, nullptr, nb * M)) ||
-        (rc = upload<int32_t>(c, &c->d_jobcnt, nullptr, nb)) ||
-        (rc = upload<uint8_t>(c, &masks, nullptr, (size_t)N * M)))
-        return rc;
-    sl::MsampArgs K{};
-    K.N = N;
-    K.F = F;
-    K.M = M;
-    K.ptab = c->d_ptab;
-    K.geno2 = c->d_geno2;
-    K.GW = GW;
-    std::vector<int32_t>& cnt = c->jobcnt_h;
-    cnt.resize(nb);
-    hipError_t e = sl::launch_mclass(K, masks, c->d_mcls, c->d_joblist, c->d_jobcnt, c->stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(cnt.data(), c->d_jobcnt, nb * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);  // and the host tables above go out of scope
-    (void)hipFree(masks);
-    SL_HIP(c, e);
-    c->max_jobs = *std::max_element(cnt.begin(), cnt.end());
+    SL_HIP(c, hipStreamSynchronize(c->stream));  // the host tables above go out of scope
     c->m_ready = true;
+    return SL_OK;
+}
+
+// What each meiosis's flip does at each locus, and the loci left to compute:
+// formed with a context's first chains.
+int setup_classes(sl_ctx* c) {
+    const int N = c->N, F = c->F, M = c->M;
+    const size_t nb = 2 * (size_t)(N - F);
+    void* bufs[4] = {};  // classes, lists, counts, and the elimination's masks
+    const size_t bytes[4] = {nb * M, nb * M * sizeof(int32_t), nb * sizeof(int32_t), (size_t)N * M};
+    std::vector<int32_t> cnt(nb);
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < 4 && e == hipSuccess; ++i) e = device_alloc(c, &bufs[i], bytes[i]);
+    if (e == hipSuccess) {
+        sl::MsampArgs K{};
+        K.N = N;
+        K.F = F;
+        K.M = M;
+        K.ptab = c->d_ptab;
+        K.geno2 = c->d_geno2;
+        K.GW = (N + 15) / 16;
+        e = sl::launch_mclass(K, (uint8_t*)bufs[3], (uint8_t*)bufs[0], (int32_t*)bufs[1], (int32_t*)bufs[2], c->stream);
+    }
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(cnt.data(), bufs[2], nb * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    const int keep = e == hipSuccess ? 3 : 0;
+    for (int i = keep; i < 4; ++i)
+        if (bufs[i]) (void)hipFree(bufs[i]);
+    SL_HIP(c, e);
+    c->d_mcls = (uint8_t*)bufs[0];
+    c->d_joblist = (int32_t*)bufs[1];
+    c->d_jobcnt = (int32_t*)bufs[2];
+    c->max_jobs = *std::max_element(cnt.begin(), cnt.end());
+    c->jobcnt_h = std::move(cnt);
     return SL_OK;
 }
 
@@ -772,8 +785,6 @@ int timed_span(sl_ctx* c, int kind, int launches, Fn body) {
 }
 
 }  // namespace
-
-static int setup_flat(sl_ctx* c);
 
 extern "C" {
 
@@ -987,12 +998,6 @@ int sl_create(const sl_pedigree_desc* ped, const sl_map_desc* map, const sl_peel
                 return fail(nullptr, SL_E_DEVICE, m);
             }
             c->samp_ready = true;
-            if ((rc = setup_flat(c))) {
-                std::string m = c->err;
-                release_all(c);
-                delete c;
-                return fail(nullptr, rc, m);
-            }
         }
     }
     e = sl::launch_fill(c->d_acc, -INFINITY, nacc, c->stream);
@@ -1219,12 +1224,14 @@ int sl_lod_kernel_for(sl_ctx* c, int32_t n_graphs, int32_t* kernel) {
 
 static sl::SampArgs samp_args(sl_ctx* c);
 
-// The flat L-sampler's records (lsampler.hip).  Leaves flat_ok false where it
-// does not apply: an op consumes more than three tables or has more than three
+// The flat L-sampler's records (lsampler.hip), formed with a context's first
+// chains or replicates.  Leaves flat_ok false where it does not apply: an op consumes more than three tables or has more than three
 // children, an index passes 16 bits, the tables alone do not fit LDS, or the
 // records pass kFlatMaxBytes or their share of the memory there is (the loci's
 // steps are then decoded in the kernel).
 static int setup_flat(sl_ctx* c) {
+    if (!c->samp_ready || c->flat_tried) return SL_OK;
+    c->flat_tried = true;
     const sl::SampProgram& P = c->sprog;
     for (int keep = 0; keep < 2; ++keep)
         c->flat_lds[keep] = sl::lsampler_flat_lds_bytes(c->precision, c->cells_cap, P.n_ops, c->N, c->F, keep != 0);
@@ -1271,6 +1278,9 @@ static int near_words(const sl_ctx* c) { return (c->M + 31) / 32; }
 static int alloc_chains(sl_ctx* c, int n_chains) {
     const size_t words = (size_t)n_chains * c->M * c->W;
     const size_t cm = (size_t)n_chains * c->M;
+    if (const int rc = setup_flat(c)) return rc;
+    if (c->m_ready && c->jobcnt_h.empty())
+        if (const int rc = setup_classes(c)) return rc;
     if (n_chains != c->n_chains) {
         void** bufs[] = {(void**)&c->d_chains, (void**)&c->d_status, (void**)&c->d_lcur, (void**)&c->d_lflip,
                          (void**)&c->d_fbuf, (void**)&c->d_maps, (void**)&c->d_mu, (void**)&c->d_near, (void**)&c->d_near_loci};
@@ -1503,7 +1513,7 @@ static int run_lsweep(sl_ctx* c, uint64_t seed, uint32_t sweep, int first_parity
 static int run_impute(sl_ctx* c, uint64_t seed, int R, int mode, int start, uint32_t chain_base) {
     const size_t per = (size_t)c->M * c->W;
     int rc;
-    if ((rc = ensure(c, &c->d_imp_graphs, &c->imp_graphs_cap, (size_t)R * per)) ||
+    if ((rc = setup_flat(c)) || (rc = ensure(c, &c->d_imp_graphs, &c->imp_graphs_cap, (size_t)R * per)) ||
         (rc = ensure(c, &c->d_imp_draw, &c->imp_draw_cap, (size_t)R)) ||
         (rc = ensure(c, &c->d_imp_weight, &c->imp_weight_cap, (size_t)R)) ||
         (rc = ensure(c, &c->d_imp_status, &c->imp_status_cap, (size_t)R)))

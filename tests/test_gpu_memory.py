@@ -3,7 +3,7 @@ the same results as these come and go."""
 import numpy as np
 import pytest
 
-from family_cases import family_case, line_family
+from family_cases import family_case, line_family, locus_cells
 from swiftlink_amd import native, synth
 from test_gpu_lanepeel import MODEL, _graphs
 
@@ -73,3 +73,27 @@ def test_batches_allocate_the_tables_they_use():
         ctx.lod_reset()
         ctx.mcmc_run(4, 0, 2, 0.5, 7)
         assert np.array_equal(out, ctx.mcmc_graphs())
+
+
+def test_sampler_tables_come_with_the_chains():
+    """4000 cells of 128 bytes of records at each of 400 loci, 200 MB, and the flip
+    classes: a context that only scores has none of them; the first chains, or the
+    first replicates, bring them."""
+    import torch
+    case, g0 = family_case(markers=400, missing=0.95, seed=1, tries=1, **line_family(300, 80))
+    records = 128 * int(locus_cells(case).sum())
+    assert records > 128 * MIB
+    free = lambda: torch.cuda.mem_get_info()[0]
+    for first in ("chains", "replicates"):
+        with native.Context(case, native.SL_FP32_RESCALED) as ctx:
+            ctx.lod_terms(g0[None])
+            before = free()
+            if first == "chains":
+                ctx.mcmc_init(g0[None])
+            else:
+                ctx.sequential_imputation(1, 1)
+            after = free()
+            assert before - after >= records
+            ctx.sequential_imputation(1, 1)  # there already
+            ctx.mcmc_init(g0[None])
+            assert after - free() < 32 * MIB
