@@ -70,6 +70,23 @@ def profile_traffic(kernel: str, workload: str):
     return float(m.group(1)) if m else None
 
 
+def evaluated_likelihoods(case) -> float:
+    """Founder-allele likelihoods a one-launch meiosis step evaluates, on average
+    over pairs of meioses.  A flip is decided by genotype elimination alone where
+    the parent cannot be heterozygous, or where its phase and the transmitted
+    allele are known; a flip left open is evaluated once, or for both values of
+    the previous meiosis's bit where that meiosis's flip is open too."""
+    b = case.meioses()
+    child, side = case.F + b // 2, b % 2
+    parent = np.where(side, case.father[child], case.mother[child])
+    q, c = case.legal[parent] & 15, case.legal[child] & 15  # bits UU, AA, AU, UA
+    u = np.where(side[:, None], c & 5, c & 9)   # traits with U from this parent
+    a = np.where(side[:, None], c & 10, c & 6)  # and with A
+    decided = ((q & 12) == 0) | (((q == 4) | (q == 8)) & ((u == 0) != (a == 0)))
+    p = 1.0 - decided.mean(axis=0)
+    return float((p * (1.0 + p)).sum())
+
+
 def cpu_threads() -> int:
     """The host cores this process may use: OMP_NUM_THREADS when set (the
     share of host cores a GPU is granted), else the CPUs in its affinity
@@ -455,18 +472,20 @@ def main():
     # ---- roofline of the meiosis-step kernel (one chain: mspec_kernel, the
     # forward-backward pass of step k beside the founder-allele likelihoods of
     # step k+1 for both values of meiosis k's bit): algorithmic bytes per
-    # launch = per (chain, meiosis, locus) ceil(2N/8) descent-graph bytes +
-    # ceil(2 N_typed/8) genotype bytes, times 2M likelihood jobs ----
+    # launch = per evaluated likelihood ceil(2N/8) descent-graph bytes +
+    # ceil(2 N_typed/8) genotype bytes (evaluated_likelihoods) ----
     ms_ms, ms_launches = prof32[native.SL_KERNEL_MSAMPLER]
     avg = lambda k: prof32[k][0] / max(prof32[k][1], 1)
     n_typed = int(np.count_nonzero(case.typed))
     bytes_per_unit = -(-2 * case.N // 8) + -(-2 * n_typed // 8)
-    bytes_per_launch = 2 * case.M * bytes_per_unit
+    bytes_per_launch = int(round(evaluated_likelihoods(case) * bytes_per_unit))
     ms_avg = ms_ms / max(ms_launches, 1)
     achieved = bytes_per_launch / (ms_avg * 1e-3) / 1e9 if ms_launches else 0.0
     lod_achieved = flops * evals_per_launch / (k32 * 1e-3) / 1e12
-    lod_name = ("lane_lod_kernel (one (graph, position) evaluation per lane)" if kern32 == native.SL_LOD_LANES
-                else "lod_kernel<float,true>")
+    # past the size at which the lane kernel's wavefronts are all resident, as the
+    # default batch is, the lane peel forms its terms and sums
+    lod_name = ("lanepeel_kernel<float, true, false> (one evaluation per lane, 64 graphs to a wavefront)"
+                if kern32 == native.SL_LOD_LANES else "lod_kernel<float,true>")
 
     res = {
         "metric": METRIC,
@@ -506,7 +525,7 @@ def main():
         "lod_roofline": {"bound": "mfma", "compute": "fp32 VALU (no MFMA: tables of 4^k cells)",
                          "kernel": lod_name, "achieved": lod_achieved, "peak": FP32_PEAK_TFLOPS,
                          "unit": "TFLOP/s", "frac": lod_achieved / FP32_PEAK_TFLOPS,
-                         "traffic": profile_traffic(lod_name.split("<")[0].split(" ")[0], args.config),
+                         "traffic": profile_traffic(lod_name.split("<")[0], args.config) if B == 64 else None,
                          "flops_per_eval": flops, "launch_ms": k32},
     }
     if extras:
