@@ -86,19 +86,25 @@ typedef struct {
 /* Trait-peel kernels (results agree to rounding; FP64 terms are identical):
  * SL_LOD_WORKGROUP runs one workgroup per (interval, chunk of
  * graphs_per_block graphs) whose wavefronts share each level of the peel;
- * SL_LOD_LANES runs one wavefront per (interval, position, 64 graphs), one
- * evaluation per lane, when its per-lane tables fit LDS (else the first);
- * SL_LOD_AUTO takes the second from 32 graphs per launch. */
+ * SL_LOD_LANES (FP32-rescaled) runs one wavefront per (interval, position, 64
+ * graphs), one evaluation per lane, when its per-lane tables fit LDS (else the
+ * first).  SL_LOD_AUTO takes the second from 32 graphs per launch, and from
+ * 16384 evaluations (graphs x intervals x positions) runs the lane peel, one
+ * evaluation per lane with tables in global memory, in place of either (of the
+ * first with one graph per block; of the second once its wavefronts would not
+ * all be on the device at once): the same arithmetic and the same chunks. */
 #define SL_LOD_AUTO 0
 #define SL_LOD_WORKGROUP 1
 #define SL_LOD_LANES 2
 
-/* M-sweep launch modes (results are identical): one launch per meiosis step,
- * computing the next step's likelihoods for both values of the current
- * meiosis's bit while its forward-backward pass runs; or two launches per
- * step; or the first while the doubled likelihood work is small.  Pedigrees
- * whose speculative workgroup would need more than 160 KiB of LDS always take
- * two launches.
+/* M-sweep launch modes (results are identical up to the rounding of the
+ * passes' scans): one launch per meiosis step, computing the next step's likelihoods
+ * for both values of the current meiosis's bit while its forward-backward pass
+ * runs; or two launches per step, the likelihoods planned over all chains; or
+ * (SL_MSAMPLER_AUTO) the first while the doubled likelihood work is small, then
+ * one launch per step with planned likelihoods while these are few, then two
+ * launches.  Pedigrees whose workgroup of a one-launch form would need more
+ * than 160 KiB of LDS take two launches.
  * SL_MSAMPLER_LDS_GRAPHS may be or-ed in: every founder-allele graph is then
  * built in LDS, as it always is for pedigrees of more than 1024 people or 512
  * founders (smaller ones keep a wavefront's graph in registers); results are
@@ -179,10 +185,10 @@ int sl_lod_terms(sl_ctx* ctx, const int32_t* graphs, int32_t n_graphs, double* o
  * recording and clears the totals).  For kernel SL_KERNEL_LOD (peel kernel),
  * SL_KERNEL_LSAMPLER (one parity launch), SL_KERNEL_MSAMPLER (one meiosis
  * step's launch: the founder-allele likelihoods, with the previous step's
- * forward-backward pass in the one-launch mode) or SL_KERNEL_MSAMPLER_FB (the
- * forward-backward pass of one meiosis step in the two-launch mode), *ms is
+ * forward-backward pass in the one-launch forms) or SL_KERNEL_MSAMPLER_FB (the
+ * forward-backward pass of one meiosis step in the two-launch form), *ms is
  * the time summed since the last enable and *launches the number of launches
- * it covers.  The one-launch mode's back-to-back step launches are timed as
+ * it covers.  The one-launch forms' back-to-back step launches are timed as
  * one span per M-sweep.  No counterpart in the reference. */
 int sl_profile(sl_ctx* ctx, int32_t enable);
 int sl_profile_read(sl_ctx* ctx, int32_t kernel, double* ms, int64_t* launches);
@@ -196,16 +202,19 @@ int sl_profile_read(sl_ctx* ctx, int32_t kernel, double* ms, int64_t* launches);
  * position) from the compiled program: flops and LDS bytes. */
 int sl_lod_work(sl_ctx* ctx, double* flops_per_eval, double* lds_bytes_per_eval);
 
-/* The trait-peel kernel (SL_LOD_WORKGROUP or SL_LOD_LANES) that scores a
- * launch of n_graphs graphs under the context's options and precision.  No
- * counterpart in the reference; for tuners and measurement. */
+/* The trait-peel kernel (SL_LOD_WORKGROUP or SL_LOD_LANES) whose arithmetic
+ * and chunks score a launch of n_graphs graphs under the context's options and
+ * precision.  Under SL_LOD_AUTO the lane peel runs in its place where the
+ * comment there says.  No counterpart in the reference; for tuners and
+ * measurement. */
 int sl_lod_kernel_for(sl_ctx* ctx, int32_t n_graphs, int32_t* kernel);
 
 /* ---- MCMC chains on the device (the intended GPUMarkovChain,
  * gpu_markov_chain.h:76-125) ---- */
 
 /* Uploads n_chains descent graphs (host, int32 [C][M][2N]) as the chain
- * states, packed on the device; clears the per-chain status.  Counterpart of
+ * states, packed on the device; clears the per-chain status.  A context's first
+ * call also builds the samplers' per-locus tables on the device.  Counterpart of
  * GPUMarkovChain's copy_to_gpu (gpu_markov_chain.h:110).  SL_E_INVALID when
  * n_chains exceeds the device's grid y extent (at most 65535): the sampler
  * kernels index chains by the grid's y coordinate. */
@@ -409,9 +418,11 @@ int sl_set_trait_model(sl_ctx* ctx, const sl_trait_model* model);
  * (as sl_lod_terms) and [1..6] = d ln L / d(penetrance[0..2], disease_freq,
  * theta_L, theta_R), theta_L = (o+1) p_l and theta_R = (n-o) p_l being the
  * position's flanking recombination fractions (linear partial theta,
- * genetic_map.h:186-192).  One workgroup per (graph, interval, position)
- * runs the peel forward with every table kept in LDS, then sweeps the ops
- * in reverse; nothing is stored between calls.  Requires
+ * genetic_map.h:186-192).  The peel runs forward with every table kept, then
+ * the ops in reverse: from 6144 evaluations (graphs x intervals x positions)
+ * one per lane, with table slots in global memory that stay with the context
+ * (up to 4 GiB, given back when another of its allocations is refused), below
+ * that one per workgroup.  Requires
  * sl_set_trait_model; a zero likelihood gives ln L = -inf and zero
  * derivatives. */
 int sl_trait_grad(sl_ctx* ctx, const int32_t* graphs, int32_t n_graphs, double* out);
