@@ -39,7 +39,10 @@ def test_passes_beside_jobs_near_the_limit(people, founders, threads, chains):
     for mode in (native.SL_MSAMPLER_AUTO, native.SL_MSAMPLER_TWO_LAUNCH):
         with native.Context(case, native.SL_FP64, msampler_mode=mode) as ctx:
             ctx.mcmc_init(np.repeat(g0[None], chains, axis=0))
+            ctx.profile(True)
             ctx.msweep(31, 0, order)
+            assert ctx.profile_read(native.SL_KERNEL_MSAMPLER_FB)[1] == len(order)  # two launches a step
+            ctx.profile(False)
             assert np.all(ctx.mcmc_status() == 0)
             assert ctx.mcmc_near_edge()[0] == 0
             out.append(ctx.mcmc_graphs())

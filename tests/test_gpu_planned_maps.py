@@ -23,7 +23,13 @@ def test_maps_past_a_thread_per_locus(tmp_path, markers):
         for mode in (native.SL_MSAMPLER_AUTO, native.SL_MSAMPLER_TWO_LAUNCH):
             with native.Context(case, precision, msampler_mode=mode) as ctx:
                 ctx.mcmc_init(np.repeat(g0[None], chains, axis=0))
+                ctx.profile(True)
                 ctx.msweep(61, 4)
+                passes = ctx.profile_read(native.SL_KERNEL_MSAMPLER_FB)[1]
+                ctx.profile(False)
+                # launches of a pass alone: none where the passes run beside the jobs
+                beside = mode == native.SL_MSAMPLER_AUTO and markers <= 4096
+                assert passes == (0 if beside else len(o.meioses()))
                 assert np.all(ctx.mcmc_status() == 0)
                 near = ctx.mcmc_near_edge()
                 out[precision, mode] = ctx.mcmc_graphs(), near
