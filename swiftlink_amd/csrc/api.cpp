@@ -18,8 +18,8 @@
 #include "philox.h"
 #include "program.h"
 #include "sampler_kernels.h"
-#include "slots.h"
 #include "sampler_program.h"
+#include "slots.h"
 
 using sl::PeelProgram;
 
@@ -180,7 +180,7 @@ struct sl_ctx {
     bool samp_ready = false;
     // the flat L-sampler's per-locus records (unset when the tables are outside what it takes)
     bool flat_ok = false;
-    bool flat_tried = false;
+    bool flat_tried = false;      // once, with the first chains or replicates
     size_t flat_lds[2] = {0, 0};  // of the recomputing and the keeping form
     uint32_t* d_task = nullptr;
     uint32_t* d_task_base = nullptr;
@@ -208,7 +208,7 @@ struct sl_ctx {
     uint8_t* d_mcls = nullptr;     // [2(N-F)][M] classes of a meiosis's flip by locus
     int32_t* d_joblist = nullptr;  // [2(N-F)][M] the loci whose flipped likelihood is computed
     int32_t* d_jobcnt = nullptr;   // [2(N-F)]
-    std::vector<int32_t> jobcnt_h;
+    std::vector<int32_t> jobcnt_h; // the same on the host; empty until the classes are formed
     int max_jobs = 0;              // the largest of them
     uint2* d_mplan = nullptr;      // MsampArgs::plan
     size_t mplan_cap = 0;
@@ -739,7 +739,7 @@ int setup_classes(sl_ctx* c) {
     const int keep = e == hipSuccess ? 3 : 0;
     for (int i = keep; i < 4; ++i)
         if (bufs[i]) (void)hipFree(bufs[i]);
-    SL_HIP(c, e);
+    if (e != hipSuccess) return hip_fail(c, e, "flip classes");
     c->d_mcls = (uint8_t*)bufs[0];
     c->d_joblist = (int32_t*)bufs[1];
     c->d_jobcnt = (int32_t*)bufs[2];
@@ -1225,10 +1225,11 @@ int sl_lod_kernel_for(sl_ctx* c, int32_t n_graphs, int32_t* kernel) {
 static sl::SampArgs samp_args(sl_ctx* c);
 
 // The flat L-sampler's records (lsampler.hip), formed with a context's first
-// chains or replicates.  Leaves flat_ok false where it does not apply: an op consumes more than three tables or has more than three
-// children, an index passes 16 bits, the tables alone do not fit LDS, or the
-// records pass kFlatMaxBytes or their share of the memory there is (the loci's
-// steps are then decoded in the kernel).
+// chains or replicates.  Leaves flat_ok false where it does not apply: an op
+// consumes more than three tables or has more than three children, an index
+// passes 16 bits, the tables alone do not fit LDS, or the records pass
+// kFlatMaxBytes or their share of the memory there is (the loci's steps are
+// then decoded in the kernel).
 static int setup_flat(sl_ctx* c) {
     if (!c->samp_ready || c->flat_tried) return SL_OK;
     c->flat_tried = true;
